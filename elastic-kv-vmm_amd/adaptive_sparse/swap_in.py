@@ -106,10 +106,11 @@ class HotBuffers:
         Needed after the table is edited outside the swap-in (install does it).
         """
         if self.bits is not None:
-            from .resident_lookup import build_residency_bits
-
-            build_residency_bits(self.table, out=self.bits, shift=self.bits_shift)
-        if self.resident_counts is not None:
+            helper, entries = _native.launch_helper()
+            status = helper.summary(entries["ekv_residency_summary"], self.table, self.bits, self.resident_counts,
+                                    self.bits_shift)
+            _native.launch_check(status, "refresh_bits")
+        elif self.resident_counts is not None:
             self.resident_counts.copy_(residency_counts(self.table, self.bits_shift))
 
     def check_status(self):

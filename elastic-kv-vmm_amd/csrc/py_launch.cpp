@@ -1,7 +1,8 @@
 // Python-facing launch helpers for the kernel entry points of the library:
 // the resident lookup (ekv_resolve_resident*), the row gather
 // (ekv_gather_rows), the plane gather / scatter / move (ekv_gather_kv,
-// ekv_scatter_kv, ekv_move_kv), the batch-token swap-in (ekv_swap_in*), the
+// ekv_scatter_kv, ekv_move_kv), the residency summary
+// (ekv_residency_summary), the batch-token swap-in (ekv_swap_in*), the
 // per-layer SGLang-convention swap-in (ekv_hisparse_swap_in) and the one-call
 // decode step (ekv_decode_step). Their GPU work can be a few microseconds at
 // small shapes, so
@@ -619,6 +620,37 @@ PyObject* move(PyObject*, PyObject* const* argv, Py_ssize_t argc) {
     }
 }
 
+// summary(entry, table, resident_bits, resident_counts, bits_shift)
+// -> status of ekv_residency_summary (resident_counts may be None)
+PyObject* summary(PyObject*, PyObject* const* argv, Py_ssize_t argc) {
+    if (argc != 5) {
+        PyErr_SetString(PyExc_TypeError, "summary takes 5 arguments");
+        return nullptr;
+    }
+    int64_t entry = 0, bits_shift = 0;
+    if (!read_int(argv[0], "entry", entry) || !read_int(argv[4], "bits_shift", bits_shift)) {
+        return nullptr;
+    }
+    Arg args[] = {{argv[1], "table"}, {argv[2], "resident_bits"}, {argv[3], "resident_counts"}};
+    try {
+        const int device = describe_all(args);
+        if (device < 0) {
+            return nullptr;
+        }
+        CurrentDevice current(device);
+        void* stream = c10::hip::getCurrentHIPStream(static_cast<c10::DeviceIndex>(device)).stream();
+        int status = 0;
+        Py_BEGIN_ALLOW_THREADS
+        status = reinterpret_cast<decltype(&ekv_residency_summary)>(entry)(
+            args[0].pointer(), args[1].pointer(), args[2].pointer(), bits_shift, stream);
+        Py_END_ALLOW_THREADS
+        return PyLong_FromLong(status);
+    } catch (const std::exception& error) {
+        PyErr_SetString(PyExc_RuntimeError, error.what());
+        return nullptr;
+    }
+}
+
 // swap_in(entry, counted, topk, block_size, rows, selected, slots, misses,
 //         miss_count, table, resident_bits, bits_shift, resident_counts,
 //         slot_token, stamps, slot_base, host_table, promote_src,
@@ -688,6 +720,8 @@ PyMethodDef methods[] = {
      "Describe a plane gather or scatter and call ekv_gather_kv / ekv_scatter_kv."},
     {"move", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(move)), METH_FASTCALL,
      "Describe a row move between two plane sets and call ekv_move_kv."},
+    {"summary", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(summary)), METH_FASTCALL,
+     "Describe a table, its residency summary and group counts and call ekv_residency_summary."},
     {"swap_in", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(swap_in)), METH_FASTCALL,
      "Describe the batch-token LRU swap-in's tensors and call ekv_swap_in / ekv_swap_in_counted."},
     {"abi_version", abi_version, METH_NOARGS, "EKV_ABI_VERSION this module was built against."},

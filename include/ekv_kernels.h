@@ -157,6 +157,16 @@ int ekv_residency_bits(const ekv_tensor* table, const ekv_tensor* resident_bits,
                        int64_t bits_shift, void* stream);
 
 /*
+ * ekv_residency_bits together with the group counts of ekv_swap_in, in one
+ * pass over the table: resident_counts (NULL, or at bits_shift > 0 [R, groups]
+ * or [L, R, groups] int32 with groups = ceil(T / 2^bits_shift)) gets the
+ * number of non-zero positions under each summary bit.
+ * No reference counterpart (maintenance of the summary above).
+ */
+int ekv_residency_summary(const ekv_tensor* table, const ekv_tensor* resident_bits,
+                          const ekv_tensor* resident_counts, int64_t bits_shift, void* stream);
+
+/*
  * Row gather over a fixed-position virtual layout.
  * Replaces: experimental/sparse_read.py:33-51 (gather_rows) and its kernel
  * :11-30.

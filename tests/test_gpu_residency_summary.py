@@ -14,6 +14,7 @@ import torch
 
 from adaptive_sparse.resident_lookup import build_residency_bits, resolve_resident, summary_words
 from adaptive_sparse.swap_in import HotBuffers, swap_in
+from elastic_kv import _native
 from oracle import oracle as ref
 
 pytestmark = pytest.mark.gpu
@@ -153,6 +154,39 @@ def _group_counts(table, shift):
     padded = np.zeros((*table.shape[:-1], groups << shift), bool)
     padded[..., :T] = table != 0
     return padded.reshape(*table.shape[:-1], groups, 1 << shift).sum(-1)
+
+
+@pytest.mark.parametrize("dtype", [torch.int16, torch.int32, torch.int64])
+@pytest.mark.parametrize("shift", [1, 2, 3, 6, 8, 10, 13])
+def test_one_pass_summary_and_counts_match_oracle(gpu, dtype, shift):
+    # Bits and group counts from one pass: rows that end inside a 16-byte piece, a group or a word (the storage behind
+    # them is filled, so reading past a row would show), groups of several per piece up to many loads each, and a
+    # strided table, which takes the general kernels.
+    rng = np.random.default_rng(shift * 11 + dtype.itemsize)
+    helper, entries = _native.launch_helper()
+    for shape in ((3, 1), (2, 7), (1, 2, 129), (2, 3, 4099), (3, 2, 65536), (1, 1, 32771)):
+        T = shape[-1]
+        table = rng.integers(1, 100, shape) * (rng.random(shape) < rng.choice([0.003, 0.5, 1.0], shape[:-1] + (1,)))
+        for layout in ("padded", "strided"):
+            if layout == "padded":
+                store = torch.full((*shape[:-1], -(-T // 128) * 128), 9, dtype=dtype, device=gpu)
+                view = store[..., :T]
+            else:
+                view = torch.full((*shape[:-1], 2 * T), 9, dtype=dtype, device=gpu)[..., ::2]
+            view.copy_(torch.tensor(table))
+            groups = -(-T // (1 << shift))
+            bits = torch.zeros((*shape[:-1], summary_words(T, shift)), dtype=torch.int32, device=gpu)
+            counts = torch.full((*shape[:-1], groups), -5, dtype=torch.int32, device=gpu)
+            status = helper.summary(entries["ekv_residency_summary"], view, bits, counts, shift)
+            _native.launch_check(status, "residency_summary")
+            want = ref.residency_bits(table, shift)
+            assert np.array_equal(bits.cpu().numpy()[..., :want.shape[-1]], want), (shape, layout)
+            assert not bits.cpu().numpy()[..., want.shape[-1]:].any()
+            assert np.array_equal(counts.cpu().numpy(), _group_counts(table, shift)), (shape, layout)
+    view, bits, counts = view[..., :4], bits[..., :4], counts[..., :4]
+    with pytest.raises(RuntimeError, match="bits_shift > 0"):
+        status = helper.summary(entries["ekv_residency_summary"], view, bits, counts, 0)
+        _native.launch_check(status, "residency_summary")
 
 
 @pytest.mark.parametrize("table_dtype,shift", [(torch.int16, 6), (torch.int32, 6), (torch.int16, 3)])
