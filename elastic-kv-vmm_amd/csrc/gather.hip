@@ -387,6 +387,167 @@ void launch_vw(const EngineArgs& a, int vw, hipStream_t stream) {
     }
 }
 
+// Moves whose source rows lie in host memory: the host link bounds them, and
+// it is at its best with little in flight. Once requests queue up, the link
+// serves the 8 XCDs unequally: with the whole job in flight (one workgroup
+// per tile, as above) two XCDs finished at half the time of the slowest, and
+// a few of them ran the rest of the job alone. kHostGroups workgroups with
+// one 16-byte load per lane keep 192 KiB in flight. 21,337 moves of K and V
+// rows of 512 B (22 MB), the same in each of three processes: 57.0 GB/s
+// against 51.9 in flight at once (24 workgroups 55.1, 32 56.6, 64 54-57.5, 96 54.4,
+// 128 56.3; two loads per lane 46-53 for 32). The copy engine reaches 56.4.
+// The moves are dealt out evenly: every workgroup adds up the counts of
+// kHostRows (layer, batch) rows at a time in LDS, and the vectors of all their
+// moves, in list order, are strided over the grid, so rows of unequal counts
+// and the unused tails of the lists cost nothing. The list entries of an
+// iteration are read while the load of the one before is in flight.
+constexpr uint32_t kHostGroups = 48;
+constexpr uint32_t kHostRowsPerThread = 4;
+constexpr uint32_t kHostRows = kThreads * kHostRowsPerThread;
+// Lists that could move no more than this fit in flight whole, and the tile
+// kernel's shorter way to its first load wins: 100 rows of 1 KiB from a list
+// of 256 take 9.1 us there and 9.9 us here.
+constexpr int64_t kHostMoveBytes = int64_t{512} << 10;
+
+template <int VW>
+__global__ __launch_bounds__(kThreads) void move_host_rows(const EngineArgs a, uint32_t batch_rows, FastDiv move_div) {
+    using V = typename Vec<VW>::type;
+    constexpr int kWaves = kThreads / 64;
+    __shared__ uint32_t first_move[kHostRows];   // moves of the rows below each row of this batch of rows
+    __shared__ uint32_t wave_moves[kWaves];
+    const int lane = threadIdx.x & 63;
+    const int wave = threadIdx.x >> 6;
+    const uint32_t rows = static_cast<uint32_t>(a.units);   // (layer, batch) rows
+    for (uint32_t base = 0; base < rows; base += batch_rows) {
+        // Exclusive prefix of the rows' counts, kHostRowsPerThread consecutive rows per thread.
+        uint32_t count[kHostRowsPerThread];
+#pragma unroll
+        for (uint32_t i = 0; i < kHostRowsPerThread; ++i) {
+            const uint32_t r = threadIdx.x * kHostRowsPerThread + i;
+            const bool live = r < batch_rows && base + r < rows;
+            const uint32_t at = live ? base + r : base;
+            const uint32_t l = a.div_b.div(at);
+            const int32_t c = a.move_counts[l * a.mc_l + (at - l * a.div_b.divisor) * a.mc_b];
+            count[i] = live && c > 0 ? static_cast<uint32_t>(min(int64_t{c}, a.K)) : 0u;
+        }
+        uint32_t mine = 0;
+#pragma unroll
+        for (uint32_t i = 0; i < kHostRowsPerThread; ++i) {
+            mine += count[i];
+        }
+        uint32_t inclusive = mine;
+#pragma unroll
+        for (int offset = 1; offset < 64; offset <<= 1) {
+            const uint32_t below = __shfl_up(inclusive, offset);
+            inclusive += lane >= offset ? below : 0u;
+        }
+        if (lane == 63) {
+            wave_moves[wave] = inclusive;
+        }
+        __syncthreads();
+        uint32_t at = inclusive - mine, moves = 0;
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) {
+            at += w < wave ? wave_moves[w] : 0u;
+            moves += wave_moves[w];
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < kHostRowsPerThread; ++i) {
+            first_move[threadIdx.x * kHostRowsPerThread + i] = at;
+            at += count[i];
+        }
+        __syncthreads();
+        // Vector q of the batch: move q / (kv * vectors per row), then plane, then vector of the row. Fewer than 2^31
+        // (the host sizes the batch of rows).
+        const uint32_t vectors = moves * move_div.divisor;
+        const uint32_t stride = gridDim.x * kThreads;
+        // Source and destination byte offsets of vector q; destination -1 when it moves nothing.
+        const auto place = [&](uint32_t q, int64_t& src, int64_t& dst) {
+            src = 0;
+            dst = -1;
+            if (q >= vectors) {
+                return;
+            }
+            const uint32_t move = move_div.div(q);
+            const uint32_t rest = q - move * move_div.divisor;
+            const uint32_t kv = rest >= a.vecs_per_row ? 1u : 0u;   // at most two planes
+            // The last row whose first move is at or below this one holds it (rows without moves share their
+            // first move with the next row).
+            uint32_t r = 0;
+#pragma unroll
+            for (uint32_t half = kHostRows / 2; half > 0; half >>= 1) {
+                r += first_move[r + half] <= move ? half : 0u;
+            }
+            const uint32_t i = move - first_move[r];
+            const uint32_t l = a.div_b.div(base + r);
+            const uint32_t b = base + r - l * a.div_b.divisor;
+            const int64_t from = a.move_src_rows[l * a.msr_l + b * a.msr_b + i * a.msr_i];
+            const int64_t to = a.move_dst_rows[l * a.mdr_l + b * a.mdr_b + i * a.mdr_i];
+            if (from >= 0 && from < a.ms_rows && to >= a.zero_below && to < a.pool_rows) {
+                const int64_t within = static_cast<int64_t>(rest - kv * a.vecs_per_row) * VW;
+                src = l * a.ms_layer_stride + kv * a.ms_kv_stride + from * a.ms_row_stride + within;
+                dst = l * a.layer_stride + kv * a.kv_stride + to * a.row_stride + within;
+            }
+        };
+        int64_t src, dst;
+        uint32_t q = blockIdx.x * kThreads + threadIdx.x;
+        place(q, src, dst);
+        for (uint32_t first = blockIdx.x * kThreads; first < vectors; first += stride) {   // uniform
+            const int64_t to = dst;
+            V v{};
+            if (to >= 0) {
+                v = load_vec<VW>(a.src_base + src, true);
+            }
+            q += stride;
+            place(q, src, dst);
+            if (to >= 0) {
+                store_vec<VW>(a.dst_base + to, v);
+            }
+        }
+        __syncthreads();   // the prefix is rewritten by the next batch of rows
+    }
+}
+
+// True when `address` lies in host memory (pinned and device mapped). Asked on every call: nothing is kept by address.
+bool in_host_memory(const void* address) {
+    hipPointerAttribute_t attributes{};
+    if (hipPointerGetAttributes(&attributes, address) != hipSuccess) {
+        (void)hipGetLastError();   // memory the runtime does not know is not host memory; the query's error is not ours
+        return false;
+    }
+    return attributes.type == hipMemoryTypeHost;
+}
+
+template <int VW>
+void launch_host_move(EngineArgs a, uint32_t batch_rows, hipStream_t stream) {
+    a.vecs_per_row = static_cast<uint32_t>(a.row_bytes / VW);
+    const FastDiv move_div(static_cast<uint32_t>(a.KV * a.vecs_per_row));
+    // The bytes in flight are what counts: narrower vectors take more workgroups.
+    const uint32_t groups = kHostGroups * (16 / VW);
+    move_host_rows<VW><<<dim3(groups), dim3(kThreads), 0, stream>>>(a, batch_rows, move_div);
+}
+
+// Moves from host memory through move_host_rows; false when the job does not fit its 32-bit counts.
+bool host_move(EngineArgs a, int64_t rows, int vw, hipStream_t stream) {
+    // Vectors per (layer, batch) row at most; a batch of rows stays below 2^31 with room for the last stride.
+    const int64_t per_row = a.K * a.KV * (a.row_bytes / vw);
+    const int64_t limit = (int64_t{1} << 30) / per_row;
+    if (limit < 1 || rows >= (int64_t{1} << 31)) {
+        return false;
+    }
+    const uint32_t batch_rows = static_cast<uint32_t>(std::min<int64_t>(limit, kHostRows));
+    a.units = rows;
+    a.div_b = FastDiv(static_cast<uint32_t>(a.B));
+    switch (vw) {
+        case 16: launch_host_move<16>(a, batch_rows, stream); break;
+        case 8: launch_host_move<8>(a, batch_rows, stream); break;
+        case 4: launch_host_move<4>(a, batch_rows, stream); break;
+        case 2: launch_host_move<2>(a, batch_rows, stream); break;
+        default: launch_host_move<1>(a, batch_rows, stream); break;
+    }
+    return true;
+}
+
 void need_planes(const ekv_planes* p) {
     if (p == nullptr) {
         throw std::invalid_argument("planes are required");
@@ -632,7 +793,11 @@ int move_kv(const ekv_planes* src, const ekv_tensor* src_rows_p, const ekv_plane
     if (check_only()) {
         return 0;
     }
-    launch_vw<KvMove>(a, vw, static_cast<hipStream_t>(stream));
+    const auto s = static_cast<hipStream_t>(stream);
+    const bool linked = units * a.row_bytes > kHostMoveBytes && in_host_memory(src->base);
+    if (!linked || !host_move(a, L * B, vw, s)) {
+        launch_vw<KvMove>(a, vw, s);
+    }
     check_hip(hipGetLastError(), "launch KV move");
     return 0;
 }

@@ -91,3 +91,44 @@ def test_gather_kv_rejects_bad_shapes(gpu):
     with pytest.raises(ValueError):
         gather_kv(planes, torch.zeros((2, 2, 3), dtype=torch.int32, device=gpu),
                   torch.zeros((2, 2, 2, 3, 16), dtype=torch.uint8, device=gpu))
+
+
+@pytest.mark.parametrize("row_bytes,kv,layers,batch,k", [
+    (512, 2, 2, 24, 160),      # several strides of the grid per batch of rows
+    (512, 2, 2, 700, 6),       # more (layer, batch) rows than one batch of rows holds
+    (1040, 1, 1, 3, 340),      # a row that is no power of two of vectors
+    (200, 2, 1, 5, 333), (36, 1, 2, 3, 3000), (6, 2, 1, 20, 2500), (3, 2, 1, 20, 5000),    # narrower vectors
+    (512, 2, 1, 8, 64), (512, 2, 1, 8, 65),      # the largest list of the tile kernel, the smallest past it
+    (16, 2, 1, 1, 1)])
+def test_move_from_host_memory_matches_oracle(gpu, row_bytes, kv, layers, batch, k):
+    from adaptive_sparse.host_arena import HostArena
+    from adaptive_sparse.kv_pool import KVPlanes
+    from adaptive_sparse.swap_in import move_kv
+    from oracle import oracle as ref
+
+    rng = np.random.default_rng(row_bytes + batch)
+    src_n, dst_n = 300, layers * batch * k + 1
+    arena = HostArena(layers * kv * src_n * row_bytes)
+    try:
+        source = rng.integers(0, 256, arena.nbytes, dtype=np.uint8)
+        arena.host.copy_(torch.from_numpy(source))
+        pool = torch.zeros(layers * kv * dst_n * row_bytes, dtype=torch.uint8, device=gpu)
+
+        def planes(base, rows):
+            return KVPlanes(base=base, device=0, layers=layers, kv=kv, layer_stride=kv * rows * row_bytes,
+                            kv_stride=rows * row_bytes, row_stride=row_bytes, row_bytes=row_bytes, rows=rows, owner=None)
+
+        src_planes, dst_planes = planes(arena.device_ptr, src_n), planes(pool.data_ptr(), dst_n)
+        src_rows = rng.integers(-2, src_n + 2, (layers, batch, k))
+        dst_rows = np.stack([rng.permutation(batch * k).reshape(batch, k) for _ in range(layers)])   # 0: skipped
+        counts = rng.integers(-1, k + 2, (layers, batch)) * (rng.random((layers, batch)) < 0.7)
+        t = lambda a: torch.tensor(a, dtype=torch.int32, device=gpu)  # noqa: E731
+        layout = lambda p: (p.layer_stride, p.kv_stride, p.row_stride, row_bytes, p.rows)  # noqa: E731
+        for current in (counts, np.full_like(counts, k), np.zeros_like(counts)):
+            pool.zero_()
+            move_kv(src_planes, t(src_rows), dst_planes, t(dst_rows), t(current))
+            want = ref.move_kv(source, layout(src_planes), np.zeros(pool.numel(), np.uint8), layout(dst_planes),
+                               src_rows, dst_rows, current, kv, zero_below=1)
+            assert np.array_equal(pool.cpu().numpy(), want)
+    finally:
+        arena.close()
