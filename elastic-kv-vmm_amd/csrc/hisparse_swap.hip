@@ -24,7 +24,7 @@
 // recent), device_buffer_locs[r, i] (device row of slot i; column H is the
 // reserved newest-token row), host_cache_locs[r, t] (host row of token t).
 //
-// One 256-thread workgroup per batch row:
+// One 1024-thread workgroup per batch row:
 //   1. the hot tokens are hashed into LDS (open addressing, at least 2H
 //      buckets holding slot ids, so every probe sequence meets an empty
 //      bucket);
@@ -39,8 +39,8 @@
 //   4. the same scan over contiguous runs of the old LRU order gives each
 //      slot's place in the new order and the victims (empty slots first, then
 //      untouched slots);
-//   5. the misses' rows are copied from mapped pinned host memory, 16 bytes
-//      per lane when rows and bases allow.
+//   5. a second launch copies the misses' rows from mapped pinned host memory,
+//      16 bytes per lane when rows and bases allow.
 // Locations outside the device buffer are reported as -1 and never written.
 #include "../../include/ekv_kernels.h"
 #include "ekv_common.h"
@@ -49,18 +49,25 @@
 #include "ekv_tensor_util.h"
 #include "ekv_vec.h"
 
+#include <algorithm>
 #include <atomic>
 #include <climits>
 
 namespace ekv {
 namespace {
 
-constexpr int kThreads = 256;
+// Threads of the swap: one workgroup per batch row holds its CU alone (134 KiB of
+// LDS at the largest shape) and is a chain of barriers, so the more waves share its
+// loops the shorter it is: 23 us for 24 rows of 2048 lanes and 4096 slots with
+// 1024 threads, 44 us with 256.
+constexpr int kThreads = 1024;
 constexpr int kWaves = kThreads / 64;
 constexpr int64_t kMaxHot = 4096;     // hot slots per request (LDS holds the hash and the order)
 constexpr int64_t kMaxLanes = 2048;   // selected lanes per row (Top-K blocks x block size)
 constexpr int kLanesPerThread = static_cast<int>(kMaxLanes / kThreads);
-constexpr int kBatch = 8;             // state loads in flight per thread
+constexpr int kBatch = 4;             // state loads in flight per thread
+constexpr int kSlotBits = 12;         // a miss left for the copy launch: -2 - (miss rank << kSlotBits | slot)
+static_assert(kMaxHot <= 1 << kSlotBits && kMaxLanes << kSlotBits < int64_t{1} << 30, "slot and rank fit an entry");
 constexpr int32_t kEmpty = -1;
 constexpr int kMaxDevices = 64;
 
@@ -111,7 +118,6 @@ struct Lds {
     int32_t* lane_aux;    // [W] hit: slot; miss: hash bucket
     int32_t* lane_pos;    // [W] output position (-1: not selected)
     int32_t* lane_val;    // [W] hit: its device row (-1: outside the buffer); miss: its host row
-    int32_t* miss_host;   // [W] host row of the m-th miss
     int32_t* miss_loc;    // [W] device row of the m-th miss (-1: none)
     uint8_t* lane_kind;   // [W]
     int32_t* scratch;     // [3 * kWaves + 4]
@@ -170,43 +176,6 @@ __device__ __forceinline__ int64_t device_row(const HsArgs& a, int64_t r, int64_
     return row >= 0 && row < a.dev_rows ? row : -1;
 }
 
-template <typename V>
-__device__ __forceinline__ void copy_rows(const HsArgs& a, const Lds& s, int32_t misses) {
-    // The pieces of all misses (both planes) are dealt to the workgroup's
-    // threads in order; each thread issues 4 loads over the host link before
-    // its 4 stores, so 4 x 256 pieces are in flight per workgroup.
-    constexpr int64_t kWidth = sizeof(V);
-    const uint32_t per_plane = static_cast<uint32_t>(a.row_bytes / kWidth);
-    const uint32_t total = static_cast<uint32_t>(misses) * 2u * per_plane;
-    for (uint32_t first = 0; first < total; first += 4 * kThreads) {
-        V v[4];
-        int64_t dst[4];
-        bool ok[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const uint32_t q = first + k * kThreads + threadIdx.x;
-            const uint32_t m = q < total ? a.row_div.div(q) : 0u;   // miss index
-            const uint32_t p = q - m * 2u * per_plane;              // piece within the miss's K and V rows
-            const int64_t kv = p >= per_plane ? 1 : 0;
-            const int64_t at = static_cast<int64_t>(p) - kv * per_plane;
-            ok[k] = q < total && s.miss_loc[m] >= 0;
-            dst[k] = 0;
-            if (ok[k]) {
-                const int64_t src_row = s.miss_host[m];
-                dst[k] = kv * a.dev_kv + static_cast<int64_t>(s.miss_loc[m]) * a.dev_rs + at * kWidth;
-                v[k] = *reinterpret_cast<const V*>(a.host_k + kv * a.host_kv + src_row * a.host_rs + at * kWidth);
-            }
-        }
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            if (ok[k]) {
-                *reinterpret_cast<V*>(a.dev_k + dst[k]) = v[k];
-            }
-        }
-    }
-}
-
-template <int kVecWidth>
 __global__ __launch_bounds__(kThreads) void hisparse_swap_kernel(const HsArgs a) {
     extern __shared__ __align__(16) unsigned char shared[];
     const int64_t b = blockIdx.x;
@@ -231,7 +200,6 @@ __global__ __launch_bounds__(kThreads) void hisparse_swap_kernel(const HsArgs a)
         s.lane_aux = reinterpret_cast<int32_t*>(take(W * 4));
         s.lane_pos = reinterpret_cast<int32_t*>(take(W * 4));
         s.lane_val = reinterpret_cast<int32_t*>(take(W * 4));
-        s.miss_host = reinterpret_cast<int32_t*>(take(W * 4));
         s.miss_loc = reinterpret_cast<int32_t*>(take(W * 4));
         s.lane_kind = reinterpret_cast<uint8_t*>(take(W));
         s.scratch = reinterpret_cast<int32_t*>(take((3 * kWaves + 4) * 4));
@@ -440,7 +408,6 @@ __global__ __launch_bounds__(kThreads) void hisparse_swap_kernel(const HsArgs a)
             if (first_miss(o)) {
                 s.lane_rank[o] = static_cast<int16_t>(miss_rank);
                 s.miss_lane[miss_rank] = static_cast<int16_t>(o);
-                s.miss_host[miss_rank] = value;
                 ++miss_rank;
             }
         }
@@ -533,31 +500,153 @@ __global__ __launch_bounds__(kThreads) void hisparse_swap_kernel(const HsArgs a)
         __syncthreads();
     }
 
-    // 6. Outputs of miss lanes (a repeated token reuses its first lane's
-    //    location) and the -1 tail.
+    // 6. Outputs of miss lanes and the -1 tail. A token's first lane leaves
+    //    -2 - (miss rank << kSlotBits | slot) for the copy launch, which copies
+    //    the slot's rows and puts its location there; a repeated token takes
+    //    the location at once.
     for (int64_t o = threadIdx.x; o < W; o += kThreads) {
         if (s.lane_kind[o] == kMiss) {
             const int32_t owner = s.hash[s.lane_aux[o]] - static_cast<int32_t>(H);
-            out[s.lane_pos[o] * a.out_so] = s.miss_loc[s.lane_rank[owner]];
+            const int32_t m = s.lane_rank[owner];
+            const int32_t loc = s.miss_loc[m];
+            out[s.lane_pos[o] * a.out_so] = owner == o && loc >= 0 ? -2 - (m << kSlotBits | int32_t{s.victim[m]}) : loc;
         }
     }
     for (int64_t o = selected + threadIdx.x; o < W; o += kThreads) {
         out[o * a.out_so] = -1;
     }
+}
 
-    // 7. Copy the misses' K and V rows from the host cache.
-    copy_rows<typename Vec<kVecWidth>::type>(a, s, misses);
+// The misses' K and V rows, copied from the host cache by a launch of its own
+// right behind the swap: the host link bounds it, and one workgroup per
+// batch row kept it busy neither with few rows (16 KiB in flight each) nor with
+// many (unequal misses, and the link serves the XCDs unequally once requests
+// queue up). kCopyGroups workgroups of one 16-byte load per lane keep 192 KiB
+// in flight, the amount that reached the link's rate for the row moves (57 GB/s).
+// A miss to copy is an output entry -2 - slot (the swap's step 6): the slot
+// names its token, which names its host row, and its device row, which
+// replaces the entry. So the launches share no memory beyond the caller's own
+// state, in a graph as well. A wave takes a.span entries at a time; the four
+// reads that lead to their host rows run up to three spans ahead of the
+// copies. @@
+constexpr uint32_t kCopyGroups = 48;
+constexpr int kCopyThreads = 256;
+constexpr int kScan = 16;                            // entries in flight per thread
+constexpr uint32_t kRound = kCopyThreads * kScan;        // entries per round of the scan
+constexpr uint32_t kCopyBatch = 2048;                // misses whose copy pieces are counted in 32 bits (checked by the host)
+constexpr uint32_t kListed = kCopyBatch + kRound;    // misses listed at most: the list is emptied above kCopyBatch
+
+template <typename V>
+__global__ __launch_bounds__(kCopyThreads) void copy_missed_rows(const HsArgs a, int64_t first_row, uint32_t entries,
+                                                             FastDiv width_div, FastDiv group_div) {
+    constexpr int64_t kWidth = sizeof(V);
+    constexpr int kResolve = 4;            // misses resolved per thread at a time
+    __shared__ uint32_t host_of[kListed];  // entry, then host row (all ones: none)
+    __shared__ int32_t dev_of[kListed];    // slot, then device row (-1: none)
+    __shared__ uint32_t listed;
+    const uint32_t per_plane = static_cast<uint32_t>(a.row_bytes / kWidth);
+    const int32_t* out = a.out + first_row * a.out_sb;
+    if (threadIdx.x == 0) {
+        listed = 0;
+    }
+    __syncthreads();
+    for (uint32_t base = 0; base < entries; base += kRound) {
+        int32_t held[kScan];
+#pragma unroll
+        for (int k = 0; k < kScan; ++k) {
+            const uint32_t e = base + k * kCopyThreads + threadIdx.x;
+            const uint32_t at = e < entries ? e : 0u;
+            const uint32_t row = width_div.div(at);
+            held[k] = out[row * a.out_sb + (at - row * width_div.divisor) * a.out_so];
+        }
+#pragma unroll
+        for (int k = 0; k < kScan; ++k) {
+            const uint32_t e = base + k * kCopyThreads + threadIdx.x;
+            if (e < entries && held[k] <= -2) {
+                const uint32_t code = static_cast<uint32_t>(-2 - held[k]);
+                const uint32_t deal = (code >> kSlotBits) + width_div.div(e);
+                if (deal - group_div.div(deal) * group_div.divisor == blockIdx.x) {
+                    const uint32_t i = atomicAdd(&listed, 1u);
+                    host_of[i] = e;
+                    dev_of[i] = static_cast<int32_t>(code & ((1u << kSlotBits) - 1));
+                }
+            }
+        }
+        __syncthreads();
+        const uint32_t n = listed;
+        if (n <= kCopyBatch && entries - base > kRound) {   // uniform: more of the scan fits
+            __syncthreads();   // the next round counts on only after every thread has read the count
+            continue;
+        }
+        for (uint32_t first = 0; first < n; first += kResolve * kCopyThreads) {
+            int64_t request[kResolve], loc[kResolve], host[kResolve];
+            int32_t token[kResolve];
+            uint32_t entry[kResolve];
+#pragma unroll
+            for (int k = 0; k < kResolve; ++k) {
+                const uint32_t i = first + k * kCopyThreads + threadIdx.x;
+                entry[k] = host_of[i < n ? i : first];
+                request[k] = a.req[first_row + width_div.div(entry[k])];
+            }
+#pragma unroll
+            for (int k = 0; k < kResolve; ++k) {
+                const uint32_t i = first + k * kCopyThreads + threadIdx.x;
+                const int64_t slot = dev_of[i < n ? i : first];
+                token[k] = a.tokens[request[k] * a.tok_sr + slot * a.tok_ss];
+                loc[k] = device_row(a, request[k], slot);
+            }
+#pragma unroll
+            for (int k = 0; k < kResolve; ++k) {
+                const bool known = token[k] >= 0 && token[k] < a.T;
+                const int64_t row = load_index(a.host_locs, a.host_locs64,
+                                               known ? request[k] * a.hl_sr + token[k] * a.hl_st : 0);
+                host[k] = known && row >= 0 && row < a.host_rows ? row : -1;
+            }
+            __syncthreads();   // entry `first` stands in for threads past the list until all of them have read it
+#pragma unroll
+            for (int k = 0; k < kResolve; ++k) {
+                const uint32_t i = first + k * kCopyThreads + threadIdx.x;
+                if (i < n) {
+                    const uint32_t row = width_div.div(entry[k]);
+                    a.out[(first_row + row) * a.out_sb + (entry[k] - row * width_div.divisor) * a.out_so] =
+                        static_cast<int32_t>(loc[k]);
+                    host_of[i] = static_cast<uint32_t>(host[k]);
+                    dev_of[i] = static_cast<int32_t>(loc[k]);
+                }
+            }
+            __syncthreads();
+        }
+        for (uint32_t from = 0; from < n; from += kCopyBatch) {
+            const uint32_t pieces = (n - from < kCopyBatch ? n - from : kCopyBatch) * 2u * per_plane;
+            for (uint32_t q = threadIdx.x; q < pieces; q += kCopyThreads) {
+                const uint32_t m = a.row_div.div(q);
+                const uint32_t p = q - m * 2u * per_plane;   // piece within the miss's K and V rows
+                const int64_t kv = p >= per_plane ? 1 : 0;
+                const int64_t within = (static_cast<int64_t>(p) - kv * per_plane) * kWidth;
+                const uint32_t src = host_of[from + m];
+                const int64_t dst = dev_of[from + m];
+                if (src != ~0u && dst >= 0) {
+                    *reinterpret_cast<V*>(a.dev_k + kv * a.dev_kv + dst * a.dev_rs + within) =
+                        *reinterpret_cast<const V*>(a.host_k + kv * a.host_kv + src * a.host_rs + within);
+                }
+            }
+        }
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            listed = 0;
+        }
+        __syncthreads();
+    }
 }
 
 size_t lds_bytes(int64_t H, int64_t HB, int64_t W) {
     auto round = [](int64_t bytes) { return static_cast<size_t>((bytes + 15) & ~int64_t{15}); };
-    return round(HB * 4) + round(H * 4) * 2 + round(H * 2) * 2 + round(W * 2) * 3 + round(W * 4) * 6 + round(W) +
+    return round(HB * 4) + round(H * 4) * 2 + round(H * 2) * 2 + round(W * 2) * 3 + round(W * 4) * 5 + round(W) +
            round((3 * kWaves + 4) * 4);
 }
 
-template <int kVecWidth>
-void launch(const HsArgs& a, size_t lds, hipStream_t stream) {
-    const auto kernel = hisparse_swap_kernel<kVecWidth>;
+void launch_swap(const HsArgs& a, size_t lds, hipStream_t stream) {
+    const auto kernel = hisparse_swap_kernel;
     // The LDS limit is raised once per device, to the largest size any call
     // needs, so calls recorded into a graph make no attribute call.
     static std::atomic<bool> raised[kMaxDevices];
@@ -575,6 +664,19 @@ void launch(const HsArgs& a, size_t lds, hipStream_t stream) {
     }
     kernel<<<dim3(static_cast<uint32_t>(a.batch)), dim3(kThreads), lds, stream>>>(a);
     check_hip(hipGetLastError(), "launch hisparse swap-in");
+}
+
+template <int kVecWidth>
+void launch_copy(const HsArgs& a, hipStream_t stream) {
+    // The bytes in flight are what counts: narrower pieces take more workgroups.
+    const uint32_t groups = kCopyGroups * (16 / kVecWidth);
+    const int64_t rows_at_once = (int64_t{1} << 30) / a.width;   // entries are counted in 32 bits
+    for (int64_t first = 0; first < a.batch; first += rows_at_once) {
+        const int64_t rows = std::min(rows_at_once, a.batch - first);
+        copy_missed_rows<typename Vec<kVecWidth>::type><<<dim3(groups), dim3(kCopyThreads), 0, stream>>>(
+            a, first, static_cast<uint32_t>(rows * a.width), FastDiv(a.width), FastDiv(groups));
+        check_hip(hipGetLastError(), "launch hisparse row copies");
+    }
 }
 
 void need_index2(const ekv_tensor& t, const char* name) {
@@ -732,12 +834,16 @@ int hisparse_swap_in(const ekv_tensor* topk_p, const ekv_tensor* tokens_p, const
         throw std::invalid_argument("rows too large for one swap-in (copy pieces exceed 2^31)");
     }
     a.row_div = FastDiv(static_cast<uint32_t>(pieces));
+    launch_swap(a, lds, st);
+    if (R == 0 || T == 0) {
+        return 0;   // no row has state or no token a host row: nothing missed
+    }
     switch (vw) {
-        case 16: launch<16>(a, lds, st); break;
-        case 8: launch<8>(a, lds, st); break;
-        case 4: launch<4>(a, lds, st); break;
-        case 2: launch<2>(a, lds, st); break;
-        default: launch<1>(a, lds, st); break;
+        case 16: launch_copy<16>(a, st); break;
+        case 8: launch_copy<8>(a, st); break;
+        case 4: launch_copy<4>(a, st); break;
+        case 2: launch_copy<2>(a, st); break;
+        default: launch_copy<1>(a, st); break;
     }
     return 0;
 }

@@ -270,3 +270,41 @@ def test_graph_replays_with_padding_rows_match_the_oracle(gpu):
         assert np.array_equal(lru.cpu().numpy().astype(np.int64), want[1]), step
         assert np.array_equal(device_k.cpu().numpy(), want[2]) and np.array_equal(device_v.cpu().numpy(), want[3])
         torch.randn(1000, device=gpu).sum().item()        # eager work between replays
+
+
+@pytest.mark.parametrize("batch,row_bytes", [(52, 16), (1, 1024), (3, 72), (7, 6)])
+def test_copy_launch_deals_out_every_miss(gpu, batch, row_bytes):
+    # A cold step (every lane misses: 2,048 rows per request, over 2,048 of them for one copy workgroup at 52
+    # requests), then a mixed one: each miss is copied once, by the workgroup its rank falls to.
+    rng = np.random.default_rng(batch)
+    hot, bs, k, context = 2048, 16, 128, 4096
+    host_rows = batch * context
+    host_locs = rng.permutation(host_rows).reshape(batch, context)
+    dev_locs = rng.permutation(batch * (hot + 1)).reshape(batch, hot + 1) + 1
+    host = torch.randint(0, 256, (2, host_rows, row_bytes), dtype=torch.uint8).pin_memory()
+    device_k = torch.zeros((batch * (hot + 1) + 1, row_bytes), dtype=torch.uint8, device=gpu)
+    device_v = torch.zeros_like(device_k)
+    tokens = torch.full((batch, hot + 1), -1, dtype=torch.int32, device=gpu)
+    lru = torch.arange(hot, dtype=torch.int16, device=gpu).repeat(batch, 1)
+    out = torch.empty((batch, k * bs), dtype=torch.int32, device=gpu)
+    req = rng.permutation(batch)
+    host_locs_d, dev_locs_d = torch.tensor(host_locs, device=gpu), torch.tensor(dev_locs, device=gpu)
+    want = (tokens.cpu().numpy(), lru.cpu().numpy().astype(np.int64), device_k.cpu().numpy(),
+            device_v.cpu().numpy())
+    seq = np.full(batch, context)
+    for step in range(2):
+        blocks = np.stack([rng.permutation(context // bs)[:k] for _ in range(batch)])
+        load_blocks_to_device_buffer_mha(
+            top_k_blocks=torch.tensor(blocks, dtype=torch.int32, device=gpu), device_buffer_tokens=tokens,
+            host_cache_locs=host_locs_d, device_buffer_locs=dev_locs_d, host_cache_k=host[0], host_cache_v=host[1],
+            device_buffer_k=device_k, device_buffer_v=device_v, top_k_device_locs=out,
+            req_pool_indices=torch.tensor(req, device=gpu),
+            seq_lens=torch.tensor(seq, dtype=torch.int32, device=gpu), lru_slots=lru, item_size_bytes=row_bytes,
+            hot_buffer_size=hot, sparse_block_size=bs)
+        want_out, *rest = ref.hisparse_swap(blocks, want[0], host_locs, dev_locs, host[0].numpy(), host[1].numpy(),
+                                            want[2], want[3], req, seq, want[1], hot, bs, batch)
+        want = (rest[0], rest[1], rest[2], rest[3])
+        assert np.array_equal(out.cpu().numpy(), want_out), step
+        assert np.array_equal(tokens.cpu().numpy(), want[0]), step
+        assert np.array_equal(lru.cpu().numpy().astype(np.int64), want[1]), step
+        assert np.array_equal(device_k.cpu().numpy(), want[2]) and np.array_equal(device_v.cpu().numpy(), want[3])
