@@ -25,7 +25,7 @@
 // (an LDS hash of the miss tokens names each token's first miss), and its
 // later lanes share that slot and record empty promotions.
 //
-// One 256-thread workgroup per (row, layer): hits are touched in LDS, a
+// One workgroup per (row, layer): hits are touched in LDS, a
 // radix select over the stamps finds the victims (the slots of the smallest
 // (stamp, slot) keys), which one scan lists in slot order; the i-th distinct
 // miss (in miss-list order) takes the i-th of them. (Which victim slot a
@@ -38,12 +38,15 @@
 //
 // Residency summary. At bits_shift 0 a bit is one position: an evicted
 // token clears it, an inserted token sets it. A coarser bit covers 2^shift
-// positions; with per-bit resident counts the summary stays exact: every
-// eviction decrements its group's count and clears the bit when it reaches
-// zero, then (after a workgroup barrier, so no clear can follow a set) every
-// insertion increments its group's count and sets the bit from zero.
-// Without counts a coarse bit is only ever set, and the summary is a
-// superset of the table.
+// positions; with per-bit resident counts the summary stays exact: a group's
+// evictions and insertions change its count, and its bit is cleared when the
+// count reaches zero and set when it leaves zero. Without counts a coarse
+// bit is only ever set, and the summary is a superset of the table. A row's
+// words (or changes of counts) are gathered in LDS and written once: the row
+// belongs to this workgroup. As an atomic per eviction and insertion they
+// were a quarter of the call at 2560 rows (178.6 against 133.5 us). Rows too
+// long for LDS still take atomics, evictions before a barrier, insertions after it, so
+// that no clear can follow a set.
 //
 // Refused rows. Two selected rows naming one request would race on its hot
 // buffer, and a step whose stamps would overflow int32 cannot be ordered:
@@ -57,15 +60,17 @@
 
 #include <algorithm>
 #include <climits>
+#include <type_traits>
 
 namespace ekv {
 namespace {
 
-constexpr int kThreads = 256;
-constexpr int kMaxCapacity = 8192;   // slots per hot buffer (stamps held in LDS; 16-bit scan fields)
+constexpr int kMaxCapacity = 8192;   // slots per hot buffer (touches held in LDS; 16-bit scan fields)
 constexpr int kMaxWidth = 4096;      // lanes per row whose miss tokens are hashed in LDS
-static_assert(kMaxWidth <= 16 * kThreads && kMaxCapacity <= 32 * kThreads,
-              "the kernel's register batches hold at most 16 lanes and 32 stamps per thread");
+constexpr int kDigits = 256;         // of one radix-select pass
+// Summary words (bits_shift 0), or groups of a coarse summary, that a row's changes are gathered over in LDS: 8 KiB,
+// contexts of 65,536 tokens at bits_shift 0 and 131,072 at 6. Longer rows take global atomics.
+constexpr int64_t kMaxGathered = 2048;
 // Stamps per LRU step: hits take step * kStepStamps + lane, misses
 // step * kStepStamps + kMaxWidth + lane, so a call with fewer lanes than the
 // one before still stamps above it.
@@ -111,58 +116,46 @@ struct SwapArgs {
     int64_t step;
     const int64_t* step_counter;    // when set, the step is read from device memory (graph replays)
     int32_t* status;                // EKV_SWAP_* error bits, OR-ed in (may be null)
-    uint32_t touched_words;         // ceil(C / 32): words of the touched-slot bits
+    uint32_t gathered;              // summary words (bits_shift 0) or line_counts groups kept in LDS (0: global atomics)
+    uint32_t info_words;            // words of the info region
     uint32_t hash_size, hash_log2;  // miss-token hash buckets: a power of two >= 2W (and >= 2)
     uint32_t token_bitmap;          // 1: T <= 16 * hash_size, the region first serves as a token bitmap
     uint32_t bitmap_words;          // ceil(T / 32)
 };
 
-// A Top-K id (int32 or int64 elements) without a branch on the element type:
-// the low word, then the high word (for int32 ids the low word again,
-// replaced by its sign). A branch per id would make the compiler wait for
-// each load before issuing the next.
-__device__ __forceinline__ int64_t load_id(const void* row, int32_t is64, int64_t index) {
-    const char* at = static_cast<const char*>(row) + index * (is64 ? 8 : 4);
-    const int32_t lo = *reinterpret_cast<const int32_t*>(at);
-    const int32_t high = *reinterpret_cast<const int32_t*>(at + (is64 ? 4 : 0));
-    return static_cast<int64_t>((static_cast<uint64_t>(static_cast<uint32_t>(is64 ? high : lo >> 31)) << 32) |
-                                static_cast<uint32_t>(lo));
-}
-
-// Writes a token -> slot table entry (int32 global slot or int16 local slot + 1).
-__device__ __forceinline__ void set_entry(const SwapArgs& a, int64_t offset, int32_t value) {
-    if (a.table16) {
-        static_cast<int16_t*>(a.table)[offset] = static_cast<int16_t>(value);
+// Element i of a row at `row`. Dense rows (unit strides, byte extents below
+// 4 GiB, checked by the host) take a 32-bit byte offset from the
+// workgroup-uniform row; other rows a 64-bit product per access, of which a
+// row of 4096 slots needs about sixty per thread.
+template <bool kDense, typename T>
+__device__ __forceinline__ T* element(T* row, int64_t stride, uint32_t i) {
+    if constexpr (kDense) {
+        using Byte = std::conditional_t<std::is_const_v<T>, const char, char>;
+        return reinterpret_cast<T*>(reinterpret_cast<Byte*>(row) + i * static_cast<uint32_t>(sizeof(T)));
     } else {
-        static_cast<int32_t*>(a.table)[offset] = value;
+        return row + static_cast<int64_t>(i) * stride;
     }
 }
 
-// Exclusive prefix sum of one int per thread over the workgroup (wave64
-// shuffles, then one LDS exchange of the wave totals); `total` receives the
-// sum. Every thread must call it.
-__device__ __forceinline__ int32_t workgroup_exclusive_scan(int32_t value, int32_t* wave_totals, int32_t& total) {
-    const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
-    int32_t inclusive = value;
-#pragma unroll
-    for (int offset = 1; offset < 64; offset <<= 1) {
-        const int32_t below = __shfl_up(inclusive, offset);
-        inclusive += lane >= offset ? below : 0;
+// The low 32 bits of element i of an int32 or int64 row, or (`high`) its high ones; no branch on the element type.
+template <bool kDense>
+__device__ __forceinline__ int32_t index_word(const void* row, int32_t is64, int64_t stride, uint32_t i, bool high) {
+    const char* at = static_cast<const char*>(row);
+    if constexpr (kDense) {
+        return *reinterpret_cast<const int32_t*>(at + ((i << (is64 ? 3 : 2)) + (high ? 4u : 0u)));
+    } else {
+        return *reinterpret_cast<const int32_t*>(at + i * stride * (is64 ? 8 : 4) + (high ? 4 : 0));
     }
-    if (lane == 63) {
-        wave_totals[wave] = inclusive;
+}
+
+// Writes a token -> slot table entry (int32 global slot or int16 local slot + 1) of the row starting at element `row`.
+template <bool kDense>
+__device__ __forceinline__ void set_entry(const SwapArgs& a, int64_t row, uint32_t token, int32_t value) {
+    if (a.table16) {
+        *element<kDense>(static_cast<int16_t*>(a.table) + row, a.tb_t, token) = static_cast<int16_t>(value);
+    } else {
+        *element<kDense>(static_cast<int32_t*>(a.table) + row, a.tb_t, token) = value;
     }
-    __syncthreads();
-    int32_t before = 0;
-    total = 0;
-#pragma unroll
-    for (int w = 0; w < kThreads / 64; ++w) {
-        before += w < wave ? wave_totals[w] : 0;
-        total += wave_totals[w];
-    }
-    __syncthreads();  // wave_totals may be rewritten by the next scan
-    return before + inclusive - value;
 }
 
 // A workgroup barrier that orders LDS only: waves wait for their own LDS
@@ -180,31 +173,94 @@ __device__ __forceinline__ int32_t lanes_below(uint64_t mask) {
                                                           __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(mask), 0u)));
 }
 
-// Sum, minimum and maximum of one value per thread over the workgroup
-// (wave shuffles, then one LDS exchange of the wave results). Every thread
-// must call it; `partial` holds 3 * (kThreads / 64) words.
-__device__ __forceinline__ void workgroup_sum_min_max(uint32_t& sum, uint32_t& lo, uint32_t& hi, uint32_t* partial) {
-#pragma unroll
-    for (int offset = 32; offset > 0; offset >>= 1) {
-        sum += __shfl_xor(sum, offset);
-        lo = min(lo, static_cast<uint32_t>(__shfl_xor(lo, offset)));
-        hi = max(hi, static_cast<uint32_t>(__shfl_xor(hi, offset)));
-    }
-    const int wave = threadIdx.x >> 6;
-    if ((threadIdx.x & 63) == 0) {
-        partial[3 * wave] = sum;
-        partial[3 * wave + 1] = lo;
-        partial[3 * wave + 2] = hi;
+// Inclusive scan of one value per lane over the wave, in six DPP steps (within
+// rows of 16 lanes, then row 0 to 1 and 2 to 3, then lane 31 to rows 2 and 3)
+// instead of six LDS permutes of a round trip each.
+enum WaveOp { kAdd, kMin, kMax };
+
+template <WaveOp kOp>
+__device__ __forceinline__ uint32_t wave_scan(uint32_t v) {
+    constexpr uint32_t kNone = kOp == kMin ? 0xffffffffu : 0u;   // what a lane without a source combines
+    const auto combine = [](uint32_t a, int b) {
+        const uint32_t other = static_cast<uint32_t>(b);
+        return kOp == kAdd ? a + other : (kOp == kMin ? min(a, other) : max(a, other));
+    };
+    constexpr int kRowShr = 0x110, kRowBcast15 = 0x142, kRowBcast31 = 0x143;   // DPP controls
+    v = combine(v, __builtin_amdgcn_update_dpp(static_cast<int>(kNone), static_cast<int>(v), kRowShr + 1, 0xf, 0xf, false));
+    v = combine(v, __builtin_amdgcn_update_dpp(static_cast<int>(kNone), static_cast<int>(v), kRowShr + 2, 0xf, 0xf, false));
+    v = combine(v, __builtin_amdgcn_update_dpp(static_cast<int>(kNone), static_cast<int>(v), kRowShr + 4, 0xf, 0xf, false));
+    v = combine(v, __builtin_amdgcn_update_dpp(static_cast<int>(kNone), static_cast<int>(v), kRowShr + 8, 0xf, 0xf, false));
+    v = combine(v, __builtin_amdgcn_update_dpp(static_cast<int>(kNone), static_cast<int>(v), kRowBcast15, 0xa, 0xf, false));
+    v = combine(v, __builtin_amdgcn_update_dpp(static_cast<int>(kNone), static_cast<int>(v), kRowBcast31, 0xc, 0xf, false));
+    return v;
+}
+
+// True in every thread when `value` is true in any. Every thread must call it
+// (one LDS barrier); `cells` holds one word per wave, used by this call only.
+template <int kWaves>
+__device__ __forceinline__ bool workgroup_any(bool value, uint32_t* cells) {
+    const uint32_t lane = threadIdx.x & 63;
+    const bool any = __ballot(value) != 0;
+    if (lane == 0) {
+        cells[threadIdx.x >> 6] = any ? 1u : 0u;
     }
     lds_barrier();
-    sum = 0;
-    lo = 0xffffffffu;
-    hi = 0;
+    return __ballot(lane < kWaves && cells[lane < kWaves ? lane : 0] != 0) != 0;
+}
+
+// Elements are held as register k of thread t = element t + k * threads, so
+// wave w's registers k cover consecutive elements. Each wave leaves its counts
+// (two 16-bit fields per word) of every register in `cells`; after a barrier,
+// pair_bases gives the count of all elements before register k of this wave.
+template <int kWaves, int kRegs>
+__device__ __forceinline__ void pair_counts(const uint32_t (&count)[kRegs], uint32_t* cells) {
+    if ((threadIdx.x & 63) == 0) {
 #pragma unroll
-    for (int w = 0; w < kThreads / 64; ++w) {
-        sum += partial[3 * w];
-        lo = min(lo, partial[3 * w + 1]);
-        hi = max(hi, partial[3 * w + 2]);
+        for (int k = 0; k < kRegs; ++k) {
+            cells[k * kWaves + (threadIdx.x >> 6)] = count[k];
+        }
+    }
+}
+
+template <int kWaves, int kRegs>
+__device__ __forceinline__ void pair_bases(const uint32_t* cells, uint32_t (&base)[kRegs], uint32_t& total) {
+    constexpr int kPairs = kWaves * kRegs;
+    constexpr int kPer = (kPairs + 63) / 64;
+    static_assert(kPer <= 2, "at most two cells per lane");
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+    uint32_t cell[kPer], sum = 0;
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+        const int at = lane * kPer + j;
+        cell[j] = cells[at < kPairs ? at : 0];
+        cell[j] = at < kPairs ? cell[j] : 0u;
+        sum += cell[j];
+    }
+    const uint32_t inclusive = wave_scan<kAdd>(sum);
+    const uint32_t before = inclusive - sum;
+    total = __builtin_amdgcn_readlane(inclusive, (kPairs - 1) / kPer);
+#pragma unroll
+    for (int k = 0; k < kRegs; ++k) {
+        const int pair = k * kWaves + wave;
+        base[k] = __builtin_amdgcn_readlane(before, pair / kPer);
+        if (kPer > 1 && (pair & 1)) {
+            base[k] += __builtin_amdgcn_readlane(cell[0], pair / kPer);
+        }
+    }
+}
+
+// Sum, minimum and maximum of one value per thread over the workgroup, added
+// to range[0..2] (starting at 0, all ones and 0) by each wave's last lane; read
+// them after a barrier. Every thread must call it.
+__device__ __forceinline__ void add_range(uint32_t sum, uint32_t lo, uint32_t hi, uint32_t* range) {
+    sum = wave_scan<kAdd>(sum);
+    lo = wave_scan<kMin>(lo);
+    hi = wave_scan<kMax>(hi);
+    if ((threadIdx.x & 63) == 63) {
+        atomicAdd(&range[0], sum);
+        atomicMin(&range[1], lo);
+        atomicMax(&range[2], hi);
     }
 }
 
@@ -260,7 +316,7 @@ __device__ __forceinline__ void bucket_min(uint32_t* words, uint32_t h, uint32_t
 // every probe meets its token or an empty bucket. Every thread must call it.
 __device__ __forceinline__ void hash_miss_tokens(uint32_t* hash, const int32_t* info, int32_t m, uint32_t log2_size) {
     const uint32_t mask = (1u << log2_size) - 1u;
-    for (int32_t i = threadIdx.x; i < m; i += kThreads) {
+    for (int32_t i = threadIdx.x; i < m; i += blockDim.x) {
         const int32_t token = info[i];
         if (token < 0) {
             continue;
@@ -281,15 +337,26 @@ __device__ __forceinline__ void hash_miss_tokens(uint32_t* hash, const int32_t* 
 }
 
 // Dynamic LDS of one workgroup (C = capacity, W = lanes per row):
-//   stamp    int32 [C]  recency stamps;
-//   info     int32 [W]  token of miss i (-1: an entry naming no valid lane);
-//   touched  uint32 [ceil(C / 32)]  one bit per slot a hit touches;
-//   region   hash_size 16-bit buckets (the miss-token hash), then the int16
+//   touch    int32 [C]  lowest lane that hits the slot (INT32_MAX: none), then the new stamp of a victim;
+//   info     int32 [W]  when tokens repeat: token of miss i (-1: an entry naming no valid lane),
+//            then int16 [W], the victim's rank of a first miss, and behind it
+//   summary  int32 [gathered]  the row's summary words, or the changes of its groups' counts;
+//   region   the token bitmap, or hash_size 16-bit buckets (the miss-token hash), then the int16
 //            list of the victims' slots in slot order;
-//   owner    int16 [W]  the first miss of the same token (-1: an entry naming
-//            no valid lane); a first miss's own entry then becomes -2 - the
-//            rank of its victim.
-// 36.5 KiB at C = 4096, W = 2048, so 4 workgroups share a CU.
+//
+// What bounds it. A row is a chain of about ten barrier-separated phases over
+// a few KiB of LDS, so what counts is how short a phase's code is and how many waves
+// share it: a thread holds kSlotRegs stamps and kLaneRegs lanes in registers,
+// and the host picks the workgroup size that gives four and two (threads of
+// 64 to 1024). With 256 threads for every shape a row of 4096 slots was 16
+// and 8 registers of unrolled code, 53 KB of instructions fetched once per
+// row, and the same code ran for a row of 256 slots. Scans are DPP steps,
+// the summary is changed in LDS and written once, and dense rows are addressed
+// with 32-bit offsets. With the launch, against those 256 threads and global
+// atomics: 48 rows of 1024 lanes (2048 slots) 27.2 -> 14.4 us, 2560 rows of 256 lanes
+// 77.3 -> 26.3, of 2048 lanes 187.9 -> 115.1. The last moves 246 MB from and
+// 215 MB to HBM by the counters (scattered table entries as whole lines), 84 us
+// at the rate of a copy.
 //
 // Global reads come in three batches, each issued as a fixed number of
 // unrolled loads from clamped, in-bounds addresses and waited for once: the
@@ -297,22 +364,21 @@ __device__ __forceinline__ void hash_miss_tokens(uint32_t* hash, const int32_t* 
 // ids of the miss entries; the victims' old tokens and host rows. (A loop
 // with a run-time trip count waits for each load before issuing the next: a
 // workgroup then spends most of its life on a chain of HBM round trips.)
-// kSlotRegs >= C / kThreads stamps and kLaneRegs >= W / kThreads lanes per
-// thread are held in registers.
-template <int kSlotRegs, int kLaneRegs>
+template <int kThreads, int kSlotRegs, int kLaneRegs, bool kDense>
 __global__ __launch_bounds__(kThreads) void swap_in_kernel(const SwapArgs a) {
+    constexpr int kWaves = kThreads / 64;
+    constexpr uint32_t kReadAhead = 4;     // summary words or group counts per thread that are read ahead
     extern __shared__ __align__(16) unsigned char shared[];
-    __shared__ int32_t wave_totals[kThreads / 64];
-    __shared__ int32_t digit_count[2][256];   // radix-select histograms of one 8-bit digit (two passes)
-    __shared__ int32_t chosen[2];          // the digit holding the need-th key, and the keys below it
-    __shared__ uint32_t key_range[3 * (kThreads / 64)];   // empties, smallest and largest other key per wave
-    __shared__ int32_t row_counts[2][kSlotRegs][kThreads / 64];   // keys below T / at T per (row, wave)
-    int32_t* stamp = reinterpret_cast<int32_t*>(shared);
-    int32_t* info = stamp + a.capacity;
-    uint32_t* touched = reinterpret_cast<uint32_t*>(info + a.width);
-    uint32_t* hash = touched + a.touched_words;
+    __shared__ __align__(16) int32_t digit_count[2 * kDigits];   // radix-select histograms of two passes
+    __shared__ uint32_t key_range[3];      // empties, smallest and largest other key
+    __shared__ uint32_t first_cells[kLaneRegs * kWaves], victim_cells[kSlotRegs * kWaves];
+    __shared__ uint32_t any_cells[2][kWaves];
+    int32_t* touch = reinterpret_cast<int32_t*>(shared);
+    int32_t* info = touch + a.capacity;
+    int16_t* owner = reinterpret_cast<int16_t*>(info);   // the tokens are in registers again by then
+    int32_t* summary = info + (a.width + 1) / 2;
+    uint32_t* hash = reinterpret_cast<uint32_t*>(info + a.info_words);
     int16_t* victims = reinterpret_cast<int16_t*>(hash);
-    int16_t* owner = reinterpret_cast<int16_t*>(hash + a.hash_size / 2);
     // The prologue's reads are vector loads issued together: as scalar loads
     // (uniform reads) the compiler waited for each before the next one, and
     // the selection entry, request row, miss count, step and slot base were a
@@ -379,16 +445,16 @@ __global__ __launch_bounds__(kThreads) void swap_in_kernel(const SwapArgs a) {
     int32_t held_stamp[kSlotRegs];
 #pragma unroll
     for (int k = 0; k < kSlotRegs; ++k) {
-        const int64_t s = min(static_cast<int64_t>(threadIdx.x) + int64_t{k} * kThreads, C - 1);
-        held_stamp[k] = stamps[s * a.sp_c];
+        const uint32_t s = min(threadIdx.x + k * kThreads, static_cast<uint32_t>(C) - 1);
+        held_stamp[k] = *element<kDense>(stamps, a.sp_c, s);
     }
     int32_t lane_slot[kLaneRegs];
     int32_t miss_lane[kLaneRegs];
 #pragma unroll
     for (int k = 0; k < kLaneRegs; ++k) {
-        const int64_t o = min(static_cast<int64_t>(threadIdx.x) + int64_t{k} * kThreads, W - 1);
-        lane_slot[k] = slots[o * a.sl_o];
-        miss_lane[k] = misses[o * a.mi_o];   // entries at or past the count are read but not used
+        const uint32_t o = min(threadIdx.x + k * kThreads, a.width - 1);
+        lane_slot[k] = *element<kDense>(slots, a.sl_o, o);
+        miss_lane[k] = *element<kDense>(misses, a.mi_o, o);   // entries at or past the count are read but not used
     }
     const bool first_in_range =
         first_j < selected_count && first_j != blockIdx.x && first_other >= 0 && first_other < a.batch;
@@ -399,15 +465,55 @@ __global__ __launch_bounds__(kThreads) void swap_in_kernel(const SwapArgs a) {
         shared_request |= j != blockIdx.x && other >= 0 && other < a.batch && a.rows[other] == req;
     }
     // Batch 2: the Top-K ids of the miss entries.
-    int64_t miss_block[kLaneRegs];
+    int32_t block_low[kLaneRegs], block_high[kLaneRegs];
 #pragma unroll
     for (int k = 0; k < kLaneRegs; ++k) {
         const uint32_t lane = static_cast<uint32_t>(min(max(miss_lane[k], 0), static_cast<int32_t>(W - 1)));
         const uint32_t blk = a.block_size == 1 ? lane : a.block_div.div(lane);
-        miss_block[k] = load_id(topk_row, a.topk64, blk * a.topk_sk);
+        block_low[k] = index_word<kDense>(topk_row, a.topk64, a.topk_sk, blk, false);
+        block_high[k] = index_word<kDense>(topk_row, a.topk64, a.topk_sk, blk, a.topk64 != 0);
     }
     const int32_t m = counted < 0 ? 0 : (counted > W ? static_cast<int32_t>(W) : counted);
-    shared_request = __syncthreads_or(shared_request);
+    // LDS starts, published by the barrier of the request check: nothing touched, the region a token bitmap (all clear)
+    // when the tokens fit it, else the empty hash.
+#pragma unroll
+    for (int k = 0; k < kSlotRegs; ++k) {
+        const uint32_t s = threadIdx.x + k * kThreads;
+        if (s < C) {
+            touch[s] = INT32_MAX;
+        }
+    }
+    const uint32_t region_words = a.token_bitmap ? a.bitmap_words : a.hash_size / 2;
+    const uint32_t region_fill = a.token_bitmap ? 0u : 0xffffffffu;
+    for (uint32_t w = threadIdx.x; w < region_words; w += kThreads) {
+        hash[w] = region_fill;
+    }
+    for (uint32_t d = threadIdx.x; d < 2 * kDigits; d += kThreads) {
+        digit_count[d] = 0;
+    }
+    if (threadIdx.x < 3) {
+        key_range[threadIdx.x] = threadIdx.x == 1 ? 0xffffffffu : 0u;
+    }
+    // The row's summary words, or its groups' counts, read ahead of their use.
+    int32_t* bits = a.bits != nullptr ? a.bits + l * a.bt_l + req * a.bt_r : nullptr;
+    // Group counts keep a coarse summary exact: their changes gathered in LDS and applied once per group, or
+    // decremented and incremented in place around a barrier.
+    int32_t* line_counts = bits != nullptr && a.bits_shift > 0 && a.line_counts != nullptr
+                               ? a.line_counts + l * a.lc_l + req * a.lc_r
+                               : nullptr;
+    const uint32_t gathered = a.gathered;   // 0 without a summary
+    int32_t* const state = line_counts != nullptr ? line_counts : bits;
+    const int64_t state_stride = line_counts != nullptr ? a.lc_q : a.bt_w;
+    int32_t held_state[kReadAhead];
+#pragma unroll
+    for (uint32_t g = 0; g < kReadAhead; ++g) {
+        const uint32_t q = threadIdx.x + g * kThreads;
+        held_state[g] = 0;
+        if (gathered > 0) {   // uniform
+            held_state[g] = *element<kDense>(state, state_stride, q < gathered ? q : gathered - 1);
+        }
+    }
+    shared_request = workgroup_any<kWaves>(shared_request, any_cells[0]);
     const bool overflow = step < 0 || (step + 1) * kStepStamps >= (int64_t{1} << 31);
     if (shared_request || overflow) {
         // Change nothing, record empty promotions (the move that follows
@@ -421,171 +527,144 @@ __global__ __launch_bounds__(kThreads) void swap_in_kernel(const SwapArgs a) {
         }
         return;
     }
-    const int64_t stamp_base = step * kStepStamps;
-#pragma unroll
-    for (int k = 0; k < kSlotRegs; ++k) {
-        const int64_t s = threadIdx.x + int64_t{k} * kThreads;
-        if (s < C) {
-            stamp[s] = held_stamp[k];
-        }
-    }
+    const int32_t stamp_base = static_cast<int32_t>(step * kStepStamps);
     const int64_t base = index_value(a.slot_base, base_read);
-    int32_t hit_local[kLaneRegs];   // local slot a lane hits, or -1
-#pragma unroll
-    for (int k = 0; k < kLaneRegs; ++k) {
-        const int64_t o = threadIdx.x + int64_t{k} * kThreads;
-        const int64_t offset = static_cast<int64_t>(lane_slot[k]) - base;
-        hit_local[k] = o < W && lane_slot[k] > 0 && offset >= 0 && offset < C ? static_cast<int32_t>(offset) : -1;
-        const int64_t i = o;   // this thread's k-th miss-list entry
-        if (i < m) {
-            const int32_t lane = miss_lane[k];
-            const int64_t offset_in_block =
-                a.block_size == 1 ? 0 : static_cast<int64_t>(lane) - int64_t{a.block_div.div(static_cast<uint32_t>(lane))} *
-                                                                          a.block_size;
-            const int64_t token = lane >= 0 && lane < W ? miss_block[k] * a.block_size + offset_in_block : int64_t{-1};
-            info[i] = token >= 0 && token < a.table_cols ? static_cast<int32_t>(token) : -1;
-        }
-    }
-    for (uint32_t w = threadIdx.x; w < a.touched_words; w += kThreads) {
-        touched[w] = 0;
-    }
-    // The region starts as a token bitmap (all clear) when the tokens fit it,
-    // else as the empty hash.
-    const uint32_t region_words = a.token_bitmap ? a.bitmap_words : a.hash_size / 2;
-    const uint32_t region_fill = a.token_bitmap ? 0u : 0xffffffffu;
-    for (uint32_t w = threadIdx.x; w < region_words; w += kThreads) {
-        hash[w] = region_fill;
-    }
-    __syncthreads();
-    // Touch hits. A token repeated in the row is one access of its first lane:
-    // a touched slot's stamp becomes stamp_base + the lowest lane that hit it
-    // (marked, raised to INT32_MAX, then lowered by every hitting lane).
-#pragma unroll
-    for (int k = 0; k < kLaneRegs; ++k) {
-        if (hit_local[k] >= 0) {
-            atomicOr(&touched[hit_local[k] >> 5], 1u << (hit_local[k] & 31));
-        }
-    }
-    // Repeated miss tokens. With the token bitmap, each valid entry sets its
-    // token's bit; a bit found set means some token repeats, and only then is
-    // the exact hash built (each token's lowest miss index). Without repeats
-    // every valid entry is its token's first miss.
+    // Touch hits: a token repeated in the row is one access of its first lane. Repeated miss tokens: with the token
+    // bitmap, each valid entry sets its token's bit; a bit found set means some token repeats, and only then is the
+    // exact hash built (each token's lowest miss index). Without repeats every valid entry is its token's first miss.
+    int32_t token_of[kLaneRegs];   // token of this thread's k-th miss entry, or -1
+    int32_t first_of[kLaneRegs];   // the first miss of that token, or -1
     bool repeated = false;
-    if (a.token_bitmap) {   // uniform
+#pragma unroll
+    for (int k = 0; k < kLaneRegs; ++k) {
+        const int32_t o = static_cast<int32_t>(threadIdx.x) + k * kThreads;
+        const int64_t offset = static_cast<int64_t>(lane_slot[k]) - base;
+        if (o < W && lane_slot[k] > 0 && offset >= 0 && offset < C) {
+            atomicMin(&touch[static_cast<uint32_t>(offset)], o);
+        }
+        // The entry's token: its block id times the block size, and the lane's place in the block.
+        const int32_t lane = miss_lane[k];
+        const int32_t high = a.topk64 ? block_high[k] : block_low[k] >> 31;
+        int64_t token = static_cast<int64_t>(static_cast<uint64_t>(static_cast<uint32_t>(high)) << 32 |
+                                             static_cast<uint32_t>(block_low[k]));
+        if (a.block_size != 1) {   // uniform
+            token = token * a.block_size +
+                    (static_cast<uint32_t>(lane) - a.block_div.div(static_cast<uint32_t>(lane)) * a.block_size);
+        }
+        const bool valid = o < m && lane >= 0 && lane < W && token >= 0 && token < a.table_cols;
+        token_of[k] = valid ? static_cast<int32_t>(token) : -1;
+        first_of[k] = valid ? o : -1;
+        if (a.token_bitmap && token_of[k] >= 0) {
+            const uint32_t bit = 1u << (token_of[k] & 31);
+            repeated |= (atomicOr(&hash[token_of[k] >> 5], bit) & bit) != 0u;
+        }
+    }
+    const bool exact_hash = workgroup_any<kWaves>(repeated, any_cells[1]) || !a.token_bitmap;   // uniform
+    if (exact_hash) {
 #pragma unroll
         for (int k = 0; k < kLaneRegs; ++k) {
             const int32_t i = static_cast<int32_t>(threadIdx.x) + k * kThreads;
-            const int32_t token = i < m ? info[i] : -1;
-            if (token >= 0) {
-                const uint32_t bit = 1u << (token & 31);
-                repeated |= (atomicOr(&hash[token >> 5], bit) & bit) != 0u;
+            if (i < m) {
+                info[i] = token_of[k];
             }
         }
-    } else {
+        if (a.token_bitmap) {
+            for (uint32_t w = threadIdx.x; w < a.hash_size / 2; w += kThreads) {
+                hash[w] = 0xffffffffu;
+            }
+        }
+        lds_barrier();
         hash_miss_tokens(hash, info, m, a.hash_log2);
-    }
-    const bool exact_hash = !a.token_bitmap || __syncthreads_or(repeated);   // uniform
-    if (a.token_bitmap && exact_hash) {
-        for (uint32_t w = threadIdx.x; w < a.hash_size / 2; w += kThreads) {
-            hash[w] = 0xffffffffu;
-        }
-        __syncthreads();
-        hash_miss_tokens(hash, info, m, a.hash_log2);
-    }
-    __syncthreads();
+        lds_barrier();
+        const uint32_t mask = a.hash_size - 1;
 #pragma unroll
-    for (int k = 0; k < kSlotRegs; ++k) {
-        const uint32_t s = threadIdx.x + k * kThreads;
-        if (s < C && ((touched[s >> 5] >> (s & 31)) & 1u)) {
-            stamp[s] = INT32_MAX;
-        }
-    }
-    const uint32_t mask = a.hash_size - 1;
-#pragma unroll
-    for (int k = 0; k < kLaneRegs; ++k) {
-        const int32_t i = static_cast<int32_t>(threadIdx.x) + k * kThreads;
-        if (i >= m) {
-            continue;
-        }
-        const int32_t token = info[i];
-        int32_t first = -1;
-        if (token >= 0 && !exact_hash) {
-            first = i;
-        } else if (token >= 0) {
-            for (uint32_t h = token_hash(token, a.hash_log2);; h = (h + 1) & mask) {
+        for (int k = 0; k < kLaneRegs; ++k) {
+            if (token_of[k] < 0) {
+                continue;
+            }
+            for (uint32_t h = token_hash(token_of[k], a.hash_log2);; h = (h + 1) & mask) {
                 const uint32_t held = bucket_of(hash, h);
                 if (held == kEmptyBucket) {
                     break;   // not reached: every inserted token lies on its probe path
                 }
-                if (info[held] == token) {
-                    first = static_cast<int32_t>(held);
+                if (info[held] == token_of[k]) {
+                    first_of[k] = static_cast<int32_t>(held);
                     break;
                 }
             }
         }
-        owner[i] = static_cast<int16_t>(first);
     }
-    __syncthreads();
+    // This thread's keys, slots t + k * kThreads, in the order-preserving
+    // unsigned form of the stamps (an empty slot is key 0): a touched slot's
+    // stamp is stamp_base + its first lane, any other keeps what it held.
+    uint32_t key[kSlotRegs];
 #pragma unroll
-    for (int k = 0; k < kLaneRegs; ++k) {
-        if (hit_local[k] >= 0) {
-            atomicMin(&stamp[hit_local[k]],
-                      static_cast<int32_t>(stamp_base + threadIdx.x + static_cast<int64_t>(k) * kThreads));
-        }
+    for (int k = 0; k < kSlotRegs; ++k) {
+        const uint32_t s = threadIdx.x + k * kThreads;
+        const int32_t hit = s < C ? touch[s] : INT32_MAX;
+        const int32_t stamp = hit != INT32_MAX ? stamp_base + hit : held_stamp[k];
+        key[k] = s < C ? static_cast<uint32_t>(stamp) ^ 0x80000000u : 0xffffffffu;
     }
-    if (m > 0) {
-        // Rank of each first miss among the first misses, in miss-list order:
-        // every thread counts a contiguous run of entries, one scan. (The
-        // scan's barriers also order the touches above before the select.)
-        const int32_t per_thread = (m + kThreads - 1) / kThreads;
-        const int32_t run_begin = min(m, static_cast<int32_t>(threadIdx.x) * per_thread);
-        const int32_t run_end = min(m, run_begin + per_thread);
-        int32_t firsts = 0;
-        for (int32_t i = run_begin; i < run_end; ++i) {
-            firsts += owner[i] == i;
+    uint32_t chosen = 0;   // bit k: slot t + k * kThreads is a victim
+    if (m > 0) {   // uniform
+        // Rank of each first miss among the first misses, in miss-list order,
+        // and the range of the keys, over one barrier.
+        uint32_t first_count[kLaneRegs], rank_of[kLaneRegs], unique = 0;
+#pragma unroll
+        for (int k = 0; k < kLaneRegs; ++k) {
+            const bool first = first_of[k] >= 0 && first_of[k] == static_cast<int32_t>(threadIdx.x) + k * kThreads;
+            first_count[k] = __popcll(__ballot(first));
         }
-        int32_t unique = 0;
-        int32_t rank = workgroup_exclusive_scan(firsts, wave_totals, unique);
-        for (int32_t i = run_begin; i < run_end; ++i) {
-            if (owner[i] == i) {
-                owner[i] = static_cast<int16_t>(-2 - rank++);   // a first miss: its victim's rank, below -1
+        pair_counts<kWaves, kLaneRegs>(first_count, first_cells);
+        uint32_t empties = 0, lo = 0xffffffffu, hi = 0;
+#pragma unroll
+        for (int k = 0; k < kSlotRegs; ++k) {
+            const uint32_t v = key[k];
+            const bool other = v != 0 && threadIdx.x + k * kThreads < C;
+            empties += v == 0 ? 1u : 0u;
+            lo = other ? min(lo, v) : lo;
+            hi = other ? max(hi, v) : hi;
+        }
+        add_range(empties, lo, hi, key_range);
+        lds_barrier();
+        // The info region is free of tokens now: summary words are changed in
+        // place, counts' changes start at zero (published by the victims' barrier).
+#pragma unroll
+        for (uint32_t g = 0; g < kReadAhead; ++g) {
+            const uint32_t q = threadIdx.x + g * kThreads;
+            if (q < gathered) {
+                summary[q] = line_counts != nullptr ? 0 : held_state[g];
+            }
+        }
+        for (uint32_t q = threadIdx.x + kReadAhead * kThreads; q < gathered; q += kThreads) {
+            summary[q] = line_counts != nullptr ? 0 : *element<kDense>(state, state_stride, q);
+        }
+        pair_bases<kWaves, kLaneRegs>(first_cells, rank_of, unique);
+        empties = key_range[0], lo = key_range[1], hi = key_range[2];
+#pragma unroll
+        for (int k = 0; k < kLaneRegs; ++k) {
+            const int32_t i = static_cast<int32_t>(threadIdx.x) + k * kThreads;
+            const bool first = first_of[k] >= 0 && first_of[k] == i;
+            rank_of[k] += lanes_below(__ballot(first));
+            if (exact_hash && first) {
+                owner[i] = static_cast<int16_t>(rank_of[k]);   // read by repeats past the next barriers
             }
         }
         // The `unique` victims: the slots of the smallest (stamp, slot) keys,
-        // empty slots (INT32_MIN) first, then the least recently used. In
-        // the order-preserving unsigned form of the stamps an empty slot is
-        // key 0. When the empties do not cover the victims, a radix select
-        // over the other keys (8-bit digits, most significant first) finds
-        // the key T of the (unique - empties)-th smallest of them and how
-        // many keys at T it takes; it starts at the highest digit where the
-        // smallest and largest of those keys differ (the stamps of a buffer
-        // span a few steps: two digits). The victims are then listed in slot
-        // order, and the i-th first miss takes the i-th of them.
+        // empty slots (INT32_MIN) first, then the least recently used. When
+        // the empties do not cover the victims, a radix select over the other
+        // keys (8-bit digits, most significant first) finds the key T of the
+        // (unique - empties)-th smallest of them and how many keys at T it
+        // takes; it starts at the highest digit where the smallest and largest
+        // of those keys differ (the stamps of a buffer span a few steps: two
+        // digits). The victims are then listed in slot order, and the i-th
+        // first miss takes the i-th of them.
         if (unique > 0) {   // uniform
-            // This thread's keys, slots t + 256 k, read once (the touches
-            // landed before the rank scan's barriers); 0xffffffff past C.
-            uint32_t key[kSlotRegs];
-#pragma unroll
-            for (int k = 0; k < kSlotRegs; ++k) {
-                const uint32_t s = threadIdx.x + k * kThreads;
-                key[k] = s < C ? static_cast<uint32_t>(stamp[s]) ^ 0x80000000u : 0xffffffffu;
-            }
-            digit_count[0][threadIdx.x] = 0;   // the first pass's histogram; the reduction's barrier follows
-            uint32_t empties = 0, lo = 0xffffffffu, hi = 0;
-#pragma unroll
-            for (int k = 0; k < kSlotRegs; ++k) {
-                const uint32_t v = key[k];
-                const bool other = v != 0 && threadIdx.x + k * kThreads < C;
-                empties += v == 0 ? 1u : 0u;
-                lo = other ? min(lo, v) : lo;
-                hi = other ? max(hi, v) : hi;
-            }
-            workgroup_sum_min_max(empties, lo, hi, key_range);
             uint32_t prefix = 0, prefix_mask = 0xffffffffu;
-            int32_t need = unique;   // keys still to take at the prefix (uniform)
+            uint32_t need = unique;  // keys still to take at the prefix (uniform)
             int first_shift = -8;    // no select: the empties alone, or every other key equal
-            if (static_cast<uint32_t>(unique) > empties) {
-                need = unique - static_cast<int32_t>(empties);
+            if (unique > empties) {
+                need = unique - empties;
                 const uint32_t differ = lo ^ hi;
                 prefix = lo;
                 if (differ != 0) {
@@ -595,7 +674,13 @@ __global__ __launch_bounds__(kThreads) void swap_in_kernel(const SwapArgs a) {
                 }
             }
             for (int shift = first_shift, pass = 0; shift >= 0; shift -= 8, ++pass) {
-                int32_t* count = digit_count[pass & 1];
+                int32_t* count = digit_count + (pass & 1) * kDigits;
+                if (pass >= 2) {   // uniform: the histogram of two passes ago, read by every wave before the last barrier
+                    for (uint32_t d = threadIdx.x; d < kDigits; d += kThreads) {
+                        count[d] = 0;
+                    }
+                    lds_barrier();
+                }
                 // Runs of one digit in a thread's slots count with one atomic:
                 // recent stamps share their high digits, which would otherwise
                 // serialize thousands of atomics on one counter.
@@ -618,128 +703,68 @@ __global__ __launch_bounds__(kThreads) void swap_in_kernel(const SwapArgs a) {
                     atomicAdd(&count[run_digit], run);
                 }
                 lds_barrier();
-                // Wave 0 scans the 256 counts (4 digits per lane) and names the
-                // digit holding the need-th key; the others clear the next
-                // pass's histogram meanwhile.
-                if (threadIdx.x < 64) {
-                    int32_t c[4];
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        c[j] = count[4 * threadIdx.x + j];
-                    }
-                    const int32_t mine = c[0] + c[1] + c[2] + c[3];
-                    int32_t inclusive = mine;
-#pragma unroll
-                    for (int offset = 1; offset < 64; offset <<= 1) {
-                        const int32_t lower = __shfl_up(inclusive, offset);
-                        inclusive += threadIdx.x >= static_cast<uint32_t>(offset) ? lower : 0;
-                    }
-                    int32_t below = inclusive - mine;
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        if (below < need && need <= below + c[j]) {   // exactly one digit holds the need-th key
-                            chosen[0] = static_cast<int32_t>(4 * threadIdx.x + j);
-                            chosen[1] = below;
-                        }
-                        below += c[j];
-                    }
-                }
-                for (uint32_t d = threadIdx.x; d < 256; d += kThreads) {
-                    digit_count[(pass + 1) & 1][d] = 0;
-                }
-                lds_barrier();
-                prefix |= static_cast<uint32_t>(chosen[0]) << shift;
+                // Every wave scans the 256 counts itself (4 digits per lane)
+                // and finds the digit holding the need-th key: no second barrier.
+                const uint32_t lane = threadIdx.x & 63;
+                const int4 c = reinterpret_cast<const int4*>(count)[lane];
+                const uint32_t c0 = c.x, c1 = c0 + c.y, c2 = c1 + c.z, c3 = c2 + c.w;
+                const uint32_t inclusive = wave_scan<kAdd>(c3);
+                const uint32_t below = inclusive - c3;
+                const uint64_t holds = __ballot(below < need && need <= inclusive);   // exactly one lane
+                const int holder = __ffsll(static_cast<unsigned long long>(holds)) - 1;
+                const uint32_t rest = need - below;   // in the holder: 1..c3
+                const uint32_t j = rest <= c0 ? 0u : (rest <= c1 ? 1u : (rest <= c2 ? 2u : 3u));
+                const uint32_t skipped = below + (j == 0 ? 0u : (j == 1 ? c0 : (j == 2 ? c1 : c2)));
+                prefix |= (4u * holder + __builtin_amdgcn_readlane(j, holder)) << shift;
                 prefix_mask |= 255u << shift;
-                need -= chosen[1];
+                need -= __builtin_amdgcn_readlane(skipped, holder);
             }
             // T = prefix. Slot s is a victim when its key is below T (every
             // empty slot, when the empties do not cover the victims), or at T
             // and fewer than `need` slots below s hold T; its place in the list
-            // is the number of victims below it. Thread t takes slots
-            // t + 256 k (conflict-free LDS reads); the slot-order counts of
-            // both kinds come from per-wave ballots over each row of 256 slots.
-            const int wave = threadIdx.x >> 6;
-            uint32_t my_lower = 0, my_tie = 0;
+            // is the number of victims below it. The slot-order counts of both
+            // kinds (16 bits each) come from per-wave ballots.
+            uint32_t kinds[kSlotRegs], before[kSlotRegs], all = 0;
+#pragma unroll
+            for (int k = 0; k < kSlotRegs; ++k) {
+                const bool in = threadIdx.x + k * kThreads < C;
+                kinds[k] = static_cast<uint32_t>(__popcll(__ballot(in && key[k] < prefix))) |
+                           static_cast<uint32_t>(__popcll(__ballot(in && key[k] == prefix))) << 16;
+            }
+            pair_counts<kWaves, kSlotRegs>(kinds, victim_cells);
+            lds_barrier();
+            pair_bases<kWaves, kSlotRegs>(victim_cells, before, all);
 #pragma unroll
             for (int k = 0; k < kSlotRegs; ++k) {
                 const uint32_t s = threadIdx.x + k * kThreads;
-                const uint32_t v = key[k];
-                const bool lower = s < C && v < prefix;
-                const bool tie = s < C && v == prefix;
-                const uint64_t lower_lanes = __ballot(lower);
-                const uint64_t tie_lanes = __ballot(tie);
-                my_lower |= lower ? 1u << k : 0u;
-                my_tie |= tie ? 1u << k : 0u;
-                if ((threadIdx.x & 63) == 0) {
-                    row_counts[0][k][wave] = __popcll(lower_lanes);
-                    row_counts[1][k][wave] = __popcll(tie_lanes);
-                }
-            }
-            lds_barrier();
-            // Lane j < kSlotRegs of each wave takes row j: its keys of each kind
-            // in all waves and in the waves below this one; a shuffle scan over
-            // the lanes adds the rows below j, and the row loop reads row k's
-            // base from lane k.
-            const int lane = threadIdx.x & 63;
-            int32_t row_lower = 0, row_tie = 0, wave_lower = 0, wave_tie = 0;
-            if (lane < kSlotRegs) {
-#pragma unroll
-                for (int w = 0; w < kThreads / 64; ++w) {
-                    const int32_t lower_here = row_counts[0][lane][w];
-                    const int32_t tie_here = row_counts[1][lane][w];
-                    row_lower += lower_here;
-                    row_tie += tie_here;
-                    wave_lower += w < wave ? lower_here : 0;
-                    wave_tie += w < wave ? tie_here : 0;
-                }
-            }
-            int32_t lower_scan = row_lower, tie_scan = row_tie;
-#pragma unroll
-            for (int offset = 1; offset < kSlotRegs; offset <<= 1) {
-                const int32_t lower_up = __shfl_up(lower_scan, offset);
-                const int32_t tie_up = __shfl_up(tie_scan, offset);
-                lower_scan += lane >= offset ? lower_up : 0;
-                tie_scan += lane >= offset ? tie_up : 0;
-            }
-            const int32_t lower_base = lower_scan - row_lower + wave_lower;   // row `lane`'s base for this wave
-            const int32_t tie_base = tie_scan - row_tie + wave_tie;
-#pragma unroll
-            for (int k = 0; k < kSlotRegs; ++k) {
-                const bool lower = (my_lower >> k) & 1u;
-                const bool tie = (my_tie >> k) & 1u;
-                const int32_t lower_before = __builtin_amdgcn_readlane(lower_base, k) + lanes_below(__ballot(lower));
-                const int32_t ties_before = __builtin_amdgcn_readlane(tie_base, k) + lanes_below(__ballot(tie));
+                const bool lower = s < C && key[k] < prefix;
+                const bool tie = s < C && key[k] == prefix;
+                const uint32_t lower_before = (before[k] & 0xffffu) + lanes_below(__ballot(lower));
+                const uint32_t ties_before = (before[k] >> 16) + lanes_below(__ballot(tie));
                 if (lower || (tie && ties_before < need)) {
-                    victims[lower_before + min(ties_before, need)] = static_cast<int16_t>(threadIdx.x + k * kThreads);
+                    victims[lower_before + min(ties_before, need)] = static_cast<int16_t>(s);
+                    chosen |= 1u << k;
                 }
             }
-            lds_barrier();
         }
-        int32_t* bits = a.bits != nullptr ? a.bits + l * a.bt_l + req * a.bt_r : nullptr;
-        // Group counts keep a coarse summary exact: decrements here, increments after the barrier.
-        int32_t* line_counts = bits != nullptr && a.bits_shift > 0 && a.line_counts != nullptr
-                                   ? a.line_counts + l * a.lc_l + req * a.lc_r
-                                   : nullptr;
+        lds_barrier();   // the victims (and the ranks of repeated tokens) are read by other threads below
         // Batch 3: each entry's victim (from LDS), then the victims' old
         // tokens and the promoted tokens' host rows, all loads issued before
-        // any is used. Entry encoding: -1 names no valid lane; <= -2 is a
-        // first miss, whose victim has rank -2 - entry; otherwise the index
-        // of its first miss.
-        int32_t entry_of[kLaneRegs];
+        // any is used.
+        const char* host_row = static_cast<const char*>(a.host_table.data) +
+                               req * a.host_sr * (a.host_table.is64 ? 8 : 4);
         int32_t victim_of[kLaneRegs];
         int32_t old_of[kLaneRegs];
         int32_t host_row_of[kLaneRegs];
 #pragma unroll
         for (int k = 0; k < kLaneRegs; ++k) {
             const int32_t i = static_cast<int32_t>(threadIdx.x) + k * kThreads;
-            const int32_t entry = i < m ? static_cast<int32_t>(owner[i]) : -1;
-            const int32_t rank = entry == -1 ? 0 : -2 - (entry <= -2 ? entry : static_cast<int32_t>(owner[entry]));
-            const int32_t victim = entry == -1 ? 0 : static_cast<int32_t>(static_cast<uint16_t>(victims[rank]));
-            const int64_t token = entry == -1 ? 0 : info[i];   // >= 0 for an entry with a valid lane
-            entry_of[k] = entry;
-            victim_of[k] = victim;
-            old_of[k] = slot_token[static_cast<int64_t>(victim) * a.st_c];
-            host_row_of[k] = a.host_table.low(req * a.host_sr + token * a.host_st);
+            const bool valid = token_of[k] >= 0;
+            const uint32_t rank = first_of[k] == i ? rank_of[k] : (valid ? static_cast<uint32_t>(owner[first_of[k]]) : 0u);
+            victim_of[k] = valid ? static_cast<int32_t>(victims[rank]) : 0;
+            old_of[k] = *element<kDense>(slot_token, a.st_c, static_cast<uint32_t>(victim_of[k]));
+            host_row_of[k] = index_word<kDense>(host_row, a.host_table.is64, a.host_st,
+                                                valid ? static_cast<uint32_t>(token_of[k]) : 0u, false);
         }
 #pragma unroll
         for (int k = 0; k < kLaneRegs; ++k) {
@@ -747,31 +772,28 @@ __global__ __launch_bounds__(kThreads) void swap_in_kernel(const SwapArgs a) {
             if (i >= m) {
                 continue;
             }
-            const int32_t entry = entry_of[k];
             const int32_t lane = miss_lane[k];
-            if (entry == -1) {
-                // Not an entry of a miss list written by the lookup: record an
-                // empty promotion so the move that follows skips it.
-                promote_src[i * a.ps_o] = -1;
-                promote_dst[i * a.pd_o] = -1;
+            const int32_t victim = victim_of[k];
+            const int32_t token = token_of[k];
+            const int32_t global = static_cast<int32_t>(static_cast<uint32_t>(base) + static_cast<uint32_t>(victim));
+            if (token >= 0) {
+                *element<kDense>(slots, a.sl_o, static_cast<uint32_t>(lane)) = global;
+            }
+            if (first_of[k] != i) {
+                // Not an entry of a miss list written by the lookup, or a repeat of an earlier miss (which shares that
+                // miss's slot and promotion): record an empty promotion so the move that follows skips it.
+                *element<kDense>(promote_src, a.ps_o, i) = -1;
+                *element<kDense>(promote_dst, a.pd_o, i) = -1;
                 continue;
             }
-            const bool first = entry <= -2;
-            const int64_t victim = victim_of[k];
-            const int32_t global = static_cast<int32_t>(base + victim);
-            const int64_t token = info[i];
             const int32_t old = old_of[k];
-            const int32_t host_row = host_row_of[k];
-            slots[static_cast<int64_t>(lane) * a.sl_o] = global;
-            if (!first) {
-                // A repeat of an earlier miss: it shares that miss's slot and promotion.
-                promote_src[i * a.ps_o] = -1;
-                promote_dst[i * a.pd_o] = -1;
-                continue;
-            }
             if (old >= 0 && old < a.table_cols) {
-                set_entry(a, table_row + old * a.tb_t, 0);
-                if (bits != nullptr && a.bits_shift == 0) {
+                set_entry<kDense>(a, table_row, old, 0);
+                if (gathered > 0 && a.bits_shift == 0) {
+                    atomicAnd(reinterpret_cast<unsigned int*>(&summary[old >> 5]), ~(1u << (old & 31)));
+                } else if (gathered > 0) {
+                    atomicSub(&summary[old >> a.bits_shift], 1);
+                } else if (bits != nullptr && a.bits_shift == 0) {
                     atomicAnd(reinterpret_cast<unsigned int*>(bits + (old >> 5) * a.bt_w), ~(1u << (old & 31)));
                 } else if (line_counts != nullptr) {
                     // The group's last resident position leaves: clear its bit.
@@ -783,36 +805,79 @@ __global__ __launch_bounds__(kThreads) void swap_in_kernel(const SwapArgs a) {
                 // Without counts a coarse bit stays set (other positions of
                 // its group may still be resident): a superset.
             }
-            set_entry(a, table_row + token * a.tb_t, a.table16 ? static_cast<int32_t>(victim + 1) : global);
-            if (bits != nullptr && line_counts == nullptr) {
+            set_entry<kDense>(a, table_row, token, a.table16 ? victim + 1 : global);
+            if (gathered > 0 && a.bits_shift == 0) {
+                atomicOr(reinterpret_cast<unsigned int*>(&summary[token >> 5]), 1u << (token & 31));
+            } else if (gathered > 0) {
+                atomicAdd(&summary[token >> a.bits_shift], 1);
+            } else if (bits != nullptr && line_counts == nullptr) {
                 const int64_t q = token >> a.bits_shift;
                 atomicOr(reinterpret_cast<unsigned int*>(bits + (q >> 5) * a.bt_w), 1u << (q & 31));
             }
-            slot_token[victim * a.st_c] = static_cast<int32_t>(token);
-            stamp[victim] = static_cast<int32_t>(stamp_base + kMaxWidth + lane);
-            promote_src[i * a.ps_o] = host_row;
-            promote_dst[i * a.pd_o] = global;
+            *element<kDense>(slot_token, a.st_c, static_cast<uint32_t>(victim)) = token;
+            touch[victim] = stamp_base + kMaxWidth + lane;
+            *element<kDense>(promote_src, a.ps_o, i) = host_row_of[k];
+            *element<kDense>(promote_dst, a.pd_o, i) = global;
         }
-        if (line_counts != nullptr) {   // uniform
+        if (gathered > 0 || line_counts == nullptr) {   // uniform
+            lds_barrier();     // the victims' stamps and the summary's changes are read by other threads below
+        } else {
             __syncthreads();   // the evictions' count decrements (global atomics) precede the increments
             // Insertions: after every eviction's clear above, so a group that
             // both loses and gains positions ends with its bit set.
-            for (int32_t i = threadIdx.x; i < m; i += kThreads) {
-                if (owner[i] <= -2) {   // a first miss: info[i] is its valid token
-                    const int64_t q = static_cast<int64_t>(info[i]) >> a.bits_shift;
+#pragma unroll
+            for (int k = 0; k < kLaneRegs; ++k) {
+                if (token_of[k] >= 0 && first_of[k] == static_cast<int32_t>(threadIdx.x) + k * kThreads) {
+                    const int64_t q = static_cast<int64_t>(token_of[k]) >> a.bits_shift;
                     if (atomicAdd(line_counts + q * a.lc_q, 1) == 0) {
                         atomicOr(reinterpret_cast<unsigned int*>(bits + (q >> 5) * a.bt_w), 1u << (q & 31));
                     }
                 }
             }
-        } else {
-            lds_barrier();     // the victims' stamps land in LDS before the write-back
         }
-    } else {
-        __syncthreads();   // the touches above land before the stamps are written back
+        // The summary words, or each group's count and the bits of the groups that empty or fill (a wave's 64 groups are
+        // two words).
+        for (uint32_t g = 0; g * kThreads < gathered; ++g) {   // uniform over the workgroup
+            const uint32_t q = threadIdx.x + g * kThreads;
+            const int32_t mine = q < gathered ? summary[q] : 0;
+            if (line_counts == nullptr) {   // uniform
+                if (q < gathered) {
+                    *element<kDense>(bits, a.bt_w, q) = mine;
+                }
+                continue;
+            }
+            int32_t held = held_state[0];
+#pragma unroll
+            for (uint32_t r = 1; r < kReadAhead; ++r) {
+                held = g == r ? held_state[r] : held;
+            }
+            if (g >= kReadAhead) {   // uniform
+                held = line_counts[(q < gathered ? q : gathered - 1) * a.lc_q];
+            }
+            if (mine != 0) {
+                line_counts[q * a.lc_q] = held + mine;
+            }
+            const uint64_t clears = __ballot(mine != 0 && held > 0 && held + mine <= 0);
+            const uint64_t sets = __ballot(mine != 0 && held <= 0 && held + mine > 0);
+            if ((threadIdx.x & 31) == 0) {
+                const uint32_t clear = static_cast<uint32_t>(clears >> (threadIdx.x & 32));
+                const uint32_t set = static_cast<uint32_t>(sets >> (threadIdx.x & 32));
+                auto* word = reinterpret_cast<unsigned int*>(bits + (q >> 5) * a.bt_w);
+                if (clear != 0) {
+                    atomicAnd(word, ~clear);
+                }
+                if (set != 0) {
+                    atomicOr(word, set);
+                }
+            }
+        }
     }
-    for (int64_t s = threadIdx.x; s < C; s += kThreads) {
-        stamps[s * a.sp_c] = stamp[s];
+#pragma unroll
+    for (int k = 0; k < kSlotRegs; ++k) {
+        const uint32_t s = threadIdx.x + k * kThreads;
+        if (s < C) {
+            *element<kDense>(stamps, a.sp_c, s) = (chosen >> k) & 1u ? touch[s] : static_cast<int32_t>(key[k] ^ 0x80000000u);
+        }
     }
 }
 
@@ -821,6 +886,18 @@ __global__ void advance_step_kernel(int64_t* counter) {
     if (threadIdx.x == 0) {
         counter[0] += 1;
     }
+}
+
+template <int kThreads, int kSlotRegs, int kLaneRegs>
+void launch_swap(const SwapArgs& a, bool dense, dim3 grid, size_t lds, hipStream_t stream) {
+    auto* kernel = dense ? swap_in_kernel<kThreads, kSlotRegs, kLaneRegs, true>
+                         : swap_in_kernel<kThreads, kSlotRegs, kLaneRegs, false>;
+    if (lds > 48 * 1024) {
+        check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)),
+                  "raise the swap-in LDS limit");
+    }
+    kernel<<<grid, dim3(kThreads), lds, stream>>>(a);
 }
 
 void need_i32(const ekv_tensor& t, const char* name) {
@@ -1028,28 +1105,62 @@ int swap_in(const ekv_tensor* topk_p, int64_t block_size, const ekv_tensor* rows
         a.hash_size <<= 1;
         ++a.hash_log2;
     }
-    a.touched_words = static_cast<uint32_t>((C + 31) / 32);
     // The hash region holds 16 * hash_size bits: a bitmap of the tokens when they fit.
     a.token_bitmap = T <= int64_t{16} * a.hash_size ? 1u : 0u;
     a.bitmap_words = static_cast<uint32_t>(a.token_bitmap ? (T + 31) / 32 : 0);
-    // stamps, miss tokens, touched bits, the 16-bit hash buckets (then the
-    // victim list, 2 bytes per victim: at most W <= hash_size / 2), the owners
+    if (a.line_counts != nullptr || (a.bits != nullptr && bits_shift == 0)) {
+        const int64_t cover = bits_shift == 0 ? 32 : int64_t{1} << bits_shift;   // positions per word or group
+        const int64_t entries = (T + cover - 1) / cover;
+        a.gathered = entries <= kMaxGathered ? static_cast<uint32_t>(entries) : 0u;
+    }
+    // touches; the miss tokens, then the ranks (2 bytes each) and the summary;
+    // the 16-bit hash buckets or the token bitmap, then the victim list
+    // (2 bytes per victim: at most W <= hash_size / 2)
     static_assert(kMaxWidth <= 0x7fff && kMaxCapacity <= 0x7fff, "miss indices and slots fit 16 bits");
-    const size_t lds = static_cast<size_t>(C) * 4 + static_cast<size_t>(W) * 4 +
-                       static_cast<size_t>(a.touched_words) * 4 + static_cast<size_t>(a.hash_size) * 2 +
-                       static_cast<size_t>(W) * 2;
+    a.info_words = static_cast<uint32_t>(std::max<int64_t>(W, (W + 1) / 2 + a.gathered));
+    const size_t lds = (static_cast<size_t>(C) + a.info_words + std::max(a.hash_size / 2, a.bitmap_words)) * 4;
     const dim3 grid(static_cast<uint32_t>(count), static_cast<uint32_t>(L));
     const auto s = static_cast<hipStream_t>(stream);
-    // Registers per thread: 16 stamps up to C = 4096 (else 32), 8 lanes up to W = 2048 (else 16).
-    const bool wide_slots = C > 16 * kThreads, wide_lanes = W > 8 * kThreads;
-    auto* kernel = wide_slots ? (wide_lanes ? swap_in_kernel<32, 16> : swap_in_kernel<32, 8>)
-                              : (wide_lanes ? swap_in_kernel<16, 16> : swap_in_kernel<16, 8>);
-    if (lds > 64 * 1024) {
-        check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)),
-                  "raise the swap-in LDS limit");
+    // The workgroup size: the smallest whose threads hold four slots and two
+    // lanes each while every row has a CU to itself, so that the most waves
+    // share a row's phases; with more rows than CUs the smallest whose threads
+    // hold eight and four, since what each wave repeats (scans, ranges) then
+    // costs the rows beside it. Measured (us, with the launch; capacity is twice the lanes):
+    //   rows x lanes        eight and four   four and two
+    //   48 x 1024                20.0             15.7
+    //   48 x 2048                23.0             21.0
+    //   256 x 2048               24.7             23.2
+    //   512 x 2048               30.7             38.9
+    //   2560 x 512               39.7             45.8
+    //   2560 x 1024              69.5             74.3
+    //   2560 x 2048             133.5            179.8
+    // (2560 x 256: 34.0 against 28.0, so rows of up to 512 slots stay with
+    // four. Taken before the scans became DPP steps, which took up to 18 us off both.)
+    constexpr int64_t kCus = 256;
+    const bool dense = a.topk_sk == 1 && a.sl_o == 1 && a.mi_o == 1 && a.st_c == 1 && a.sp_c == 1 && a.ps_o == 1 &&
+                       a.pd_o == 1 && a.tb_t == 1 && a.host_st == 1 && (a.bits == nullptr || a.bt_w == 1) &&
+                       (a.line_counts == nullptr || a.lc_q == 1) && T < (int64_t{1} << 29);
+    const int64_t four = std::max((C + 3) / 4, (W + 1) / 2), eight = std::max((C + 7) / 8, (W + 3) / 4);
+    const bool crowded = count * L > kCus && four > 128;
+    if (four <= 64) {
+        launch_swap<64, 4, 2>(a, dense, grid, lds, s);
+    } else if (four <= 128) {
+        launch_swap<128, 4, 2>(a, dense, grid, lds, s);
+    } else if (crowded && eight <= 128) {
+        launch_swap<128, 8, 4>(a, dense, grid, lds, s);
+    } else if (four <= 256) {
+        launch_swap<256, 4, 2>(a, dense, grid, lds, s);
+    } else if (crowded && eight <= 256) {
+        launch_swap<256, 8, 4>(a, dense, grid, lds, s);
+    } else if (four <= 512) {
+        launch_swap<512, 4, 2>(a, dense, grid, lds, s);
+    } else if (crowded && eight <= 512) {
+        launch_swap<512, 8, 4>(a, dense, grid, lds, s);
+    } else if (four <= 1024) {
+        launch_swap<1024, 4, 2>(a, dense, grid, lds, s);
+    } else {
+        launch_swap<1024, 8, 4>(a, dense, grid, lds, s);
     }
-    kernel<<<grid, dim3(kThreads), lds, s>>>(a);
     check_hip(hipGetLastError(), "launch swap-in");
     if (counter != nullptr) {
         advance_step_kernel<<<dim3(1), dim3(64), 0, s>>>(counter);

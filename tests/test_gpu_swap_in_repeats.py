@@ -256,3 +256,46 @@ def test_rows_wider_than_2048_lanes_evict_in_lru_order(gpu, capacity, K, bs):
         state = _step(gpu, buffers, topk, bs, np.array([T, T - 5]), state, step, host_table)
         evicted += int(((before >= 0) & (state["slot_token"] != before)).sum())
     assert evicted > 0
+
+
+@pytest.mark.parametrize("L,R,C,W,T,shift,strided", [
+    (1, 3, 256, 128, 3000, 0, False), (1, 3, 257, 129, 3000, 6, False), (2, 2, 300, 300, 2500, 0, False),   # 64 to 256
+    (1, 3, 513, 100, 2000, 3, False), (1, 2, 1025, 513, 9000, 6, False), (1, 2, 2049, 600, 9000, 0, False),  # to 1024
+    (1, 1, 4097, 700, 9000, 6, False), (1, 1, 4096, 2049, 9000, 0, False),                 # eight slots, four lanes
+    (3, 90, 512, 60, 1500, 6, False), (3, 90, 513, 60, 1500, 0, False),                    # more rows than CUs
+    (3, 90, 1025, 60, 2500, 6, False), (3, 90, 2049, 60, 4000, 0, False),
+    (1, 2, 600, 300, 66000, 0, False), (1, 2, 600, 300, 20000, 3, False),                  # summaries past the LDS share
+    (1, 2, 600, 300, 2100, 0, True), (2, 2, 200, 60, 2100, 6, True), (3, 90, 1030, 60, 2100, 6, True)])
+def test_workgroup_sizes_and_layouts_match_oracle(gpu, L, R, C, W, T, shift, strided):
+    """Every workgroup size on both sides of its limits, more rows than CUs, summaries too long for LDS, and strided
+    state (64-bit addressing): nearly full buffers, recent-heavy picks, installed stamps (negative) beside new ones,
+    so the select starts at each digit; 4 steps against the oracle, summary and counts exact after each."""
+    from adaptive_sparse.resident_lookup import build_residency_bits
+    from adaptive_sparse.swap_in import residency_counts
+
+    rng = np.random.default_rng(C * 3 + W)
+    table_dtype = torch.int16 if (C + shift) % 2 else torch.int32
+    buffers = HotBuffers(L, R, T, C, gpu, table_dtype=table_dtype, bits_shift=shift)
+    if strided:
+        for name in ("table", "bits", "slot_token", "stamps", "resident_counts"):
+            held = getattr(buffers, name)
+            if held is not None:
+                wide = torch.zeros((*held.shape, 3), dtype=held.dtype, device=gpu)
+                wide[..., 1] = held
+                setattr(buffers, name, wide[..., 1])
+    filled = C - 3
+    tokens = np.stack([[rng.permutation(T)[:filled] for _ in range(R)] for _ in range(L)])
+    local = np.stack([[rng.permutation(C)[:filled] for _ in range(R)] for _ in range(L)])
+    buffers.install(torch.tensor(tokens), torch.tensor(local))
+    buffers.step = 6                                             # stamps 49152 .. 81919: three digits differ
+    host_table = torch.tensor(rng.permutation(R * T), dtype=torch.int32).reshape(R, T)
+    state = {"table": _global(buffers), "slot_token": buffers.slot_token.cpu().numpy(),
+             "stamps": buffers.stamps.cpu().numpy()}
+    for step in range(6, 10):
+        topk = np.stack([[rng.permutation(T)[:W] for _ in range(R)] for _ in range(L)])
+        if step == 8:
+            topk[..., 1::37] = topk[..., :1]                     # repeated tokens
+        state = _step(gpu, buffers, topk, 1, np.full(R, T), state, step, host_table)
+        assert torch.equal(buffers.bits.contiguous(), build_residency_bits(buffers.table, shift=shift)), step
+        if shift:
+            assert torch.equal(buffers.resident_counts.contiguous(), residency_counts(buffers.table, shift)), step
