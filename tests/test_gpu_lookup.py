@@ -333,3 +333,49 @@ def test_launch_goes_to_the_current_stream(gpu):
     # torch's default stream is the null stream: handle 0, which ctypes reads back as None.
     assert (_native.stream_handle(gpu).value or 0) == torch.cuda.current_stream(gpu).cuda_stream
     assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("bs,k,cols", [(8, 1, 8), (8, 5, 61), (16, 7, 4001), (64, 32, 4000), (128, 17, 3003), (24, 100, 2500)])
+@pytest.mark.parametrize("dtype", [torch.int16, torch.int32])
+def test_whole_block_lookups_match_oracle_and_general_path(gpu, bs, k, cols, dtype):
+    # Blocks of a multiple of 8 tokens: runs at the row's ragged end, rows of several chunks, stray selections and
+    # requests, short and negative lengths; the same call with a misaligned output takes the general kernel.
+    from adaptive_sparse.resident_lookup import build_residency_bits
+    from oracle import oracle as ref
+
+    rng = np.random.default_rng(bs * 100 + k)
+    layers, batch, table_rows = 2, 5, 4
+    local = rng.integers(1, 1 << 15, (layers, table_rows, cols)) * (rng.random((layers, table_rows, cols)) < 0.6)
+    local = np.where(rng.random(local.shape) < 0.02, -local, local)              # negative: not resident when local
+    base = rng.integers(1, 1 << 20, table_rows)
+    table = np.where(local > 0, base.reshape(1, -1, 1) + local - 1, 0) if dtype == torch.int16 else local
+    topk = rng.integers(-1, cols // bs + 2, (layers, batch, k))
+    topk[..., 0] = (cols - 1) // bs
+    lengths = np.array([cols, cols - 3, cols // 2, -4, cols + 9])
+    rows = np.array([2, 0, 3, 1, table_rows])                                     # the last names no table row
+    width = k * bs
+    store = torch.full((layers, table_rows, -(-cols // 128) * 128), 7, dtype=dtype, device=gpu)
+    table_d = store[..., :cols]
+    table_d.copy_(torch.tensor(local))
+    for selected in (np.arange(batch), np.array([3, 0, -1, 4, batch, 2])):
+        want, want_misses, want_counts = ref.resolve_resident(topk, table, None, rows, lengths, selected, bs,
+                                                              np.full((layers, batch, width), -77, np.int32),
+                                                              with_misses=True)
+        for topk_dtype, bits, shifted in ((torch.int32, False, 0), (torch.int64, True, 0), (torch.int32, True, 1)):
+            wide = torch.full((layers, batch, width + 4 * shifted), -77, dtype=torch.int32, device=gpu)
+            out = wide[..., shifted:width + shifted]
+            misses = torch.full((layers, batch, width), -5, dtype=torch.int32, device=gpu)
+            counts = torch.full((layers, batch), -5, dtype=torch.int32, device=gpu)
+            args = (torch.tensor(topk, dtype=topk_dtype, device=gpu), table_d, None, torch.tensor(rows, device=gpu),
+                    torch.tensor(lengths, dtype=torch.int32, device=gpu), torch.tensor(selected, device=gpu), out, bs)
+            extra = dict(resident_bits=build_residency_bits(table_d) if bits else None,
+                         slot_base=torch.tensor(base, device=gpu) if dtype == torch.int16 else None)
+            resolve_resident(*args, misses=misses, miss_count=counts, **extra)
+            assert np.array_equal(out.cpu().numpy(), want), (selected, topk_dtype, bits, shifted)
+            got_counts, got = counts.cpu().numpy(), misses.cpu().numpy()
+            for (layer, r), lanes in want_misses.items():
+                assert got_counts[layer, r] == want_counts[layer, r] == len(lanes)
+                assert np.array_equal(got[layer, r, :len(lanes)], lanes)
+            out.fill_(-77)
+            resolve_resident(*args, **extra)                                       # without compaction
+            assert np.array_equal(out.cpu().numpy(), want)
