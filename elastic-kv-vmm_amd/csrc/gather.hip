@@ -24,6 +24,7 @@
 #include "ekv_common.h"
 #include "ekv_device.h"
 #include "ekv_fastdiv.h"
+#include "ekv_step.h"
 #include "ekv_tensor_util.h"
 #include "ekv_vec.h"
 
@@ -96,6 +97,8 @@ struct EngineArgs {
     int64_t mdr_l, mdr_b, mdr_i;
     const int32_t* move_counts;
     int64_t mc_l, mc_b;
+    IndexRef move_selected;  // data null: every batch row; else entry j of B stands for batch row move_selected[j]
+    int64_t move_batch;      // batch rows
 
     // Rows modes: unit u = b * S + s.
     const char* raw;
@@ -135,14 +138,24 @@ __device__ __forceinline__ void split_unit(const EngineArgs& a, int64_t u, int64
     }
 }
 
+// Batch row of list row j of a move, or -1 when a selection names none there.
+__device__ __forceinline__ int64_t move_row(const EngineArgs& a, int64_t j) {
+    if (a.move_selected.data == nullptr) {   // uniform
+        return j;
+    }
+    const int64_t row = a.move_selected[j];
+    return row >= 0 && row < a.move_batch ? row : -1;
+}
+
 template <int M>
 __device__ __forceinline__ void locate(const EngineArgs& a, int64_t u, int64_t& src, int64_t& dst) {
     if constexpr (M == KvMove) {
-        int64_t l, b, kv, k;
-        split_unit(a, u, l, b, kv, k);
+        int64_t l, j, kv, k;
+        split_unit(a, u, l, j, kv, k);
         src = -1;
         dst = -1;
-        if (k < a.move_counts[l * a.mc_l + b * a.mc_b]) {
+        const int64_t b = move_row(a, j);
+        if (b >= 0 && k < a.move_counts[l * a.mc_l + b * a.mc_b]) {
             const int64_t from = a.move_src_rows[l * a.msr_l + b * a.msr_b + k * a.msr_i];
             const int64_t to = a.move_dst_rows[l * a.mdr_l + b * a.mdr_b + k * a.mdr_i];
             if (from >= 0 && from < a.ms_rows && to >= a.zero_below && to < a.pool_rows) {
@@ -414,6 +427,7 @@ __global__ __launch_bounds__(kThreads) void move_host_rows(const EngineArgs a, u
     using V = typename Vec<VW>::type;
     constexpr int kWaves = kThreads / 64;
     __shared__ uint32_t first_move[kHostRows];   // moves of the rows below each row of this batch of rows
+    __shared__ int32_t batch_row[kHostRows];     // batch row of each
     __shared__ uint32_t wave_moves[kWaves];
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
@@ -427,8 +441,10 @@ __global__ __launch_bounds__(kThreads) void move_host_rows(const EngineArgs a, u
             const bool live = r < batch_rows && base + r < rows;
             const uint32_t at = live ? base + r : base;
             const uint32_t l = a.div_b.div(at);
-            const int32_t c = a.move_counts[l * a.mc_l + (at - l * a.div_b.divisor) * a.mc_b];
-            count[i] = live && c > 0 ? static_cast<uint32_t>(min(int64_t{c}, a.K)) : 0u;
+            const int64_t b = move_row(a, at - l * a.div_b.divisor);
+            const int32_t c = a.move_counts[l * a.mc_l + (b >= 0 ? b : 0) * a.mc_b];
+            count[i] = live && b >= 0 && c > 0 ? static_cast<uint32_t>(min(int64_t{c}, a.K)) : 0u;
+            batch_row[r] = static_cast<int32_t>(b);   // read for rows with moves only
         }
         uint32_t mine = 0;
 #pragma unroll
@@ -480,7 +496,7 @@ __global__ __launch_bounds__(kThreads) void move_host_rows(const EngineArgs a, u
             }
             const uint32_t i = move - first_move[r];
             const uint32_t l = a.div_b.div(base + r);
-            const uint32_t b = base + r - l * a.div_b.divisor;
+            const int64_t b = batch_row[r];
             const int64_t from = a.move_src_rows[l * a.msr_l + b * a.msr_b + i * a.msr_i];
             const int64_t to = a.move_dst_rows[l * a.mdr_l + b * a.mdr_b + i * a.mdr_i];
             if (from >= 0 && from < a.ms_rows && to >= a.zero_below && to < a.pool_rows) {
@@ -718,7 +734,8 @@ int gather_rows(const ekv_tensor* raw_p, const ekv_tensor* positions_p, const ek
 }
 
 int move_kv(const ekv_planes* src, const ekv_tensor* src_rows_p, const ekv_planes* dst,
-            const ekv_tensor* dst_rows_p, const ekv_tensor* counts_p, int64_t zero_below, void* stream) {
+            const ekv_tensor* dst_rows_p, const ekv_tensor* counts_p, int64_t zero_below, void* stream,
+            const ekv_tensor* selected = nullptr) {
     need_planes(src);
     need_planes(dst);
     const ekv_tensor& src_rows = need(src_rows_p, "src_rows");
@@ -747,7 +764,8 @@ int move_kv(const ekv_planes* src, const ekv_tensor* src_rows_p, const ekv_plane
     if (zero_below < 0) {
         throw std::invalid_argument("zero_below must be >= 0");
     }
-    const int64_t units = L * B * dst->kv * K;
+    const int64_t list_rows = selected != nullptr ? selected->shape[0] : B;
+    const int64_t units = L * list_rows * dst->kv * K;
     if (units == 0 || dst->row_bytes == 0) {
         return 0;
     }
@@ -778,12 +796,16 @@ int move_kv(const ekv_planes* src, const ekv_tensor* src_rows_p, const ekv_plane
     a.mc_l = counts.stride[0], a.mc_b = counts.stride[1];
     a.K = K;
     a.KV = dst->kv;
-    a.B = B;
+    a.B = list_rows;
+    a.move_batch = B;
+    if (selected != nullptr) {
+        a.move_selected = index_ref(*selected, 0);
+    }
     a.small_units = units < (int64_t{1} << 31);
     if (a.small_units) {
         a.div_k = FastDiv(static_cast<uint32_t>(K));
         a.div_kv = FastDiv(static_cast<uint32_t>(dst->kv));
-        a.div_b = FastDiv(static_cast<uint32_t>(B));
+        a.div_b = FastDiv(static_cast<uint32_t>(list_rows));
     }
     a.src_base = a.msrc;
     a.dst_base = static_cast<char*>(dst->base);
@@ -795,7 +817,7 @@ int move_kv(const ekv_planes* src, const ekv_tensor* src_rows_p, const ekv_plane
     }
     const auto s = static_cast<hipStream_t>(stream);
     const bool linked = units * a.row_bytes > kHostMoveBytes && in_host_memory(src->base);
-    if (!linked || !host_move(a, L * B, vw, s)) {
+    if (!linked || !host_move(a, L * list_rows, vw, s)) {
         launch_vw<KvMove>(a, vw, s);
     }
     check_hip(hipGetLastError(), "launch KV move");
@@ -823,6 +845,12 @@ int host_alloc(uint64_t bytes, void** host, void** device) {
 }
 
 }  // namespace
+
+void move_selected(const ekv_planes* src, const ekv_tensor* src_rows, const ekv_planes* dst, const ekv_tensor* dst_rows,
+                   const ekv_tensor* counts, const ekv_tensor* selected, int64_t zero_below, void* stream) {
+    move_kv(src, src_rows, dst, dst_rows, counts, zero_below, stream, selected);
+}
+
 }  // namespace ekv
 
 extern "C" int ekv_move_kv(const ekv_planes* src, const ekv_tensor* src_rows, const ekv_planes* dst,

@@ -56,6 +56,7 @@
 #include "../../include/ekv_kernels.h"
 #include "ekv_common.h"
 #include "ekv_fastdiv.h"
+#include "ekv_step.h"
 #include "ekv_tensor_util.h"
 
 #include <algorithm>
@@ -91,7 +92,8 @@ struct SwapArgs {
     int64_t sl_l, sl_b, sl_o;
     const int32_t* misses;          // [L, B, W] miss lanes
     int64_t mi_l, mi_b, mi_o;
-    const int32_t* counts;          // [L, B]
+    int32_t* counts;                // [L, B]
+    IndexRef lengths;               // [B], when the lookup runs in the same launch
     int64_t ct_l, ct_b;
     void* table;                    // [L, R, T] token -> global slot (int32) or local slot + 1 (int16); 0 = not resident
     int32_t table16;
@@ -364,7 +366,16 @@ __device__ __forceinline__ void hash_miss_tokens(uint32_t* hash, const int32_t* 
 // ids of the miss entries; the victims' old tokens and host rows. (A loop
 // with a run-time trip count waits for each load before issuing the next: a
 // workgroup then spends most of its life on a chain of HBM round trips.)
-template <int kThreads, int kSlotRegs, int kLaneRegs, bool kDense>
+//
+// kLookup: the lookup of the rows runs here as well (the one-call decode step).
+// A thread's lanes then are their own miss entries: their Top-K ids are read
+// in the prologue, their table entries in place of the lookup's slots (no summary: what it
+// could spare is the entry reads of the misses), the misses are ranked over the
+// barrier of the request check, and slots and miss count are written here. It saves the
+// lookup's launch and chain of reads, and the slots and miss list through memory.
+// In the decode step of 8 rows of 64 lanes: 12.2 us, where the two kernels took
+// 6.3 and 13.0.
+template <int kThreads, int kSlotRegs, int kLaneRegs, bool kDense, bool kLookup>
 __global__ __launch_bounds__(kThreads) void swap_in_kernel(const SwapArgs a) {
     constexpr int kWaves = kThreads / 64;
     constexpr uint32_t kReadAhead = 4;     // summary words or group counts per thread that are read ahead
@@ -373,6 +384,7 @@ __global__ __launch_bounds__(kThreads) void swap_in_kernel(const SwapArgs a) {
     __shared__ uint32_t key_range[3];      // empties, smallest and largest other key
     __shared__ uint32_t first_cells[kLaneRegs * kWaves], victim_cells[kSlotRegs * kWaves];
     __shared__ uint32_t any_cells[2][kWaves];
+    __shared__ uint32_t miss_cells[kLookup ? kLaneRegs * kWaves : 1];
     int32_t* touch = reinterpret_cast<int32_t*>(shared);
     int32_t* info = touch + a.capacity;
     int16_t* owner = reinterpret_cast<int16_t*>(info);   // the tokens are in registers again by then
@@ -392,7 +404,27 @@ __global__ __launch_bounds__(kThreads) void swap_in_kernel(const SwapArgs a) {
     const int64_t guess = blockIdx.x < a.batch ? blockIdx.x : 0;
     const PendingIndex entry_read = issue_index(a.selected, blockIdx.x, zero);
     const PendingIndex req_read = issue_index(a.rows, guess, zero);
-    const int32_t counted_read = a.counts[l * a.ct_l + guess * a.ct_b + zero];
+    int32_t counted_read = 0;
+    PendingIndex length_read{0, 0};
+    int32_t block_low[kLaneRegs], block_high[kLaneRegs];   // Top-K ids of this thread's lanes, or of its miss entries
+    const auto topk_row_of = [&](int64_t row) {
+        return a.topk64 ? static_cast<const void*>(static_cast<const int64_t*>(a.topk) + l * a.topk_sl + row * a.topk_sb)
+                        : static_cast<const void*>(static_cast<const int32_t*>(a.topk) + l * a.topk_sl + row * a.topk_sb);
+    };
+    const auto read_id = [&](const void* topk_row, uint32_t lane, int k) {
+        const uint32_t blk = a.block_size == 1 ? lane : a.block_div.div(lane);
+        block_low[k] = index_word<kDense>(topk_row, a.topk64, a.topk_sk, blk, false);
+        block_high[k] = index_word<kDense>(topk_row, a.topk64, a.topk_sk, blk, a.topk64 != 0);
+    };
+    if constexpr (kLookup) {
+        length_read = issue_index(a.lengths, guess, zero);
+#pragma unroll
+        for (int k = 0; k < kLaneRegs; ++k) {
+            read_id(topk_row_of(guess), min(threadIdx.x + k * kThreads, a.width - 1), k);
+        }
+    } else {
+        counted_read = a.counts[l * a.ct_l + guess * a.ct_b + zero];
+    }
     // The device step of a graph replay; without one, a word of the counts
     // stands in and is not used.
     const bool device_step = a.step_counter != nullptr;   // uniform
@@ -405,6 +437,7 @@ __global__ __launch_bounds__(kThreads) void swap_in_kernel(const SwapArgs a) {
     const int64_t b = index_value(a.selected, entry_read);
     int64_t req = index_value(a.rows, req_read);
     int32_t counted = __builtin_amdgcn_readfirstlane(counted_read);
+    int64_t length = kLookup ? index_value(a.lengths, length_read) : 0;
     const int64_t step =
         device_step ? static_cast<int64_t>((static_cast<uint64_t>(static_cast<uint32_t>(
                                                 __builtin_amdgcn_readfirstlane(step_hi))) << 32) |
@@ -413,9 +446,27 @@ __global__ __launch_bounds__(kThreads) void swap_in_kernel(const SwapArgs a) {
     const bool live = b >= 0 && b < a.batch;   // uniform
     if (live && b != guess) {   // uniform: the selection is not the identity here
         req = a.rows.fetch(b);
-        counted = a.counts[l * a.ct_l + b * a.ct_b];
+        if constexpr (kLookup) {
+            length = a.lengths.fetch(b);
+#pragma unroll
+            for (int k = 0; k < kLaneRegs; ++k) {
+                read_id(topk_row_of(b), min(threadIdx.x + k * kThreads, a.width - 1), k);
+            }
+        } else {
+            counted = a.counts[l * a.ct_l + b * a.ct_b];
+        }
     }
     if (!live || req < 0 || req >= a.table_rows) {
+        if constexpr (kLookup) {
+            if (live) {   // uniform: no lane of it is valid
+                for (uint32_t o = threadIdx.x; o < a.width; o += kThreads) {
+                    *element<kDense>(a.slots + l * a.sl_l + b * a.sl_b, a.sl_o, o) = -1;
+                }
+                if (threadIdx.x == 0) {
+                    a.counts[l * a.ct_l + b * a.ct_b] = 0;
+                }
+            }
+        }
         return;  // uniform: a stray selection, or a row outside the tables (nothing resident)
     }
     const int64_t C = a.capacity;
@@ -428,9 +479,6 @@ __global__ __launch_bounds__(kThreads) void swap_in_kernel(const SwapArgs a) {
     int32_t* slot_token = a.slot_token + l * a.st_l + req * a.st_r;
     int32_t* stamps = a.stamps + l * a.sp_l + req * a.sp_r;
     const int32_t* misses = a.misses + l * a.mi_l + b * a.mi_b;
-    const void* topk_row = a.topk64
-        ? static_cast<const void*>(static_cast<const int64_t*>(a.topk) + l * a.topk_sl + b * a.topk_sb)
-        : static_cast<const void*>(static_cast<const int32_t*>(a.topk) + l * a.topk_sl + b * a.topk_sb);
 
     // One workgroup owns each (layer, request) hot buffer: a second selected
     // row naming the same request would race on it, so both rows are refused.
@@ -448,13 +496,50 @@ __global__ __launch_bounds__(kThreads) void swap_in_kernel(const SwapArgs a) {
         const uint32_t s = min(threadIdx.x + k * kThreads, static_cast<uint32_t>(C) - 1);
         held_stamp[k] = *element<kDense>(stamps, a.sp_c, s);
     }
-    int32_t lane_slot[kLaneRegs];
-    int32_t miss_lane[kLaneRegs];
+    int32_t lane_slot[kLaneRegs];   // kLookup: the table entry until the base is known
+    int32_t miss_lane[kLaneRegs];   // lane of this thread's k-th entry (kLookup: its k-th lane)
+    bool valid_lane[kLaneRegs];     // kLookup
+    int64_t lane_token[kLaneRegs];
+    // The token of an entry: its block id times the block size, and the lane's place in the block.
+    const auto token_at = [&](int k, int32_t lane) {
+        const int32_t high = a.topk64 ? block_high[k] : block_low[k] >> 31;
+        int64_t token = static_cast<int64_t>(static_cast<uint64_t>(static_cast<uint32_t>(high)) << 32 |
+                                             static_cast<uint32_t>(block_low[k]));
+        if (a.block_size != 1) {   // uniform
+            token = token * a.block_size +
+                    (static_cast<uint32_t>(lane) - a.block_div.div(static_cast<uint32_t>(lane)) * a.block_size);
+        }
+        return token;
+    };
+    if constexpr (kLookup) {
+        const int64_t bound = length < a.table_cols ? length : a.table_cols;
+        uint32_t at[kLaneRegs];
 #pragma unroll
-    for (int k = 0; k < kLaneRegs; ++k) {
-        const uint32_t o = min(threadIdx.x + k * kThreads, a.width - 1);
-        lane_slot[k] = *element<kDense>(slots, a.sl_o, o);
-        miss_lane[k] = *element<kDense>(misses, a.mi_o, o);   // entries at or past the count are read but not used
+        for (int k = 0; k < kLaneRegs; ++k) {
+            miss_lane[k] = static_cast<int32_t>(threadIdx.x) + k * kThreads;
+            lane_token[k] = token_at(k, miss_lane[k]);
+            const int32_t high = a.topk64 ? block_high[k] : block_low[k];
+            valid_lane[k] = miss_lane[k] < W && high >= 0 && lane_token[k] < bound;   // a block id of at least 0
+            at[k] = valid_lane[k] ? static_cast<uint32_t>(lane_token[k]) : 0u;
+        }
+        if (a.table16) {   // uniform
+#pragma unroll
+            for (int k = 0; k < kLaneRegs; ++k) {
+                lane_slot[k] = *element<kDense>(static_cast<const int16_t*>(a.table) + table_row, a.tb_t, at[k]);
+            }
+        } else {
+#pragma unroll
+            for (int k = 0; k < kLaneRegs; ++k) {
+                lane_slot[k] = *element<kDense>(static_cast<const int32_t*>(a.table) + table_row, a.tb_t, at[k]);
+            }
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < kLaneRegs; ++k) {
+            const uint32_t o = min(threadIdx.x + k * kThreads, a.width - 1);
+            lane_slot[k] = *element<kDense>(slots, a.sl_o, o);
+            miss_lane[k] = *element<kDense>(misses, a.mi_o, o);   // entries at or past the count are read but not used
+        }
     }
     const bool first_in_range =
         first_j < selected_count && first_j != blockIdx.x && first_other >= 0 && first_other < a.batch;
@@ -465,15 +550,13 @@ __global__ __launch_bounds__(kThreads) void swap_in_kernel(const SwapArgs a) {
         shared_request |= j != blockIdx.x && other >= 0 && other < a.batch && a.rows[other] == req;
     }
     // Batch 2: the Top-K ids of the miss entries.
-    int32_t block_low[kLaneRegs], block_high[kLaneRegs];
+    if constexpr (!kLookup) {
 #pragma unroll
-    for (int k = 0; k < kLaneRegs; ++k) {
-        const uint32_t lane = static_cast<uint32_t>(min(max(miss_lane[k], 0), static_cast<int32_t>(W - 1)));
-        const uint32_t blk = a.block_size == 1 ? lane : a.block_div.div(lane);
-        block_low[k] = index_word<kDense>(topk_row, a.topk64, a.topk_sk, blk, false);
-        block_high[k] = index_word<kDense>(topk_row, a.topk64, a.topk_sk, blk, a.topk64 != 0);
+        for (int k = 0; k < kLaneRegs; ++k) {
+            read_id(topk_row_of(b), static_cast<uint32_t>(min(max(miss_lane[k], 0), static_cast<int32_t>(W - 1))), k);
+        }
     }
-    const int32_t m = counted < 0 ? 0 : (counted > W ? static_cast<int32_t>(W) : counted);
+    int32_t m = counted < 0 ? 0 : (counted > W ? static_cast<int32_t>(W) : counted);
     // LDS starts, published by the barrier of the request check: nothing touched, the region a token bitmap (all clear)
     // when the tokens fit it, else the empty hash.
 #pragma unroll
@@ -513,7 +596,44 @@ __global__ __launch_bounds__(kThreads) void swap_in_kernel(const SwapArgs a) {
             held_state[g] = *element<kDense>(state, state_stride, q < gathered ? q : gathered - 1);
         }
     }
+    const int64_t base = index_value(a.slot_base, base_read);
+    uint32_t list_at[kLaneRegs];   // place of this thread's k-th entry in the miss and promotion lists
+    bool listed[kLaneRegs];        // it is a miss entry
+    if constexpr (kLookup) {
+        // The looked-up slots, and the misses' ranks in lane order (over the request check's barrier).
+        uint32_t missed[kLaneRegs];
+#pragma unroll
+        for (int k = 0; k < kLaneRegs; ++k) {
+            const int32_t held = lane_slot[k];
+            const int32_t slot = a.table16 ? (held > 0 ? static_cast<int32_t>(base + held - 1) : 0) : held;
+            lane_slot[k] = valid_lane[k] ? slot : -1;
+            listed[k] = valid_lane[k] && slot == 0;
+            missed[k] = __popcll(__ballot(listed[k]));
+        }
+        pair_counts<kWaves, kLaneRegs>(missed, miss_cells);
+    }
     shared_request = workgroup_any<kWaves>(shared_request, any_cells[0]);
+    if constexpr (kLookup) {
+        uint32_t total = 0;
+        pair_bases<kWaves, kLaneRegs>(miss_cells, list_at, total);
+        m = static_cast<int32_t>(total);
+#pragma unroll
+        for (int k = 0; k < kLaneRegs; ++k) {
+            list_at[k] += lanes_below(__ballot(listed[k]));
+            if (miss_lane[k] < W && !listed[k]) {   // a miss's slot is written with its victim below
+                *element<kDense>(slots, a.sl_o, static_cast<uint32_t>(miss_lane[k])) = lane_slot[k];
+            }
+        }
+        if (threadIdx.x == 0) {
+            a.counts[l * a.ct_l + b * a.ct_b] = m;
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < kLaneRegs; ++k) {
+            list_at[k] = threadIdx.x + k * kThreads;
+            listed[k] = static_cast<int32_t>(list_at[k]) < m;
+        }
+    }
     const bool overflow = step < 0 || (step + 1) * kStepStamps >= (int64_t{1} << 31);
     if (shared_request || overflow) {
         // Change nothing, record empty promotions (the move that follows
@@ -525,10 +645,17 @@ __global__ __launch_bounds__(kThreads) void swap_in_kernel(const SwapArgs a) {
             promote_src[i * a.ps_o] = -1;
             promote_dst[i * a.pd_o] = -1;
         }
+        if constexpr (kLookup) {
+#pragma unroll
+            for (int k = 0; k < kLaneRegs; ++k) {
+                if (listed[k]) {
+                    *element<kDense>(slots, a.sl_o, static_cast<uint32_t>(miss_lane[k])) = 0;
+                }
+            }
+        }
         return;
     }
     const int32_t stamp_base = static_cast<int32_t>(step * kStepStamps);
-    const int64_t base = index_value(a.slot_base, base_read);
     // Touch hits: a token repeated in the row is one access of its first lane. Repeated miss tokens: with the token
     // bitmap, each valid entry sets its token's bit; a bit found set means some token repeats, and only then is the
     // exact hash built (each token's lowest miss index). Without repeats every valid entry is its token's first miss.
@@ -542,16 +669,9 @@ __global__ __launch_bounds__(kThreads) void swap_in_kernel(const SwapArgs a) {
         if (o < W && lane_slot[k] > 0 && offset >= 0 && offset < C) {
             atomicMin(&touch[static_cast<uint32_t>(offset)], o);
         }
-        // The entry's token: its block id times the block size, and the lane's place in the block.
         const int32_t lane = miss_lane[k];
-        const int32_t high = a.topk64 ? block_high[k] : block_low[k] >> 31;
-        int64_t token = static_cast<int64_t>(static_cast<uint64_t>(static_cast<uint32_t>(high)) << 32 |
-                                             static_cast<uint32_t>(block_low[k]));
-        if (a.block_size != 1) {   // uniform
-            token = token * a.block_size +
-                    (static_cast<uint32_t>(lane) - a.block_div.div(static_cast<uint32_t>(lane)) * a.block_size);
-        }
-        const bool valid = o < m && lane >= 0 && lane < W && token >= 0 && token < a.table_cols;
+        const int64_t token = kLookup ? lane_token[k] : token_at(k, lane);
+        const bool valid = listed[k] && lane >= 0 && lane < W && token >= 0 && token < a.table_cols;
         token_of[k] = valid ? static_cast<int32_t>(token) : -1;
         first_of[k] = valid ? o : -1;
         if (a.token_bitmap && token_of[k] >= 0) {
@@ -561,10 +681,11 @@ __global__ __launch_bounds__(kThreads) void swap_in_kernel(const SwapArgs a) {
     }
     const bool exact_hash = workgroup_any<kWaves>(repeated, any_cells[1]) || !a.token_bitmap;   // uniform
     if (exact_hash) {
+        const int32_t entries = kLookup ? static_cast<int32_t>(W) : m;   // entries a thread may hold (-1: no miss)
 #pragma unroll
         for (int k = 0; k < kLaneRegs; ++k) {
             const int32_t i = static_cast<int32_t>(threadIdx.x) + k * kThreads;
-            if (i < m) {
+            if (i < entries) {
                 info[i] = token_of[k];
             }
         }
@@ -574,7 +695,7 @@ __global__ __launch_bounds__(kThreads) void swap_in_kernel(const SwapArgs a) {
             }
         }
         lds_barrier();
-        hash_miss_tokens(hash, info, m, a.hash_log2);
+        hash_miss_tokens(hash, info, entries, a.hash_log2);
         lds_barrier();
         const uint32_t mask = a.hash_size - 1;
 #pragma unroll
@@ -769,7 +890,7 @@ __global__ __launch_bounds__(kThreads) void swap_in_kernel(const SwapArgs a) {
 #pragma unroll
         for (int k = 0; k < kLaneRegs; ++k) {
             const int32_t i = static_cast<int32_t>(threadIdx.x) + k * kThreads;
-            if (i >= m) {
+            if (!listed[k]) {
                 continue;
             }
             const int32_t lane = miss_lane[k];
@@ -782,8 +903,8 @@ __global__ __launch_bounds__(kThreads) void swap_in_kernel(const SwapArgs a) {
             if (first_of[k] != i) {
                 // Not an entry of a miss list written by the lookup, or a repeat of an earlier miss (which shares that
                 // miss's slot and promotion): record an empty promotion so the move that follows skips it.
-                *element<kDense>(promote_src, a.ps_o, i) = -1;
-                *element<kDense>(promote_dst, a.pd_o, i) = -1;
+                *element<kDense>(promote_src, a.ps_o, list_at[k]) = -1;
+                *element<kDense>(promote_dst, a.pd_o, list_at[k]) = -1;
                 continue;
             }
             const int32_t old = old_of[k];
@@ -816,8 +937,8 @@ __global__ __launch_bounds__(kThreads) void swap_in_kernel(const SwapArgs a) {
             }
             *element<kDense>(slot_token, a.st_c, static_cast<uint32_t>(victim)) = token;
             touch[victim] = stamp_base + kMaxWidth + lane;
-            *element<kDense>(promote_src, a.ps_o, i) = host_row_of[k];
-            *element<kDense>(promote_dst, a.pd_o, i) = global;
+            *element<kDense>(promote_src, a.ps_o, list_at[k]) = host_row_of[k];
+            *element<kDense>(promote_dst, a.pd_o, list_at[k]) = global;
         }
         if (gathered > 0 || line_counts == nullptr) {   // uniform
             lds_barrier();     // the victims' stamps and the summary's changes are read by other threads below
@@ -890,8 +1011,9 @@ __global__ void advance_step_kernel(int64_t* counter) {
 
 template <int kThreads, int kSlotRegs, int kLaneRegs>
 void launch_swap(const SwapArgs& a, bool dense, dim3 grid, size_t lds, hipStream_t stream) {
-    auto* kernel = dense ? swap_in_kernel<kThreads, kSlotRegs, kLaneRegs, true>
-                         : swap_in_kernel<kThreads, kSlotRegs, kLaneRegs, false>;
+    auto* kernel = a.lengths.data != nullptr ? swap_in_kernel<kThreads, kSlotRegs, kLaneRegs, true, true>
+                   : dense                   ? swap_in_kernel<kThreads, kSlotRegs, kLaneRegs, true, false>
+                                             : swap_in_kernel<kThreads, kSlotRegs, kLaneRegs, false, false>;
     if (lds > 48 * 1024) {
         check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                                       hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)),
@@ -899,6 +1021,9 @@ void launch_swap(const SwapArgs& a, bool dense, dim3 grid, size_t lds, hipStream
     }
     kernel<<<grid, dim3(kThreads), lds, stream>>>(a);
 }
+
+// swap_in's answer when it was asked to run the lookup too and the layouts need the lookup's own kernels.
+constexpr int kNeedsLookup = 1;
 
 void need_i32(const ekv_tensor& t, const char* name) {
     if (t.dtype != EKV_INT32) {
@@ -912,7 +1037,8 @@ int swap_in(const ekv_tensor* topk_p, int64_t block_size, const ekv_tensor* rows
             const ekv_tensor* slot_token_p,
             const ekv_tensor* stamps_p, const ekv_tensor* slot_base_p, const ekv_tensor* host_table_p,
             const ekv_tensor* promote_src_p, const ekv_tensor* promote_dst_p, int64_t step,
-            const ekv_tensor* step_counter_p, const ekv_tensor* status_p, void* stream) {
+            const ekv_tensor* step_counter_p, const ekv_tensor* status_p, void* stream,
+            const ekv_tensor* lengths_p = nullptr) {
     const ekv_tensor& topk = need(topk_p, "topk");
     const ekv_tensor& rows = need(rows_p, "rows");
     const ekv_tensor& selected = need(selected_p, "selected");
@@ -1065,7 +1191,7 @@ int swap_in(const ekv_tensor* topk_p, int64_t block_size, const ekv_tensor* rows
     a.sl_l = slots.stride[0], a.sl_b = slots.stride[1], a.sl_o = slots.stride[2];
     a.misses = static_cast<const int32_t*>(misses.data);
     a.mi_l = misses.stride[0], a.mi_b = misses.stride[1], a.mi_o = misses.stride[2];
-    a.counts = static_cast<const int32_t*>(counts.data);
+    a.counts = static_cast<int32_t*>(counts.data);
     a.ct_l = counts.stride[0], a.ct_b = counts.stride[1];
     a.table = table.data;
     a.table16 = table.dtype == EKV_INT16;
@@ -1140,6 +1266,12 @@ int swap_in(const ekv_tensor* topk_p, int64_t block_size, const ekv_tensor* rows
     const bool dense = a.topk_sk == 1 && a.sl_o == 1 && a.mi_o == 1 && a.st_c == 1 && a.sp_c == 1 && a.ps_o == 1 &&
                        a.pd_o == 1 && a.tb_t == 1 && a.host_st == 1 && (a.bits == nullptr || a.bt_w == 1) &&
                        (a.line_counts == nullptr || a.lc_q == 1) && T < (int64_t{1} << 29);
+    if (lengths_p != nullptr) {
+        if (!dense) {
+            return kNeedsLookup;
+        }
+        a.lengths = index_ref(*lengths_p, 0);
+    }
     const int64_t four = std::max((C + 3) / 4, (W + 1) / 2), eight = std::max((C + 7) / 8, (W + 3) / 4);
     const bool crowded = count * L > kCus && four > 128;
     if (four <= 64) {
@@ -1170,6 +1302,15 @@ int swap_in(const ekv_tensor* topk_p, int64_t block_size, const ekv_tensor* rows
 }
 
 }  // namespace
+
+bool lookup_swap_in(const ekv_step_args& s, const ekv_tensor& misses, const ekv_tensor& counts, const ekv_tensor& src,
+                    const ekv_tensor& dst, void* stream) {
+    const bool counted = s.step_counter != nullptr;
+    return swap_in(s.topk, s.block_size, s.rows, s.selected, s.slots, &misses, &counts, s.table, s.resident_bits,
+                   s.bits_shift, s.resident_counts, s.slot_token, s.stamps, s.slot_base, s.host_table, &src, &dst,
+                   counted ? 0 : s.step, s.step_counter, s.status, stream, s.lengths) != kNeedsLookup;
+}
+
 }  // namespace ekv
 
 extern "C" int ekv_swap_in(const ekv_tensor* topk, int64_t block_size, const ekv_tensor* rows,

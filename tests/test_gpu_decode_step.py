@@ -254,3 +254,59 @@ def test_argument_errors_name_the_argument(gpu, host):
     torch.cuda.synchronize()
     assert bool((slots == -9).all()) and bool((out == 0x5a).all())
     assert side.buffers.step == 0
+
+
+@pytest.mark.parametrize("table_dtype,shift,with_bits", [(torch.int16, 6, True), (torch.int32, 0, True),
+                                                        (torch.int32, 0, False)])
+@pytest.mark.parametrize("bs,topk_dtype,strided", [(1, torch.int32, False), (1, torch.int64, False),
+                                                   (4, torch.int32, False), (3, torch.int64, False),
+                                                   (1, torch.int32, True)])
+def test_one_launch_lookup_and_swap_equals_the_kernels(gpu, host, table_dtype, shift, with_bits, bs, topk_dtype, strided):
+    # The step looks up and swaps in with one kernel; the entry points use theirs. Over repeated and out-of-range
+    # ids, short, negative and over-long rows, requests without a table row, permuted, stray and doubled selections
+    # (refused rows) and rows sharing a request; a strided slot tensor takes the entry points' kernels in the step too.
+    host_planes, host_table, _ = host
+    staged, fused = Side(gpu, host, table_dtype, shift, False, 5), Side(gpu, host, table_dtype, shift, False, 5)
+    if not with_bits:
+        for side in (staged, fused):
+            side.buffers.bits = None
+    rng = np.random.default_rng(bs * 10 + shift)
+    k = K // bs
+    W = k * bs
+    cases = [([0, 1, 2, 3, 4], [0, 1, 2, 3, 4], [T, T - 3, 40, T, T + 9]),
+             ([3, 1, R + 2, 0, -1], [4, 2, -1, 0, 9, 1], [T, -5, T, T - 7, T]),
+             ([0, 1, 0, 3, 4], [0, 1, 2, 3], [T, T, T, T - 1, T]),              # rows 0 and 2 share a request
+             ([4, 3, 2, 1, 0], [2, 2, 0], [T, T, T - 11, T, T])]                # a doubled entry
+    for step, (rows, selected, lengths) in enumerate(cases):
+        topk = rng.integers(-1, T // bs + 3, (L, R, k))
+        near = rng.random(topk.shape) < 0.7
+        topk[near] = rng.integers((T - 600) // bs, T // bs, topk.shape)[near]
+        if step != 1:
+            topk[..., 1::23] = topk[..., :1]
+        topk = torch.tensor(topk, dtype=topk_dtype, device=gpu)
+        rows, selected = torch.tensor(rows, device=gpu), torch.tensor(selected, device=gpu)
+        lengths = torch.tensor(lengths, dtype=torch.int32, device=gpu)
+        outputs = []
+        for side in (staged, fused):
+            slots = torch.full((L, R, W, 2 if strided else 1), -9, dtype=torch.int32, device=gpu)[..., 0]
+            out = torch.empty((R, L, 2, W, ROW), dtype=torch.uint8, device=gpu)
+            b = side.buffers
+            if side is staged:
+                misses = torch.empty((L, R, W), dtype=torch.int32, device=gpu)
+                counts = torch.zeros((L, R), dtype=torch.int32, device=gpu)
+                resolve_resident(topk, b.table, None, rows, lengths, selected, slots, bs, misses=misses,
+                                 miss_count=counts, resident_bits=b.bits, bits_shift=b.bits_shift,
+                                 slot_base=b.slot_base if table_dtype == torch.int16 else None)
+                src, dst = torch.full_like(misses, -1), torch.full_like(misses, -1)
+                swap_in(topk, bs, rows, selected, slots, misses, counts, b, host_table, src, dst)
+                move_kv(host_planes, src, side.planes, dst, counts)
+                gather_kv(side.planes, slots, out)
+            else:
+                workspace = torch.full((decode_step_workspace(L, R, W),), 0x7f, dtype=torch.uint8, device=gpu)
+                decode_step(topk, rows, lengths, b, host_table, host_planes, side.planes, slots, out, block_size=bs,
+                            selected=selected, workspace=workspace)
+            kept = [t for t in (b.table, b.bits, b.resident_counts, b.slot_token, b.stamps, b.status, side.pool)
+                    if t is not None]
+            outputs.append([slots.cpu(), out.cpu()] + [t.cpu() for t in kept])
+        for a, z in zip(*outputs):
+            assert torch.equal(a, z), step
