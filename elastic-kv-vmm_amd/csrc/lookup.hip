@@ -46,6 +46,7 @@
 #include "ekv_device.h"
 #include "ekv_fastdiv.h"
 #include "ekv_tensor_util.h"
+#include "ekv_wave.h"
 
 #include <algorithm>
 #include <atomic>
@@ -98,6 +99,7 @@ struct LookupArgs {
     int32_t bits_staged;                 // stage the bitmap row in LDS
     int32_t runs;                        // int16 local form: contiguous 8-lane runs per thread
     int32_t pipe;                        // ... of one chunk, prefetching persistent form
+    int32_t direct;                      // small jobs: entries read without the summary
     int32_t block_runs;                  // whole blocks of a multiple of 8 tokens: runs of 8 neighbouring entries
     uint32_t width;
     uint32_t block_size;
@@ -841,6 +843,108 @@ void resolve_runs_pipe_kernel(const LookupArgs a, uint32_t items, uint32_t count
     }
 }
 
+// Single-level lookups read entry by entry without their summary: two memory
+// levels - ids (and the indexes, with the identity selection guessed), then
+// entries - and one barrier, where the prefetching kernels have a summary row to
+// stage in between. A row's lanes are spread over kWidth threads of kLanes
+// strided lanes, so rows of any width and alignment take it. One layer's lookup
+// of 32 requests x 2048 lanes: 5.5 -> 4.0 us; see the rule that chooses it for more.
+template <typename TopkT, typename TableT, int kWidth, int kLanes, bool kCompact>
+__global__ __launch_bounds__(kWidth) void resolve_direct_kernel(const LookupArgs a) {
+    constexpr int kWaves = kWidth / 64;
+    constexpr uint32_t kSpan = kWidth * kLanes;
+    __shared__ uint32_t cells[2][kLanes * kWaves];   // miss counts per (lane register, wave), by chunk parity
+    const int64_t layer = blockIdx.y;
+    const uint32_t zero = opaque_zero();
+    const int64_t guess = blockIdx.x < a.batch ? blockIdx.x : 0;
+    PendingIndex entry_read = issue_index(a.selected, blockIdx.x, zero);
+    PendingIndex req_read = issue_index(a.rows, guess, zero);
+    PendingIndex length_read = issue_index(a.lengths, guess, zero);
+    const TopkT* topk_rows = static_cast<const TopkT*>(a.topk) + layer * a.topk_sl;
+    TopkT block[kLanes];
+    const auto load_ids = [&](int64_t row, uint32_t chunk) {
+#pragma unroll
+        for (int k = 0; k < kLanes; ++k) {
+            const uint32_t o = chunk + threadIdx.x + k * kWidth;
+            block[k] = stream_load(element<true>(topk_rows + row * a.topk_sb, 1,
+                                                 a.block_div.div(o < a.width ? o : a.width - 1)));
+        }
+    };
+    load_ids(guess, 0);
+    asm volatile("" : "+v"(entry_read.lo), "+v"(entry_read.hi), "+v"(req_read.lo), "+v"(req_read.hi),
+                 "+v"(length_read.lo), "+v"(length_read.hi));   // one wait for all of them
+    const int64_t entry = index_value(a.selected, entry_read);
+    const bool live = entry >= 0 && entry < a.batch;  // uniform
+    const int64_t row = live ? entry : guess;
+    int64_t req = index_value(a.rows, req_read);
+    int64_t length = index_value(a.lengths, length_read);
+    if (row != guess) {  // uniform: the selection is not the identity here
+        req = a.rows.fetch(row);
+        length = a.lengths.fetch(row);
+        load_ids(row, 0);
+    }
+    const uint32_t width = live ? a.width : 0u;  // a stray entry runs no chunk
+    const bool table_ok = req >= 0 && req < a.table_rows;  // uniform (the table has entries)
+    const int64_t req_at = table_ok ? req : 0;
+    const int64_t bound = table_ok ? (length < a.table_cols ? length : a.table_cols) : 0;
+    PendingIndex base_read{0, 0};
+    if constexpr (std::is_same_v<TableT, int16_t>) {
+        base_read = issue_index(a.slot_base, req_at, zero);
+    }
+    const TableT* table = static_cast<const TableT*>(a.table) + layer * a.table_sl + req_at * a.table_sr;
+    int32_t* out = a.out + layer * a.out_sl + row * a.out_sb;
+    int32_t* misses = kCompact ? a.misses + layer * a.miss_sl + row * a.miss_sb : nullptr;
+    int32_t running = 0;
+    uint32_t parity = 0;
+    for (uint32_t chunk = 0; chunk < width; chunk += kSpan, parity ^= 1u) {
+        if (chunk != 0) {
+            load_ids(row, chunk);
+        }
+        TableT held[kLanes];
+        uint32_t valid_bits = 0;
+#pragma unroll
+        for (int k = 0; k < kLanes; ++k) {
+            bool valid;
+            const uint32_t p = lane_position(a, chunk + threadIdx.x + k * kWidth, block[k], bound, table_ok, valid);
+            valid_bits |= static_cast<uint32_t>(valid) << k;
+            held[k] = *element<true>(table, 1, p);   // invalid lanes read entry 0 of the row
+        }
+        const int64_t base = std::is_same_v<TableT, int16_t> ? index_value(a.slot_base, base_read) : 0;
+        uint32_t missed[kLanes], miss_bits = 0;
+#pragma unroll
+        for (int k = 0; k < kLanes; ++k) {
+            const uint32_t o = chunk + threadIdx.x + k * kWidth;
+            const int32_t slot = (valid_bits >> k) & 1u ? entry_slot<TableT>(held[k], base) : -1;
+            if (o < width) {
+                stream_store(slot, element<true>(out, 1, o));
+            }
+            miss_bits |= static_cast<uint32_t>(slot == 0) << k;
+            missed[k] = static_cast<uint32_t>(__popcll(__ballot(slot == 0)));
+        }
+        if constexpr (kCompact) {
+            pair_counts<kWaves, kLanes>(missed, cells[parity]);
+            __syncthreads();
+            uint32_t rank[kLanes], total = 0;
+            pair_bases<kWaves, kLanes>(cells[parity], rank, total);
+#pragma unroll
+            for (int k = 0; k < kLanes; ++k) {
+                const bool miss = (miss_bits >> k) & 1u;
+                const uint32_t at = rank[k] + lanes_below(__ballot(miss));
+                if (miss) {
+                    *element<true>(misses, 1, static_cast<uint32_t>(running) + at) =
+                        static_cast<int32_t>(chunk + threadIdx.x + k * kWidth);
+                }
+            }
+            running += static_cast<int32_t>(total);
+        }
+    }
+    if constexpr (kCompact) {
+        if (threadIdx.x == 0 && live) {
+            a.counts[layer * a.count_sl + row * a.count_sb] = running;
+        }
+    }
+}
+
 // Single-level lookups of whole token blocks (block size a multiple of 8): a
 // block's tokens are neighbours in the table, so a thread's 8 consecutive lanes
 // are one Top-K id, one 16-byte piece of an int16 table (two of an int32
@@ -1096,9 +1200,8 @@ __global__ __launch_bounds__(kThreads) void resolve_mapped_kernel(const LookupAr
 // they had been a chain of six or more dependent round trips (one layer per
 // launch: 5.9 against 6.3 us).
 
-// Where the two-stage kernel's threads store slot pieces that no output row
-// takes (past a row's width, or of an item with no batch row): written by
-// every such store, read by nothing.
+// Where the two-stage kernel's threads store the slot pieces of an item with
+// no batch row: written by every such store, read by nothing.
 __device__ i32x4 discarded_pieces[kThreads];
 
 // One item between its two stages: its table entries in flight and its lanes'
@@ -1106,7 +1209,7 @@ __device__ i32x4 discarded_pieces[kThreads];
 struct RunsPending {
     int32_t entry[kIters];
     uint32_t need;      // bit j: lane j is resident, its entry decides its slot
-    uint32_t invalid;   // bit j: lane j is padding or out of range (slot -1)
+    uint32_t invalid;   // bit j: lane j is out of range (slot -1)
 };
 
 // An item's summary row into `staged` (its first stage's barrier publishes
@@ -1122,8 +1225,7 @@ __device__ __forceinline__ void runs_stage(const RunsLoads<1>& loads, uint32_t* 
 // barrier every thread passes, classify its lanes and issue its table reads.
 template <typename TableT>
 __device__ __forceinline__ void runs_begin(const LookupArgs& a, uint32_t layer, const RunsMeta& m,
-                                           const RunsLoads<1>& loads, uint32_t* staged,
-                                           const bool (&live_piece)[2], RunsPending& p) {
+                                           const RunsLoads<1>& loads, uint32_t* staged, RunsPending& p) {
     const bool table_ok = m.row != kNoRow && m.req != kNoRow;   // uniform
     __syncthreads();
     const int32_t block[kIters] = {loads.ids[0].x, loads.ids[0].y, loads.ids[0].z, loads.ids[0].w,
@@ -1133,7 +1235,7 @@ __device__ __forceinline__ void runs_begin(const LookupArgs& a, uint32_t layer, 
     p.invalid = 0;
 #pragma unroll
     for (int j = 0; j < kIters; ++j) {
-        const bool valid = live_piece[j / 4] & table_ok & (block[j] >= 0) & (block[j] < m.bound);
+        const bool valid = table_ok & (block[j] >= 0) & (block[j] < m.bound);
         const uint32_t pos = valid ? static_cast<uint32_t>(block[j]) : 0u;
         const uint32_t q = pos >> a.bits_shift;
         const uint32_t word = staged[q >> 5];
@@ -1299,7 +1401,7 @@ void resolve_runs_pipe2_kernel(const LookupArgs a, uint32_t items, uint32_t coun
     const PendingIndex len_mine = issue_index(a.lengths, mine.row != kNoRow ? mine.row : 0u, zero);
     RunsPending pend;
     runs_stage(first_loads, staged_bits[0], last_piece);
-    runs_begin<TableT>(a, layer, cur, first_loads, staged_bits[0], live_piece, pend);
+    runs_begin<TableT>(a, layer, cur, first_loads, staged_bits[0], pend);
     meta_apply(a, mine, lane_value(a.rows, req_mine), lane_value(a.lengths, len_mine));
     if constexpr (std::is_same_v<TableT, int16_t>) {
         const PendingIndex base_mine = issue_index(a.slot_base, mine.req != kNoRow ? mine.req : 0u, zero);
@@ -1330,16 +1432,20 @@ void resolve_runs_pipe2_kernel(const LookupArgs a, uint32_t items, uint32_t coun
         runs_stage(next_loads, staged_bits[(k + 1) & 1], last_piece);
         const bool live = cur.row != kNoRow;   // uniform
         {
-            // Two stores on every path: a piece past the row or of an item
-            // with no batch row goes to a scratch word block nobody reads. With
-            // conditional stores the compiler could not count the stores in
-            // flight and waited for all of them (their acknowledgements)
-            // before staging the next item's summary row.
+            // Two stores on every path: a piece past the row holds the row's
+            // last piece (its ids were read there) and stores it again, one of
+            // an item with no batch row goes to a scratch word block nobody
+            // reads. With conditional stores the compiler could not count the
+            // stores in flight and waited for all of them (their
+            // acknowledgements) before staging the next item's summary row.
+            // (Pieces past the row went to the scratch block too, where the
+            // whole chip's stores met on one 4 KiB: 2,560 rows of 1024 lanes took 50.7 us.)
             int32_t* out = a.out + layer * a.out_sl + (live ? cur.row : 0u) * a.out_sb;
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
-                i32x4* to = live && live_piece[h] ? reinterpret_cast<i32x4*>(element<true>(out, 1, first[h]))
-                                                  : &discarded_pieces[threadIdx.x];
+                i32x4* to = live ? reinterpret_cast<i32x4*>(
+                                       element<true>(out, 1, live_piece[h] ? first[h] : a.width - kPiece))
+                                 : &discarded_pieces[threadIdx.x];
                 stream_store(i32x4{slot[4 * h], slot[4 * h + 1], slot[4 * h + 2], slot[4 * h + 3]}, to);
             }
         }
@@ -1355,7 +1461,7 @@ void resolve_runs_pipe2_kernel(const LookupArgs a, uint32_t items, uint32_t coun
         uint32_t layer_after = layer_next;
         RunsLoads<1> after_loads = next_loads;
         if (more) {
-            runs_begin<TableT>(a, layer_next, nxt, next_loads, staged_bits[(k + 1) & 1], live_piece, pend);
+            runs_begin<TableT>(a, layer_next, nxt, next_loads, staged_bits[(k + 1) & 1], pend);
             const uint32_t k_after = k + 2 < n ? k + 2 : k + 1;
             after = runs_meta(meta, k_after);
             layer_after = count_div.div(blockIdx.x + k_after * gridDim.x);
@@ -1503,6 +1609,31 @@ void launch_runs_pipe(const LookupArgs& a, dim3 grid, hipStream_t stream) {
     }
 }
 
+// Four lanes per thread: the smallest workgroup that holds the row (rows past
+// 2048 lanes are not given to the direct kernel). More lanes per thread are a longer chain in a small job
+// (32 rows of 2048 lanes: 4.57 us with 256 threads of eight, 4.02 with 512 of four).
+constexpr int kDirectLanes = 4;
+
+template <typename TopkT, typename TableT, int kWidth>
+void launch_direct_width(const LookupArgs& a, bool compact, dim3 grid, hipStream_t stream) {
+    const auto kernel = compact ? resolve_direct_kernel<TopkT, TableT, kWidth, kDirectLanes, true>
+                                : resolve_direct_kernel<TopkT, TableT, kWidth, kDirectLanes, false>;
+    kernel<<<grid, dim3(kWidth), 0, stream>>>(a);
+}
+
+template <typename TopkT, typename TableT>
+void launch_direct(const LookupArgs& a, bool compact, dim3 grid, hipStream_t stream) {
+    if (a.width <= 64 * kDirectLanes) {
+        launch_direct_width<TopkT, TableT, 64>(a, compact, grid, stream);
+    } else if (a.width <= 128 * kDirectLanes) {
+        launch_direct_width<TopkT, TableT, 128>(a, compact, grid, stream);
+    } else if (a.width <= 256 * kDirectLanes) {
+        launch_direct_width<TopkT, TableT, 256>(a, compact, grid, stream);
+    } else {
+        launch_direct_width<TopkT, TableT, 512>(a, compact, grid, stream);
+    }
+}
+
 template <typename TopkT, typename TableT>
 void launch_with_table(const LookupArgs& a, int32_t map_dtype, bool compact, bool dense, dim3 grid,
                        hipStream_t stream) {
@@ -1517,6 +1648,10 @@ void launch_with_table(const LookupArgs& a, int32_t map_dtype, bool compact, boo
                 } else {
                     resolve_blocks_kernel<TopkT, TableT, false><<<grid, block, 0, stream>>>(a);
                 }
+                return;
+            }
+            if (a.direct) {
+                launch_direct<TopkT, TableT>(a, compact, grid, stream);
                 return;
             }
         }
@@ -1846,6 +1981,28 @@ int resolve_resident(const ekv_tensor* topk_p, const ekv_tensor* table_p, const 
                            rows_aligned(output.data, a.out_sl, layers, a.out_sb, batch)
                        ? 1
                        : 0;
+    // Entry by entry without the summary: rows of up to 1024 lanes, and wider
+    // ones while few rows share the chip. The summary kernels are a memory level and
+    // several barriers longer, and their workgroups take 2048 lanes
+    // whatever the row; but at wide rows in number the entry reads that
+    // the summary spares are what counts. Before and after, us:
+    //   rows x lanes          summary kernels    direct
+    //   4 x 2048                    5.31          3.84
+    //   32 x 2047 (ragged)          7.17          4.32
+    //   198 x 479, int32            6.97          3.77
+    //   512 x 2048                  7.17          6.46
+    //   768 x 2048                  8.32         11.23
+    //   2560 x 2047 (ragged)       23.3          30.9
+    //   1280 x 1024                26.8           9.3
+    //   2560 x 1023 (ragged)       19.3          17.6
+    //   5120 x 1023 (ragged)       32.3          32.2
+    //   7680 x 512                 61.0          26.2
+    //   7680 x 257, int32          41.8          21.8
+    constexpr int64_t kNarrow = 1024, kFewRows = 512;
+    a.direct = mapping == nullptr && entry_bytes <= 4 && dense && a.table_rows > 0 && a.table_cols > 0 &&
+                       (width <= kNarrow || (width <= kChunkLanes && count * layers <= kFewRows))
+                   ? 1
+                   : 0;
     if (check_only()) {
         return 0;
     }

@@ -379,3 +379,51 @@ def test_whole_block_lookups_match_oracle_and_general_path(gpu, bs, k, cols, dty
             out.fill_(-77)
             resolve_resident(*args, **extra)                                       # without compaction
             assert np.array_equal(out.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("bs,k,batch", [(1, 1, 5), (1, 256, 5), (1, 257, 5), (1, 512, 5), (3, 171, 5), (1, 1024, 5),
+                                        (1, 1025, 5), (2, 1024, 5), (1, 2048, 5), (1, 300, 300), (1, 1032, 300),
+                                        (1, 1201, 300)])
+@pytest.mark.parametrize("dtype", [torch.int16, torch.int32])
+def test_direct_lookups_match_oracle_and_general_path(gpu, bs, k, batch, dtype):
+    # Rows on both sides of every workgroup width, few rows and more rows than the wide ones take (300 rows over two
+    # layers: the prefetching kernel, whose threads past the row store the last piece again, or the general one), stray
+    # selections and requests, short and negative lengths; a strided output takes the general kernel.
+    from adaptive_sparse.resident_lookup import build_residency_bits
+    from oracle import oracle as ref
+
+    rng = np.random.default_rng(bs * 10000 + k + batch)
+    layers, table_rows, cols = 2, 7, 4001
+    local = rng.integers(1, 1 << 15, (layers, table_rows, cols)) * (rng.random((layers, table_rows, cols)) < 0.5)
+    local = np.where(rng.random(local.shape) < 0.02, -local, local)
+    base = rng.integers(1, 1 << 20, table_rows)
+    table = np.where(local > 0, base.reshape(1, -1, 1) + local - 1, 0) if dtype == torch.int16 else local
+    topk = rng.integers(-1, cols // bs + 2, (layers, batch, k))
+    lengths = rng.integers(cols // 2, cols + 9, batch)
+    lengths[:2] = (cols, -4)
+    rows = rng.integers(0, table_rows, batch)
+    rows[3] = table_rows                                                          # names no table row
+    width = k * bs
+    table_d = torch.tensor(local, dtype=dtype, device=gpu)
+    bits = build_residency_bits(table_d, shift=6)
+    for selected in (np.arange(batch), np.array([3, 0, -1, 4, batch, 2])):
+        want, want_misses, want_counts = ref.resolve_resident(topk, table, None, rows, lengths, selected, bs,
+                                                              np.full((layers, batch, width), -77, np.int32),
+                                                              with_misses=True)
+        for topk_dtype, summary, step in ((torch.int32, True, 1), (torch.int64, False, 1), (torch.int32, True, 2)):
+            out = torch.full((layers, batch, width, step), -77, dtype=torch.int32, device=gpu)[..., 0]
+            misses = torch.full((layers, batch, width), -5, dtype=torch.int32, device=gpu)
+            counts = torch.full((layers, batch), -5, dtype=torch.int32, device=gpu)
+            args = (torch.tensor(topk, dtype=topk_dtype, device=gpu), table_d, None, torch.tensor(rows, device=gpu),
+                    torch.tensor(lengths, dtype=torch.int32, device=gpu), torch.tensor(selected, device=gpu), out, bs)
+            extra = dict(resident_bits=bits if summary else None, bits_shift=6 if summary else 0,
+                         slot_base=torch.tensor(base, device=gpu) if dtype == torch.int16 else None)
+            resolve_resident(*args, misses=misses, miss_count=counts, **extra)
+            assert np.array_equal(out.cpu().numpy(), want), (len(selected), topk_dtype, step)
+            got_counts, got = counts.cpu().numpy(), misses.cpu().numpy()
+            for (layer, r), lanes in want_misses.items():
+                assert got_counts[layer, r] == want_counts[layer, r] == len(lanes)
+                assert np.array_equal(got[layer, r, :len(lanes)], lanes)
+            out.fill_(-77)
+            resolve_resident(*args, **extra)                                       # without compaction
+            assert np.array_equal(out.cpu().numpy(), want)
