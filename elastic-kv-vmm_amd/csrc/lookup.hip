@@ -849,7 +849,9 @@ void resolve_runs_pipe_kernel(const LookupArgs a, uint32_t items, uint32_t count
 // stage in between. A row's lanes are spread over kWidth threads of kLanes
 // strided lanes, so rows of any width and alignment take it. One layer's lookup
 // of 32 requests x 2048 lanes: 5.5 -> 4.0 us; see the rule that chooses it for more.
-template <typename TopkT, typename TableT, int kWidth, int kLanes, bool kCompact>
+// MapT: void, or the element type of the second level (table -> logical id ->
+// mapping -> slot): a third memory level, as resolve_mapped_kernel reads it.
+template <typename TopkT, typename TableT, typename MapT, int kWidth, int kLanes, bool kCompact>
 __global__ __launch_bounds__(kWidth) void resolve_direct_kernel(const LookupArgs a) {
     constexpr int kWaves = kWidth / 64;
     constexpr uint32_t kSpan = kWidth * kLanes;
@@ -909,12 +911,28 @@ __global__ __launch_bounds__(kWidth) void resolve_direct_kernel(const LookupArgs
             valid_bits |= static_cast<uint32_t>(valid) << k;
             held[k] = *element<true>(table, 1, p);   // invalid lanes read entry 0 of the row
         }
+        int32_t mapped[kLanes];
+        if constexpr (!std::is_void_v<MapT>) {
+            const MapT* mapping = static_cast<const MapT*>(a.mapping) + layer * a.map_sl;
+#pragma unroll
+            for (int k = 0; k < kLanes; ++k) {
+                const int64_t logical = held[k];
+                const bool hit = ((valid_bits >> k) & 1u) && logical >= 0 && logical < a.map_len;
+                valid_bits = hit ? valid_bits : valid_bits & ~(1u << k);
+                mapped[k] = static_cast<int32_t>(mapping[hit ? logical : 0]);   // the mapping is not empty
+            }
+        }
         const int64_t base = std::is_same_v<TableT, int16_t> ? index_value(a.slot_base, base_read) : 0;
         uint32_t missed[kLanes], miss_bits = 0;
 #pragma unroll
         for (int k = 0; k < kLanes; ++k) {
             const uint32_t o = chunk + threadIdx.x + k * kWidth;
-            const int32_t slot = (valid_bits >> k) & 1u ? entry_slot<TableT>(held[k], base) : -1;
+            int32_t slot;
+            if constexpr (std::is_void_v<MapT>) {
+                slot = (valid_bits >> k) & 1u ? entry_slot<TableT>(static_cast<int32_t>(held[k]), base) : -1;
+            } else {
+                slot = (valid_bits >> k) & 1u ? mapped[k] : -1;
+            }
             if (o < width) {
                 stream_store(slot, element<true>(out, 1, o));
             }
@@ -1439,7 +1457,8 @@ void resolve_runs_pipe2_kernel(const LookupArgs a, uint32_t items, uint32_t coun
             // stores in flight and waited for all of them (their
             // acknowledgements) before staging the next item's summary row.
             // (Pieces past the row went to the scratch block too, where the
-            // whole chip's stores met on one 4 KiB: 2,560 rows of 1024 lanes took 50.7 us.)
+            // whole chip's stores met on one 4 KiB: 2,560 rows of 1024 lanes took 50.7 us,
+            // 14.7 so.)
             int32_t* out = a.out + layer * a.out_sl + (live ? cur.row : 0u) * a.out_sb;
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
@@ -1613,11 +1632,12 @@ void launch_runs_pipe(const LookupArgs& a, dim3 grid, hipStream_t stream) {
 // 2048 lanes are not given to the direct kernel). More lanes per thread are a longer chain in a small job
 // (32 rows of 2048 lanes: 4.57 us with 256 threads of eight, 4.02 with 512 of four).
 constexpr int kDirectLanes = 4;
+constexpr int64_t kMappedDirectRows = 512;
 
-template <typename TopkT, typename TableT, int kWidth>
+template <typename TopkT, typename TableT, int kWidth, typename MapT = void>
 void launch_direct_width(const LookupArgs& a, bool compact, dim3 grid, hipStream_t stream) {
-    const auto kernel = compact ? resolve_direct_kernel<TopkT, TableT, kWidth, kDirectLanes, true>
-                                : resolve_direct_kernel<TopkT, TableT, kWidth, kDirectLanes, false>;
+    const auto kernel = compact ? resolve_direct_kernel<TopkT, TableT, MapT, kWidth, kDirectLanes, true>
+                                : resolve_direct_kernel<TopkT, TableT, MapT, kWidth, kDirectLanes, false>;
     kernel<<<grid, dim3(kWidth), 0, stream>>>(a);
 }
 
@@ -1711,6 +1731,17 @@ void launch_with_table(const LookupArgs& a, int32_t map_dtype, bool compact, boo
             resolve_single_kernel<TopkT, TableT, false, false, false><<<grid, block, lds, stream>>>(a);
         }
     } else if constexpr (!std::is_same_v<TableT, int16_t>) {  // local tables are single level
+        if (a.direct) {
+            const bool narrow = a.width <= 128 * kDirectLanes;
+            if (map_dtype == EKV_INT64) {
+                narrow ? launch_direct_width<TopkT, TableT, 128, int64_t>(a, compact, grid, stream)
+                       : launch_direct_width<TopkT, TableT, 512, int64_t>(a, compact, grid, stream);
+            } else {
+                narrow ? launch_direct_width<TopkT, TableT, 128, int32_t>(a, compact, grid, stream)
+                       : launch_direct_width<TopkT, TableT, 512, int32_t>(a, compact, grid, stream);
+            }
+            return;
+        }
         if (map_dtype == EKV_INT64) {
             if (compact) {
                 resolve_mapped_kernel<TopkT, TableT, int64_t, true><<<grid, block, lds, stream>>>(a);
@@ -1981,28 +2012,31 @@ int resolve_resident(const ekv_tensor* topk_p, const ekv_tensor* table_p, const 
                            rows_aligned(output.data, a.out_sl, layers, a.out_sb, batch)
                        ? 1
                        : 0;
-    // Entry by entry without the summary: rows of up to 1024 lanes, and wider
-    // ones while few rows share the chip. The summary kernels are a memory level and
-    // several barriers longer, and their workgroups take 2048 lanes
-    // whatever the row; but at wide rows in number the entry reads that
-    // the summary spares are what counts. Before and after, us:
-    //   rows x lanes          summary kernels    direct
-    //   4 x 2048                    5.31          3.84
-    //   32 x 2047 (ragged)          7.17          4.32
-    //   198 x 479, int32            6.97          3.77
-    //   512 x 2048                  7.17          6.46
-    //   768 x 2048                  8.32         11.23
-    //   2560 x 2047 (ragged)       23.3          30.9
-    //   1280 x 1024                26.8           9.3
-    //   2560 x 1023 (ragged)       19.3          17.6
-    //   5120 x 1023 (ragged)       32.3          32.2
-    //   7680 x 512                 61.0          26.2
-    //   7680 x 257, int32          41.8          21.8
-    constexpr int64_t kNarrow = 1024, kFewRows = 512;
-    a.direct = mapping == nullptr && entry_bytes <= 4 && dense && a.table_rows > 0 && a.table_cols > 0 &&
-                       (width <= kNarrow || (width <= kChunkLanes && count * layers <= kFewRows))
-                   ? 1
-                   : 0;
+    // Entry by entry without the summary, while the entry reads that a summary
+    // would spare are few: the other kernels are a memory level and a barrier
+    // or two longer, and their workgroups take 2048 lanes whatever the row.
+    // The lines lie where the table bytes read by the whole job make up for
+    // it; measured (us; prefetching or, for ragged rows, strided kernel / direct):
+    //   4 x 2048             5.31 /  3.84    512 x 2048, int32    6.35 /  7.60
+    //   32 x 2047 ragged     7.17 /  4.32    768 x 2048           8.32 / 11.23
+    //   512 x 2048           7.17 /  6.46    1024 x 2047 ragged  11.23 / 14.26
+    //   640 x 1024, int32    5.97 /  5.17    1280 x 1024, int32   8.80 / 10.07
+    //   1280 x 1024         10.10 /  9.22    2560 x 1024         14.74 / 16.84
+    //   2560 x 1023 ragged  19.45 / 17.60    2560 x 1023, int32  18.77 / 19.58
+    //   7680 x 512          26.62 / 26.68    7680 x 512, int32   28.59 / 30.82
+    //   7680 x 511 ragged   42.89 / 28.85    7680 x 511, int32   43.14 / 32.41
+    //   7680 x 256          25.78 / 16.99    7680 x 256, int32   26.37 / 20.64
+    const int64_t entries_read = count * layers * std::min<int64_t>(width, kChunkLanes) * entry_bytes;   // bytes
+    const bool ragged = a.pipe == 0;
+    const bool spared = width <= 256    ? false
+                        : width <= 512  ? !ragged && entries_read > (int64_t{10} << 20)
+                        : width <= 1024 ? entries_read > (ragged ? int64_t{11} << 19 : int64_t{11} << 18)
+                                        : entries_read > int64_t{11} << 18;
+    const bool one_level = mapping == nullptr && entry_bytes <= 4 && !spared;
+    // Two levels have no summary to spare; direct for as many rows as were measured shorter
+    // (us): 4 x 2048 5.18 -> 3.63, 256 x 2048 9.19 -> 7.47, 512 x 2048 13.16 -> 11.96.
+    const bool two_levels = mapping != nullptr && a.map_len > 0 && a.map_s == 1 && count * layers <= kMappedDirectRows;
+    a.direct = dense && a.table_rows > 0 && a.table_cols > 0 && width <= kChunkLanes && (one_level || two_levels) ? 1 : 0;
     if (check_only()) {
         return 0;
     }

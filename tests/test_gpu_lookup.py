@@ -383,7 +383,7 @@ def test_whole_block_lookups_match_oracle_and_general_path(gpu, bs, k, cols, dty
 
 @pytest.mark.parametrize("bs,k,batch", [(1, 1, 5), (1, 256, 5), (1, 257, 5), (1, 512, 5), (3, 171, 5), (1, 1024, 5),
                                         (1, 1025, 5), (2, 1024, 5), (1, 2048, 5), (1, 300, 300), (1, 1032, 300),
-                                        (1, 1201, 300)])
+                                        (1, 1201, 300), (1, 1200, 700), (1, 2040, 360)])
 @pytest.mark.parametrize("dtype", [torch.int16, torch.int32])
 def test_direct_lookups_match_oracle_and_general_path(gpu, bs, k, batch, dtype):
     # Rows on both sides of every workgroup width, few rows and more rows than the wide ones take (300 rows over two
