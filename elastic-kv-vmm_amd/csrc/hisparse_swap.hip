@@ -24,7 +24,7 @@
 // recent), device_buffer_locs[r, i] (device row of slot i; column H is the
 // reserved newest-token row), host_cache_locs[r, t] (host row of token t).
 //
-// One 1024-thread workgroup per batch row:
+// One workgroup per batch row:
 //   1. the hot tokens are hashed into LDS (open addressing, at least 2H
 //      buckets holding slot ids, so every probe sequence meets an empty
 //      bucket);
@@ -48,6 +48,7 @@
 #include "ekv_fastdiv.h"
 #include "ekv_tensor_util.h"
 #include "ekv_vec.h"
+#include "ekv_wave.h"
 
 #include <algorithm>
 #include <atomic>
@@ -56,16 +57,13 @@
 namespace ekv {
 namespace {
 
-// Threads of the swap: one workgroup per batch row holds its CU alone (134 KiB of
-// LDS at the largest shape) and is a chain of barriers, so the more waves share its
-// loops the shorter it is: 23 us for 24 rows of 2048 lanes and 4096 slots with
-// 1024 threads, 44 us with 256.
-constexpr int kThreads = 1024;
-constexpr int kWaves = kThreads / 64;
 constexpr int64_t kMaxHot = 4096;     // hot slots per request (LDS holds the hash and the order)
 constexpr int64_t kMaxLanes = 2048;   // selected lanes per row (Top-K blocks x block size)
-constexpr int kLanesPerThread = static_cast<int>(kMaxLanes / kThreads);
-constexpr int kBatch = 4;             // state loads in flight per thread
+constexpr int kLanesPerThread = 2;    // lanes per thread of the swap at most
+constexpr int kBatch = 4;             // hot slots per thread of the swap at most
+constexpr int kMaxWaves = 16;         // of the largest swap workgroup
+static_assert(kMaxLanes <= kLanesPerThread * 64 * kMaxWaves && kMaxHot <= kBatch * 64 * kMaxWaves,
+              "the largest workgroup holds the largest row");
 constexpr int kSlotBits = 12;         // a miss left for the copy launch: -2 - (miss rank << kSlotBits | slot)
 static_assert(kMaxHot <= 1 << kSlotBits && kMaxLanes << kSlotBits < int64_t{1} << 30, "slot and rank fit an entry");
 constexpr int32_t kEmpty = -1;
@@ -120,13 +118,13 @@ struct Lds {
     int32_t* lane_val;    // [W] hit: its device row (-1: outside the buffer); miss: its host row
     int32_t* miss_loc;    // [W] device row of the m-th miss (-1: none)
     uint8_t* lane_kind;   // [W]
-    int32_t* scratch;     // [3 * kWaves + 4]
+    int32_t* scratch;     // [3 * kMaxWaves + 4]
 };
 
 // Exclusive prefix sums of N per-thread counts over the workgroup's threads
-// in thread order, and their totals: a wave64 shuffle scan, then one LDS
+// in thread order, and their totals: a wave64 scan, then one LDS
 // exchange of the wave totals. Every thread must call it (two barriers).
-template <int N>
+template <int N, int kWaves>
 __device__ __forceinline__ void scan_counts(const int32_t (&count)[N], int32_t (&prefix)[N], int32_t (&total)[N],
                                             int32_t* scratch) {
     const int lane = threadIdx.x & 63;
@@ -134,12 +132,7 @@ __device__ __forceinline__ void scan_counts(const int32_t (&count)[N], int32_t (
     int32_t inclusive[N];
 #pragma unroll
     for (int k = 0; k < N; ++k) {
-        int32_t v = count[k];
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const int32_t t = __shfl_up(v, d, 64);
-            v += lane >= d ? t : 0;
-        }
+        const int32_t v = static_cast<int32_t>(wave_scan<kAdd>(static_cast<uint32_t>(count[k])));
         inclusive[k] = v;
         if (lane == 63) {
             scratch[k * kWaves + wave] = v;
@@ -176,7 +169,14 @@ __device__ __forceinline__ int64_t device_row(const HsArgs& a, int64_t r, int64_
     return row >= 0 && row < a.dev_rows ? row : -1;
 }
 
+// One workgroup per batch row holds its CU nearly alone (134 KiB of LDS at the
+// largest shape) and is a chain of barriers, so the more waves share its loops the
+// shorter it is: kThreads is the smallest size whose threads hold four hot slots
+// and two lanes each. 24 rows of 2048 lanes and 4096 slots: 44 us with 256
+// threads, 23 us with 1024.
+template <int kThreads>
 __global__ __launch_bounds__(kThreads) void hisparse_swap_kernel(const HsArgs a) {
+    constexpr int kWaves = kThreads / 64;
     extern __shared__ __align__(16) unsigned char shared[];
     const int64_t b = blockIdx.x;
     const int64_t H = a.H, W = a.width;
@@ -202,7 +202,7 @@ __global__ __launch_bounds__(kThreads) void hisparse_swap_kernel(const HsArgs a)
         s.lane_val = reinterpret_cast<int32_t*>(take(W * 4));
         s.miss_loc = reinterpret_cast<int32_t*>(take(W * 4));
         s.lane_kind = reinterpret_cast<uint8_t*>(take(W));
-        s.scratch = reinterpret_cast<int32_t*>(take((3 * kWaves + 4) * 4));
+        s.scratch = reinterpret_cast<int32_t*>(take((3 * kMaxWaves + 4) * 4));
     }
     int32_t* out = a.out + b * a.out_sb;
     const int64_t real = a.num_real.data != nullptr ? a.num_real[0] : a.batch;
@@ -216,6 +216,17 @@ __global__ __launch_bounds__(kThreads) void hisparse_swap_kernel(const HsArgs a)
         return;  // uniform over the workgroup
     }
     int32_t* tokens = a.tokens + r * a.tok_sr;
+
+    const void* topk_row = a.topk64 ? static_cast<const void*>(static_cast<const int64_t*>(a.topk) + b * a.topk_sb)
+                                    : static_cast<const void*>(static_cast<const int32_t*>(a.topk) + b * a.topk_sb);
+    // The row's Top-K ids are requested with its state, which they do not depend on.
+    int64_t block[kLanesPerThread];
+#pragma unroll
+    for (int k = 0; k < kLanesPerThread; ++k) {
+        const int64_t o = threadIdx.x + k * kThreads;
+        const uint32_t at = static_cast<uint32_t>(o < W ? o : W - 1);
+        block[k] = load_index(topk_row, a.topk64, a.block_div.div(at) * a.topk_sk);
+    }
 
     // 1. Load the hot tokens and the LRU order (kBatch loads per thread in
     //    flight at once, clamped indices); build the hash.
@@ -274,19 +285,10 @@ __global__ __launch_bounds__(kThreads) void hisparse_swap_kernel(const HsArgs a)
     __syncthreads();
 
     // 2. Classify every lane (a thread holds lanes threadIdx.x + 256 k):
-    //    Top-K loads of all its lanes first, then the hash probes (a hit marks
-    //    its slot, a miss claims a bucket), then one batch of loads: the
-    //    device row of each hit, the host row of each miss.
-    const void* topk_row = a.topk64 ? static_cast<const void*>(static_cast<const int64_t*>(a.topk) + b * a.topk_sb)
-                                    : static_cast<const void*>(static_cast<const int32_t*>(a.topk) + b * a.topk_sb);
+    //    the hash probes (a hit marks its slot, a miss claims a bucket), then
+    //    one batch of loads: the device row of each hit, the host row of each
+    //    miss.
     {
-        int64_t block[kLanesPerThread];
-#pragma unroll
-        for (int k = 0; k < kLanesPerThread; ++k) {
-            const int64_t o = threadIdx.x + k * kThreads;
-            const uint32_t at = static_cast<uint32_t>(o < W ? o : W - 1);
-            block[k] = load_index(topk_row, a.topk64, a.block_div.div(at) * a.topk_sk);
-        }
         uint8_t kinds[kLanesPerThread];
         int32_t auxes[kLanesPerThread];
 #pragma unroll
@@ -389,7 +391,7 @@ __global__ __launch_bounds__(kThreads) void hisparse_swap_kernel(const HsArgs a)
             count[2] += first_miss(o);
         }
         int32_t prefix[3], total[3];
-        scan_counts<3>(count, prefix, total, s.scratch);
+        scan_counts<3, kWaves>(count, prefix, total, s.scratch);
         int32_t pos = prefix[0], hit_rank = prefix[1], miss_rank = prefix[2];
         for (int64_t o = begin; o < end; ++o) {
             const uint8_t kind = s.lane_kind[o];
@@ -435,7 +437,7 @@ __global__ __launch_bounds__(kThreads) void hisparse_swap_kernel(const HsArgs a)
             count[1] += c == 3;
         }
         int32_t prefix[2], total[2];
-        scan_counts<2>(count, prefix, total, s.scratch);
+        scan_counts<2, kWaves>(count, prefix, total, s.scratch);
         const int32_t empty = total[0], untouched = total[1];
         const int32_t taken_empty = misses < empty ? misses : empty;
         const int32_t taken_untouched = misses - taken_empty < untouched ? misses - taken_empty : untouched;
@@ -642,11 +644,12 @@ __global__ __launch_bounds__(kCopyThreads) void copy_missed_rows(const HsArgs a,
 size_t lds_bytes(int64_t H, int64_t HB, int64_t W) {
     auto round = [](int64_t bytes) { return static_cast<size_t>((bytes + 15) & ~int64_t{15}); };
     return round(HB * 4) + round(H * 4) * 2 + round(H * 2) * 2 + round(W * 2) * 3 + round(W * 4) * 5 + round(W) +
-           round((3 * kWaves + 4) * 4);
+           round((3 * kMaxWaves + 4) * 4);
 }
 
-void launch_swap(const HsArgs& a, size_t lds, hipStream_t stream) {
-    const auto kernel = hisparse_swap_kernel;
+template <int kThreads>
+void launch_swap_threads(const HsArgs& a, size_t lds, hipStream_t stream) {
+    const auto kernel = hisparse_swap_kernel<kThreads>;
     // The LDS limit is raised once per device, to the largest size any call
     // needs, so calls recorded into a graph make no attribute call.
     static std::atomic<bool> raised[kMaxDevices];
@@ -664,6 +667,18 @@ void launch_swap(const HsArgs& a, size_t lds, hipStream_t stream) {
     }
     kernel<<<dim3(static_cast<uint32_t>(a.batch)), dim3(kThreads), lds, stream>>>(a);
     check_hip(hipGetLastError(), "launch hisparse swap-in");
+}
+
+void launch_swap(const HsArgs& a, size_t lds, hipStream_t stream) {
+    const int64_t threads = std::max((a.H + kBatch - 1) / kBatch,
+                                     (int64_t{a.width} + kLanesPerThread - 1) / kLanesPerThread);
+    if (threads <= 256) {
+        launch_swap_threads<256>(a, lds, stream);
+    } else if (threads <= 512) {
+        launch_swap_threads<512>(a, lds, stream);
+    } else {
+        launch_swap_threads<1024>(a, lds, stream);
+    }
 }
 
 template <int kVecWidth>
