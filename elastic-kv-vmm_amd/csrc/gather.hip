@@ -154,10 +154,20 @@ __device__ __forceinline__ void locate(const EngineArgs& a, int64_t u, int64_t& 
         split_unit(a, u, l, j, kv, k);
         src = -1;
         dst = -1;
+        // The selection entry, and the count and list entries of the row it
+        // names on the guess of the identity selection, are read at once: one
+        // memory level before the row itself instead of three (entries at or past the count are read but not used).
+        const int64_t guess = j < a.move_batch ? j : 0;
+        int32_t count = a.move_counts[l * a.mc_l + guess * a.mc_b];
+        int64_t from = a.move_src_rows[l * a.msr_l + guess * a.msr_b + k * a.msr_i];
+        int64_t to = a.move_dst_rows[l * a.mdr_l + guess * a.mdr_b + k * a.mdr_i];
         const int64_t b = move_row(a, j);
-        if (b >= 0 && k < a.move_counts[l * a.mc_l + b * a.mc_b]) {
-            const int64_t from = a.move_src_rows[l * a.msr_l + b * a.msr_b + k * a.msr_i];
-            const int64_t to = a.move_dst_rows[l * a.mdr_l + b * a.mdr_b + k * a.mdr_i];
+        if (b >= 0 && b != guess) {
+            count = a.move_counts[l * a.mc_l + b * a.mc_b];
+            from = a.move_src_rows[l * a.msr_l + b * a.msr_b + k * a.msr_i];
+            to = a.move_dst_rows[l * a.mdr_l + b * a.mdr_b + k * a.mdr_i];
+        }
+        if (b >= 0 && k < count) {
             if (from >= 0 && from < a.ms_rows && to >= a.zero_below && to < a.pool_rows) {
                 src = l * a.ms_layer_stride + kv * a.ms_kv_stride + from * a.ms_row_stride;
                 dst = l * a.layer_stride + kv * a.kv_stride + to * a.row_stride;

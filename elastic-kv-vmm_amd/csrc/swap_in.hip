@@ -952,7 +952,7 @@ void launch_swap(const SwapArgs& a, bool dense, dim3 grid, size_t lds, hipStream
     auto* kernel = a.lengths.data != nullptr ? swap_in_kernel<kThreads, kSlotRegs, kLaneRegs, true, true>
                    : dense                   ? swap_in_kernel<kThreads, kSlotRegs, kLaneRegs, true, false>
                                              : swap_in_kernel<kThreads, kSlotRegs, kLaneRegs, false, false>;
-    if (lds > 48 * 1024) {
+    if (lds > 60 * 1024) {   // with the static 3 KiB, past the default 64
         check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                                       hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)),
                   "raise the swap-in LDS limit");

@@ -402,8 +402,9 @@ uint64_t ekv_decode_step_workspace_bytes(int64_t layers, int64_t batch, int64_t 
  * keeps its own entry point's contract; the miss list, counts and promotion
  * lists live in `workspace` (a 256-byte aligned device buffer of at least
  * ekv_decode_step_workspace_bytes; its contents on entry do not matter: the
- * counts are zeroed by a kernel first, so rows outside `selected` promote
- * nothing). After the step every selected lane's slot holds its token's row;
+ * promotion reads the counts of selected rows only). The lookup and the
+ * swap-in run as one kernel where the tensors' inner strides are 1. After the
+ * step every selected lane's slot holds its token's row;
  * rows outside `selected` keep their slots and are gathered as they stand.
  * Records no memset, so the call can be captured in a HIP graph.
  * Replaces, for one layer or several: the lookup + host-backed swap of the

@@ -132,3 +132,51 @@ def test_move_from_host_memory_matches_oracle(gpu, row_bytes, kv, layers, batch,
             assert np.array_equal(pool.cpu().numpy(), want)
     finally:
         arena.close()
+
+
+def test_host_moves_replay_from_a_graph(gpu):
+    # A list past the tile kernel's limit: the call asks where its source lies while a stream is captured, and replays
+    # follow rows, counts and host bytes rewritten in place.
+    from adaptive_sparse.host_arena import HostArena
+    from adaptive_sparse.kv_pool import KVPlanes
+    from adaptive_sparse.swap_in import move_kv
+
+    rng = np.random.default_rng(7)
+    batch, k, n, row_bytes = 8, 200, 900, 512
+    arena = HostArena(2 * n * row_bytes)
+    try:
+        pool = torch.zeros((2, batch * k + 1, row_bytes), dtype=torch.uint8, device=gpu)
+
+        def planes(base, rows):
+            return KVPlanes(base=base, device=0, layers=1, kv=2, layer_stride=0, kv_stride=rows * row_bytes,
+                            row_stride=row_bytes, row_bytes=row_bytes, rows=rows, owner=None)
+
+        src, dst = planes(arena.device_ptr, n), planes(pool.data_ptr(), batch * k + 1)
+        src_rows = torch.zeros((1, batch, k), dtype=torch.int32, device=gpu)
+        dst_rows = torch.arange(1, batch * k + 1, dtype=torch.int32, device=gpu).view(1, batch, k)
+        counts = torch.zeros((1, batch), dtype=torch.int32, device=gpu)
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            move_kv(src, src_rows, dst, dst_rows, counts)
+        torch.cuda.current_stream().wait_stream(side)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            move_kv(src, src_rows, dst, dst_rows, counts)
+        for _ in range(4):
+            host = rng.integers(0, 256, (2, n, row_bytes), dtype=np.uint8)
+            torch.cuda.synchronize()
+            arena.host.copy_(torch.from_numpy(host.reshape(-1)))
+            rows, count = rng.integers(0, n, (batch, k)), rng.integers(0, k + 1, batch)
+            src_rows.copy_(torch.tensor(rows).view(1, batch, k))
+            counts.copy_(torch.tensor(count).view(1, batch))
+            pool.zero_()
+            graph.replay()
+            want = np.zeros((2, batch, k, row_bytes), np.uint8)
+            for b in range(batch):
+                want[:, b, :count[b]] = host[:, rows[b, :count[b]]]
+            assert np.array_equal(pool[:, 1:].cpu().numpy().reshape(want.shape), want)
+        torch.cuda.synchronize()
+    finally:
+        arena.close()
