@@ -525,25 +525,31 @@ __global__ __launch_bounds__(kThreads) void hisparse_swap_kernel(const HsArgs a)
 // many (unequal misses, and the link serves the XCDs unequally once requests
 // queue up). kCopyGroups workgroups of one 16-byte load per lane keep 192 KiB
 // in flight, the amount that reached the link's rate for the row moves (57 GB/s).
-// A miss to copy is an output entry -2 - slot (the swap's step 6): the slot
-// names its token, which names its host row, and its device row, which
-// replaces the entry. So the launches share no memory beyond the caller's own
-// state, in a graph as well. A wave takes a.span entries at a time; the four
-// reads that lead to their host rows run up to three spans ahead of the
-// copies. @@
+// A miss to copy is an output entry -2 - (miss rank << kSlotBits | slot), left
+// by the swap's step 6. The slot names its token, which names its host row,
+// and its device row, which replaces the entry; so the launches share no memory
+// beyond the caller's own, in a graph as well. Every workgroup reads all
+// entries and takes the misses whose rank plus batch row is its own modulo
+// the grid: a row's misses are dealt round robin, whatever block-sized runs
+// they come in, and no workgroup acts on an entry that another one replaces.
+// (Entries dealt in runs of 16 left some waves far more rows than others: 511
+// against 477 us for 25.5 MB.) 24 rows took 569 us when each row's workgroup
+// copied its own misses and 476 us so; one row of 512 lanes and 512 B rows,
+// 89 and 21 us.
 constexpr uint32_t kCopyGroups = 48;
 constexpr int kCopyThreads = 256;
 constexpr int kScan = 16;                            // entries in flight per thread
-constexpr uint32_t kRound = kCopyThreads * kScan;        // entries per round of the scan
-constexpr uint32_t kCopyBatch = 2048;                // misses whose copy pieces are counted in 32 bits (checked by the host)
+constexpr uint32_t kRound = kCopyThreads * kScan;    // entries per round of the scan
+constexpr uint32_t kCopyBatch = 2048;                // misses whose copy pieces fit 32 bits (checked by the host)
 // The list is copied once it holds more than this, so that a large batch's copies
 // start early in its scan: 128 rows of 2048 lanes 2,340 us, 2,411 with 2,048 (24 rows: 493 both).
 constexpr uint32_t kFlush = 512;
 constexpr uint32_t kListed = kFlush + kRound;        // misses listed at most
 
 template <typename V>
-__global__ __launch_bounds__(kCopyThreads) void copy_missed_rows(const HsArgs a, int64_t first_row, uint32_t entries,
-                                                             FastDiv width_div, FastDiv group_div) {
+__global__ __launch_bounds__(kCopyThreads) void copy_missed_rows(const HsArgs a, int64_t first_row,
+                                                                 uint32_t entries, FastDiv width_div,
+                                                                 FastDiv group_div) {
     constexpr int64_t kWidth = sizeof(V);
     constexpr int kResolve = 4;            // misses resolved per thread at a time
     __shared__ uint32_t host_of[kListed];  // entry, then host row (all ones: none)

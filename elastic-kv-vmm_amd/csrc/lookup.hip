@@ -1036,7 +1036,8 @@ __global__ __launch_bounds__(kThreads) void resolve_blocks_kernel(const LookupAr
         i32x4 piece[kPieces];
 #pragma unroll
         for (int i = 0; i < kPieces; ++i) {   // unconditional: the row's first piece stands in
-            piece[i] = reinterpret_cast<const i32x4*>(element<true>(table, 1, whole ? static_cast<uint32_t>(first) : 0u))[i];
+            const TableT* at = element<true>(table, 1, whole ? static_cast<uint32_t>(first) : 0u);
+            piece[i] = reinterpret_cast<const i32x4*>(at)[i];
         }
         const int64_t base = std::is_same_v<TableT, int16_t> ? index_value(a.slot_base, base_read) : 0;
         TableT held[kRun];
@@ -1060,7 +1061,8 @@ __global__ __launch_bounds__(kThreads) void resolve_blocks_kernel(const LookupAr
             stream_store(i32x4{slot[4], slot[5], slot[6], slot[7]}, to + 1);
         }
         if constexpr (kCompact) {
-            // Rank of the thread's first miss: misses of lower lanes of its wave (four bit planes), then of lower waves.
+            // Rank of the thread's first miss: misses of lower lanes of its
+            // wave (four bit planes), then of lower waves.
             const uint32_t count = __popc(miss);
             uint32_t below = 0, wave_total = 0;
 #pragma unroll
@@ -2036,7 +2038,8 @@ int resolve_resident(const ekv_tensor* topk_p, const ekv_tensor* table_p, const 
     // Two levels have no summary to spare; direct for as many rows as were measured shorter
     // (us): 4 x 2048 5.18 -> 3.63, 256 x 2048 9.19 -> 7.47, 512 x 2048 13.16 -> 11.96.
     const bool two_levels = mapping != nullptr && a.map_len > 0 && a.map_s == 1 && count * layers <= kMappedDirectRows;
-    a.direct = dense && a.table_rows > 0 && a.table_cols > 0 && width <= kChunkLanes && (one_level || two_levels) ? 1 : 0;
+    const bool has_entries = a.table_rows > 0 && a.table_cols > 0;
+    a.direct = dense && has_entries && width <= kChunkLanes && (one_level || two_levels) ? 1 : 0;
     if (check_only()) {
         return 0;
     }
@@ -2093,8 +2096,8 @@ __global__ __launch_bounds__(kThreads) void residency_bits_kernel(const TableT* 
     }
 }
 
-// Summary rows (shift > 0) of any layout (strided entries, rows that do not
-// come in whole 16-byte pieces): one wave per summary word covers the 32 << shift
+// Summary rows (shift > 0) of any layout (strided entries, misaligned rows):
+// one wave per summary word covers the 32 << shift
 // positions of its 32 groups, 64 consecutive entries per iteration, each lane
 // OR-ing the bit of its entry's group; the wave's bits are OR-reduced and
 // lane 0 writes the word.
@@ -2212,8 +2215,8 @@ __global__ __launch_bounds__(kThreads) void residency_pieces_kernel(
     const uint32_t in_seg = lane & ((1u << seg_log2) - 1);
     const uint32_t words_per_load = 64u >> seg_log2;
     const uint32_t per_lane = 1u << per_lane_log2;
-    const uint32_t sets = per_lane < kSummaryLoads ? kSummaryLoads >> per_lane_log2 : 1u;   // loads of a word, times sets
-    const uint32_t steps = sets << per_lane_log2;   // a multiple of kSummaryLoads
+    const uint32_t sets = per_lane < kSummaryLoads ? kSummaryLoads >> per_lane_log2 : 1u;
+    const uint32_t steps = sets << per_lane_log2;   // loads of a word, times sets: a multiple of kSummaryLoads
     const uint32_t wave = blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6);
     const uint32_t stride = gridDim.x * (kThreads / 64) * words_per_load * sets;
     // Groups of at least a piece: 2^span_log2 consecutive lanes hold one group, over 2^fold_log2 loads.
@@ -2327,7 +2330,7 @@ void launch_residency_bits(const ekv_tensor& table, const ekv_tensor& bits, int 
     const int64_t words_per_row = summary_words(cols, shift);
     const int64_t total = layers * rows * words_per_row;
     constexpr int64_t kE = 16 / static_cast<int64_t>(sizeof(TableT));
-    const auto piece_aligned = [](int64_t elements) { return (elements * static_cast<int64_t>(sizeof(TableT))) % 16 == 0; };
+    const auto piece_aligned = [](int64_t elements) { return elements * int64_t{sizeof(TableT)} % 16 == 0; };
     const bool pieces = table.stride[d + 1] == 1 && (reinterpret_cast<uintptr_t>(table.data) & 15) == 0 &&
                         piece_aligned(table.stride[d]) && (!layered || piece_aligned(t_sl)) &&
                         total < (int64_t{1} << 31);
