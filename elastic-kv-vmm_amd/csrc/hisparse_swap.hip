@@ -47,6 +47,7 @@
 #include "ekv_device.h"
 #include "ekv_fastdiv.h"
 #include "ekv_tensor_util.h"
+#include "ekv_token.h"
 #include "ekv_vec.h"
 #include "ekv_wave.h"
 
@@ -295,10 +296,13 @@ __global__ __launch_bounds__(kThreads) void hisparse_swap_kernel(const HsArgs a)
         for (int k = 0; k < kLanesPerThread; ++k) {
             const int64_t o = threadIdx.x + k * kThreads;
             const uint32_t kb = a.block_div.div(static_cast<uint32_t>(o < W ? o : 0));
-            const int64_t t = block[k] * a.block_size + (static_cast<uint32_t>(o < W ? o : 0) - kb * a.block_size);
+            int64_t t;
+            const bool named = token_position(block[k], a.block_size,
+                                              static_cast<uint32_t>(o < W ? o : 0) - kb * a.block_size, a.T,
+                                              length < a.T ? length : a.T, t);
             uint8_t kind = kInvalid;
             int32_t aux = -1;
-            if (o < W && block[k] >= 0 && t < length && t < a.T) {
+            if (o < W && named) {
                 if (t == length - 1) {
                     kind = kNewest;
                 } else {

@@ -46,6 +46,7 @@
 #include "ekv_device.h"
 #include "ekv_fastdiv.h"
 #include "ekv_tensor_util.h"
+#include "ekv_token.h"
 #include "ekv_wave.h"
 
 #include <algorithm>
@@ -281,8 +282,9 @@ template <typename TopkT>
 __device__ __forceinline__ uint32_t lane_position(const LookupArgs& a, uint32_t o, TopkT block, int64_t bound,
                                                   bool table_ok, bool& valid) {
     const uint32_t offset = o - a.block_div.div(o) * a.block_size;
-    const int64_t p = static_cast<int64_t>(block) * a.block_size + offset;
-    valid = o < a.width && block >= 0 && p < bound && table_ok;
+    int64_t p;
+    const bool inside = token_position(block, a.block_size, offset, a.table_cols, bound, p);
+    valid = o < a.width && inside && table_ok;
     return valid ? static_cast<uint32_t>(p) : 0u;
 }
 
@@ -1028,8 +1030,8 @@ __global__ __launch_bounds__(kThreads) void resolve_blocks_kernel(const LookupAr
         }
         const bool live_run = o < width;   // runs are whole: the width is a multiple of the block size
         const uint32_t offset = o - a.block_div.div(o) * a.block_size;
-        const int64_t first = static_cast<int64_t>(block) * a.block_size + offset;
-        const bool any = live_run && block >= 0 && first < bound;
+        int64_t first;
+        const bool any = token_position(block, a.block_size, offset, a.table_cols, bound, first) && live_run;
         const bool whole = any && first + kRun <= a.table_cols;
         // Lanes of the run that are valid: a prefix.
         const int32_t valid = any ? static_cast<int32_t>(bound - first < kRun ? bound - first : kRun) : 0;

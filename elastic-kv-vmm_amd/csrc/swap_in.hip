@@ -58,6 +58,7 @@
 #include "ekv_fastdiv.h"
 #include "ekv_step.h"
 #include "ekv_tensor_util.h"
+#include "ekv_token.h"
 #include "ekv_wave.h"
 
 #include <algorithm>
@@ -437,14 +438,17 @@ __global__ __launch_bounds__(kThreads) void swap_in_kernel(const SwapArgs a) {
     int32_t miss_lane[kLaneRegs];   // lane of this thread's k-th entry (kLookup: its k-th lane)
     bool valid_lane[kLaneRegs];     // kLookup
     int64_t lane_token[kLaneRegs];
-    // The token of an entry: its block id times the block size, and the lane's place in the block.
+    // The token of an entry: its block id times the block size, and the lane's place in the block; outside
+    // [0, table_cols) when it names none.
     const auto token_at = [&](int k, int32_t lane) {
         const int32_t high = a.topk64 ? block_high[k] : block_low[k] >> 31;
         int64_t token = static_cast<int64_t>(static_cast<uint64_t>(static_cast<uint32_t>(high)) << 32 |
                                              static_cast<uint32_t>(block_low[k]));
         if (a.block_size != 1) {   // uniform
-            token = token * a.block_size +
-                    (static_cast<uint32_t>(lane) - a.block_div.div(static_cast<uint32_t>(lane)) * a.block_size);
+            const uint32_t offset =
+                static_cast<uint32_t>(lane) - a.block_div.div(static_cast<uint32_t>(lane)) * a.block_size;
+            int64_t position;
+            token = token_position(token, a.block_size, offset, a.table_cols, a.table_cols, position) ? position : -1;
         }
         return token;
     };
@@ -455,8 +459,7 @@ __global__ __launch_bounds__(kThreads) void swap_in_kernel(const SwapArgs a) {
         for (int k = 0; k < kLaneRegs; ++k) {
             miss_lane[k] = static_cast<int32_t>(threadIdx.x) + k * kThreads;
             lane_token[k] = token_at(k, miss_lane[k]);
-            const int32_t high = a.topk64 ? block_high[k] : block_low[k];
-            valid_lane[k] = miss_lane[k] < W && high >= 0 && lane_token[k] < bound;   // a block id of at least 0
+            valid_lane[k] = miss_lane[k] < W && lane_token[k] >= 0 && lane_token[k] < bound;
             at[k] = valid_lane[k] ? static_cast<uint32_t>(lane_token[k]) : 0u;
         }
         if (a.table16) {   // uniform

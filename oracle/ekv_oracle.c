@@ -46,8 +46,9 @@ void oracle_resolve_resident(int64_t L, int64_t B, int64_t K, int64_t bs, const 
             int32_t found = 0;
             for (int64_t o = 0; o < W; ++o) {
                 const int64_t block = topk[(l * B + row) * K + o / bs];
-                const int64_t pos = block * bs + o % bs;
-                const int valid = block >= 0 && pos < length;
+                /* A block starts at or past its own id: one not below T names no position (and could overflow). */
+                const int64_t pos = block >= 0 && block < T ? block * bs + o % bs : T;
+                const int valid = pos < length;
                 int in_bounds = valid && req >= 0 && req < R && pos < T;
                 int64_t value = -1;
                 if (in_bounds) {

@@ -68,6 +68,7 @@ def resolve_resident(topk, table, mapping, rows, lengths, selected, block_size, 
         layer_table = table[layer] if table.ndim == 3 else table
         R, T = layer_table.shape
         blocks = topk[layer, sel]                                            # [S, K]
+        blocks = np.where((blocks >= 0) & (blocks < T), blocks, -1)          # others name no position, and may overflow
         positions = (blocks[:, :, None] * block_size + np.arange(block_size)).reshape(len(sel), width)
         valid = (positions >= 0) & (positions < lengths[sel, None])
         req = rows[sel]

@@ -203,6 +203,61 @@ def test_fast_division_is_exact_below_2_pow_31(tmp_path):
     assert subprocess.run([str(binary)], capture_output=True, text=True).stdout.strip() == "ok"
 
 
+TOKEN_TEST = r"""
+#include "ekv_token.h"
+#include <cstdint>
+#include <cstdio>
+template <typename Id>
+int check(Id id, uint32_t size, uint32_t offset, int64_t cols, int64_t bound) {
+    const __int128 exact = static_cast<__int128>(id) * size + offset;
+    int64_t position = -9;
+    const bool got = ekv::token_position(id, size, offset, cols, bound, position);
+    const bool want = id >= 0 && exact < bound;
+    if (got != want || (got && position != exact)) {
+        std::printf("fail id %lld size %u offset %u cols %lld bound %lld\n", static_cast<long long>(id), size, offset,
+                    static_cast<long long>(cols), static_cast<long long>(bound));
+        return 1;
+    }
+    return 0;
+}
+int main() {
+    const int64_t ids[] = {0, 1, 2, 99, 499, 500, 999, 1000, 1001, INT32_MAX, int64_t{1} << 31, int64_t{1} << 32,
+                           int64_t{1} << 61, (int64_t{1} << 61) + 3, int64_t{1} << 62, (int64_t{1} << 62) + 1,
+                           INT64_MAX, INT64_MAX - 1, INT64_MAX / 3 + 1, -1, -2, INT32_MIN, INT64_MIN, INT64_MIN + 1};
+    const uint32_t sizes[] = {1, 2, 3, 4, 8, 16, 128, 2048, 0x7fffffffu};
+    const int64_t widths[] = {1, 100, 1000, 0x7fffffff};
+    int bad = 0;
+    for (const int64_t id : ids) {
+        for (const uint32_t size : sizes) {
+            const uint32_t offsets[] = {0, size / 2, size - 1};
+            for (const uint32_t offset : offsets) {
+                for (const int64_t cols : widths) {
+                    const int64_t bounds[] = {cols, cols / 2, 0, -5, INT64_MIN};
+                    for (const int64_t bound : bounds) {
+                        bad += check<int64_t>(id, size, offset, cols, bound);
+                        bad += check<int32_t>(static_cast<int32_t>(id), size, offset, cols, bound);
+                    }
+                }
+            }
+        }
+    }
+    std::puts(bad == 0 ? "ok" : "bad");
+    return bad != 0;
+}
+"""
+
+
+def test_token_positions_never_wrap(tmp_path):
+    # The kernels' block id -> position step against 128-bit arithmetic, under UBSan.
+    source = tmp_path / "token.cpp"
+    source.write_text(TOKEN_TEST)
+    binary = tmp_path / "token"
+    subprocess.run(["g++", "-O2", "-std=c++17", "-fsanitize=undefined", "-fno-sanitize-recover=undefined", "-I",
+                    str(ROOT / "elastic-kv-vmm_amd" / "csrc"), str(source), "-o", str(binary)], check=True)
+    result = subprocess.run([str(binary)], capture_output=True, text=True)
+    assert result.stdout.strip() == "ok", result.stdout + result.stderr
+
+
 def test_library_fingerprint_matches_the_sources(lib):
     from elastic_kv._source_hash import source_hash
 

@@ -776,3 +776,19 @@ def test_torch_cpu_path_matches_the_numpy_oracle():
         pool = planes.numpy().reshape(-1)
         expect = ref.gather_kv(pool, 2 * 41 * 8, 41 * 8, 8, 8, 41, flat.numpy().reshape(1, 1, -1), 2)
         assert np.array_equal(rows_out.numpy().reshape(-1), expect.reshape(-1))
+
+
+@pytest.mark.parametrize("block_size", [1, 4, 8])
+def test_block_ids_past_64_bits_name_no_token(coracle, block_size):
+    # Products of these ids with the block size wrap to small or negative positions.
+    big = np.iinfo(np.int64).max
+    topk = np.array([[[big, 1 << 62, (1 << 61) + 3, -big - 1, 1, min(big, big // block_size + 1)]]])
+    table = np.arange(1, 41).reshape(1, 40)
+    width = topk.shape[-1] * block_size
+    want = np.full((1, 1, width), -1, np.int32)
+    want[0, 0, 4 * block_size:5 * block_size] = table[0, block_size:2 * block_size]
+    for resolve in (coracle.resolve_resident, ref.resolve_resident):
+        got, _, counts = resolve(topk, table, None, [0], [1 << 40], [0], block_size,
+                                 np.full((1, 1, width), -77, np.int32), with_misses=True)
+        assert np.array_equal(got, want)
+        assert counts[0, 0] == 0
