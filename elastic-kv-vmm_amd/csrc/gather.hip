@@ -415,25 +415,40 @@ void launch_vw(const EngineArgs& a, int vw, hipStream_t stream) {
 // serves the 8 XCDs unequally: with the whole job in flight (one workgroup
 // per tile, as above) two XCDs finished at half the time of the slowest, and
 // a few of them ran the rest of the job alone. kHostGroups workgroups with
-// one 16-byte load per lane keep 192 KiB in flight. 21,337 moves of K and V
-// rows of 512 B (22 MB), the same in each of three processes: 57.0 GB/s
-// against 51.9 in flight at once (24 workgroups 55.1, 32 56.6, 64 54-57.5, 96 54.4,
-// 128 56.3; two loads per lane 46-53 for 32). The copy engine reaches 56.4.
+// one 16-byte load per lane keep 192 KiB in flight. 19,661 moves of K and V
+// rows of 512 B (20 MB), us: tile kernel 390, 48 workgroups 358, 96 373, 128
+// 363, 192 362, 256 373. The copy engine reaches 56.4 GB/s, this 56.2.
 // The moves are dealt out evenly: every workgroup adds up the counts of
 // kHostRows (layer, batch) rows at a time in LDS, and the vectors of all their
 // moves, in list order, are strided over the grid, so rows of unequal counts
 // and the unused tails of the lists cost nothing. The list entries of an
 // iteration are read while the load of the one before is in flight.
+// Beside the driver's unmaps the few requests cost the move itself (each waits
+// for the TLB flushes: 6.9 GB took 168-172 ms, 132-134 through the tile kernel),
+// but the unmaps run faster beside them (341-357 against 451-459 us a chunk), and they
+// are what the elastic step waits for: 348-370 ms a step with 774 chunks remapped
+// against 444-453, with 155 chunks 128-131 against 159-162.
 constexpr uint32_t kHostGroups = 48;
 constexpr uint32_t kHostRowsPerThread = 4;
 constexpr uint32_t kHostRows = kThreads * kHostRowsPerThread;
-// Lists that could move no more than this fit in flight whole, and the tile
-// kernel's shorter way to its first load wins: 100 rows of 1 KiB from a list
-// of 256 take 9.1 us there and 9.9 us here.
-constexpr int64_t kHostMoveBytes = int64_t{512} << 10;
+// The lists that take it: at least kHostMoveBytes could move (the whole lists), 16-byte
+// vectors and rows of at least kHostRowBytes. The tile kernel's way to its
+// first load is shorter (no prefix over the counts), short jobs fit in flight whole, and short rows and
+// narrow vectors need more requests in flight than this keeps.
+// Measured (us, tile kernel / this; 40 % of the lists used, every row another one):
+//   8 x 256 x 512 B (2 MiB)     20.1 /  25.5     48 x 256 x 256 B (6 MiB)    57.2 /  48.8
+//   16 x 256 x 512 B (4 MiB)    38.3 / 34-46     48 x 1024 x 128 B          124 / 133
+//   24 x 256 x 512 B (6 MiB)    57.2 /  49.0     128 x 2048 x 64 B          634 / 638
+//   8 x 1024 x 512 B (8 MiB)    75.3 /  70.6     48 x 1024 x 516 B (4 B)    451 / 527
+//   48 x 256 x 512 B (12 MiB)    109 /  92.4     48 x 1024 x 520 B (8 B)    455 / 485
+//   4 x 128 x 8 KiB (8 MiB)     78.3 /  62.9     4 layers 128 x 2048 x 512 B  7,800 / 7,540
+// Lists of which 2 % are used take 0.7-1.5 us longer here up to 24 MiB (24 x 256: 6.1 / 6.8) and the same past it; host rows
+// that the call itself reads a dozen times come from the memory-side cache, where more in flight is 4-11 % faster.
+constexpr int64_t kHostMoveBytes = int64_t{6} << 20;
+constexpr int64_t kHostRowBytes = 256;
 
-template <int VW>
 __global__ __launch_bounds__(kThreads) void move_host_rows(const EngineArgs a, uint32_t batch_rows, FastDiv move_div) {
+    constexpr int VW = 16;
     using V = typename Vec<VW>::type;
     constexpr int kWaves = kThreads / 64;
     __shared__ uint32_t first_move[kHostRows];   // moves of the rows below each row of this batch of rows
@@ -544,19 +559,10 @@ bool in_host_memory(const void* address) {
     return attributes.type == hipMemoryTypeHost;
 }
 
-template <int VW>
-void launch_host_move(EngineArgs a, uint32_t batch_rows, hipStream_t stream) {
-    a.vecs_per_row = static_cast<uint32_t>(a.row_bytes / VW);
-    const FastDiv move_div(static_cast<uint32_t>(a.KV * a.vecs_per_row));
-    // The bytes in flight are what counts: narrower vectors take more workgroups.
-    const uint32_t groups = kHostGroups * (16 / VW);
-    move_host_rows<VW><<<dim3(groups), dim3(kThreads), 0, stream>>>(a, batch_rows, move_div);
-}
-
 // Moves from host memory through move_host_rows; false when the job does not fit its 32-bit counts.
-bool host_move(EngineArgs a, int64_t rows, int vw, hipStream_t stream) {
+bool host_move(EngineArgs a, int64_t rows, hipStream_t stream) {
     // Vectors per (layer, batch) row at most; a batch of rows stays below 2^31 with room for the last stride.
-    const int64_t per_row = a.K * a.KV * (a.row_bytes / vw);
+    const int64_t per_row = a.K * a.KV * (a.row_bytes / 16);
     const int64_t limit = (int64_t{1} << 30) / per_row;
     if (limit < 1 || rows >= (int64_t{1} << 31)) {
         return false;
@@ -564,13 +570,9 @@ bool host_move(EngineArgs a, int64_t rows, int vw, hipStream_t stream) {
     const uint32_t batch_rows = static_cast<uint32_t>(std::min<int64_t>(limit, kHostRows));
     a.units = rows;
     a.div_b = FastDiv(static_cast<uint32_t>(a.B));
-    switch (vw) {
-        case 16: launch_host_move<16>(a, batch_rows, stream); break;
-        case 8: launch_host_move<8>(a, batch_rows, stream); break;
-        case 4: launch_host_move<4>(a, batch_rows, stream); break;
-        case 2: launch_host_move<2>(a, batch_rows, stream); break;
-        default: launch_host_move<1>(a, batch_rows, stream); break;
-    }
+    a.vecs_per_row = static_cast<uint32_t>(a.row_bytes / 16);
+    const FastDiv move_div(static_cast<uint32_t>(a.KV * a.vecs_per_row));
+    move_host_rows<<<dim3(kHostGroups), dim3(kThreads), 0, stream>>>(a, batch_rows, move_div);
     return true;
 }
 
@@ -826,8 +828,9 @@ int move_kv(const ekv_planes* src, const ekv_tensor* src_rows_p, const ekv_plane
         return 0;
     }
     const auto s = static_cast<hipStream_t>(stream);
-    const bool linked = units * a.row_bytes > kHostMoveBytes && in_host_memory(src->base);
-    if (!linked || !host_move(a, L * list_rows, vw, s)) {
+    const bool linked = vw == 16 && a.row_bytes >= kHostRowBytes && units * a.row_bytes >= kHostMoveBytes &&
+                        in_host_memory(src->base);
+    if (!linked || !host_move(a, L * list_rows, s)) {
         launch_vw<KvMove>(a, vw, s);
     }
     check_hip(hipGetLastError(), "launch KV move");

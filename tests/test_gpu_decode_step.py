@@ -310,3 +310,52 @@ def test_one_launch_lookup_and_swap_equals_the_kernels(gpu, host, table_dtype, s
             outputs.append([slots.cpu(), out.cpu()] + [t.cpu() for t in kept])
         for a, z in zip(*outputs):
             assert torch.equal(a, z), step
+
+
+def test_promotion_of_a_selection_past_the_tile_kernel(gpu):
+    # Lists of 7 MiB of pinned host rows: the step's promotion walks the selection in the host-row kernel. Permuted,
+    # stray and missing entries against the stages, whose move reads every row's count.
+    layers, rows_n, context, hot, lanes, row = 2, 14, 1400, 512, 256, 512
+    plane = rows_n * context * row
+    arena = HostArena(layers * 2 * plane)
+    try:
+        arena.host.copy_(torch.randint(0, 256, (arena.nbytes,), dtype=torch.uint8))
+        host = KVPlanes(base=arena.device_ptr, device=0, layers=layers, kv=2, layer_stride=2 * plane, kv_stride=plane,
+                        row_stride=row, row_bytes=row, rows=rows_n * context, owner=arena)
+        host_table = torch.arange(rows_n * context, dtype=torch.int32, device=gpu).reshape(rows_n, context)
+        rng = np.random.default_rng(11)
+        buffers = [HotBuffers(layers, rows_n, context, hot, gpu, table_dtype=torch.int16, bits_shift=6) for _ in range(2)]
+        pools = [torch.zeros((layers, 2, 1 + rows_n * hot, row), dtype=torch.uint8, device=gpu) for _ in range(2)]
+        rows = torch.tensor(rng.permutation(rows_n), device=gpu)
+        lengths = torch.tensor(rng.integers(context // 2, context + 5, rows_n), dtype=torch.int32, device=gpu)
+        for step in range(3):
+            picks = [np.arange(rows_n), np.concatenate([rng.permutation(rows_n), [-1, rows_n]]), rng.permutation(rows_n)[:9]][step]
+            selected = torch.tensor(rng.permutation(picks) if step == 1 else picks, device=gpu)
+            topk = torch.tensor(np.stack([rng.permutation(context)[:lanes] for _ in range(layers * rows_n)]).reshape(
+                layers, rows_n, lanes), dtype=torch.int32, device=gpu)
+            outputs = []
+            for staged, b, pool in zip((True, False), buffers, pools):
+                size = (1 + rows_n * hot) * row
+                planes = KVPlanes(base=pool.data_ptr(), device=0, layers=layers, kv=2, layer_stride=2 * size,
+                                  kv_stride=size, row_stride=row, row_bytes=row, rows=1 + rows_n * hot, owner=pool)
+                slots = torch.full((layers, rows_n, lanes), -9, dtype=torch.int32, device=gpu)
+                out = torch.empty((rows_n, layers, 2, lanes, row), dtype=torch.uint8, device=gpu)
+                if staged:
+                    misses, counts = torch.empty_like(slots), torch.zeros((layers, rows_n), dtype=torch.int32, device=gpu)
+                    resolve_resident(topk, b.table, None, rows, lengths, selected, slots, 1, misses=misses,
+                                     miss_count=counts, resident_bits=b.bits, bits_shift=6, slot_base=b.slot_base)
+                    src, dst = torch.empty_like(slots), torch.empty_like(slots)
+                    swap_in(topk, 1, rows, selected, slots, misses, counts, b, host_table, src, dst)
+                    move_kv(host, src, planes, dst, counts)
+                    gather_kv(planes, slots, out)
+                else:
+                    workspace = torch.full((decode_step_workspace(layers, rows_n, lanes),), 0x7f, dtype=torch.uint8,
+                                           device=gpu)
+                    decode_step(topk, rows, lengths, b, host_table, host, planes, slots, out, selected=selected,
+                                workspace=workspace)
+                outputs.append([t.cpu() for t in (slots, out, pool, b.table, b.bits, b.slot_token, b.stamps)])
+            for a, z in zip(*outputs):
+                assert torch.equal(a, z), step
+    finally:
+        torch.cuda.synchronize()
+        arena.close()

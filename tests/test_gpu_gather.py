@@ -98,8 +98,12 @@ def test_gather_kv_rejects_bad_shapes(gpu):
     (512, 2, 2, 700, 6),       # more (layer, batch) rows than one batch of rows holds
     (1040, 1, 1, 3, 340),      # a row that is no power of two of vectors
     (200, 2, 1, 5, 333), (36, 1, 2, 3, 3000), (6, 2, 1, 20, 2500), (3, 2, 1, 20, 5000),    # narrower vectors
-    (512, 2, 1, 8, 64), (512, 2, 1, 8, 65),      # the largest list of the tile kernel, the smallest past it
-    (16, 2, 1, 1, 1)])
+    (512, 2, 1, 8, 64), (512, 2, 1, 8, 65),
+    (16, 2, 1, 1, 1),
+    (512, 2, 1, 6, 1023), (512, 2, 1, 6, 1024),  # the largest list of the tile kernel, the smallest past it
+    (1040, 1, 1, 3, 2100),
+    (256, 2, 1, 24, 513), (240, 2, 1, 24, 600),  # the shortest row past the tile kernel, a shorter one
+    (520, 2, 1, 12, 520)])                       # 8-byte vectors: the tile kernel
 def test_move_from_host_memory_matches_oracle(gpu, row_bytes, kv, layers, batch, k):
     from adaptive_sparse.host_arena import HostArena
     from adaptive_sparse.kv_pool import KVPlanes
@@ -142,7 +146,7 @@ def test_host_moves_replay_from_a_graph(gpu):
     from adaptive_sparse.swap_in import move_kv
 
     rng = np.random.default_rng(7)
-    batch, k, n, row_bytes = 8, 200, 900, 512
+    batch, k, n, row_bytes = 8, 800, 900, 512
     arena = HostArena(2 * n * row_bytes)
     try:
         pool = torch.zeros((2, batch * k + 1, row_bytes), dtype=torch.uint8, device=gpu)
