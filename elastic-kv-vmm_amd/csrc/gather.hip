@@ -18,6 +18,9 @@
 //   KvGather / KvScatter  - planes (layer, kv) x slot rows <-> dense rows
 //                           (l, b, kv, k); slots outside [zero_below, rows)
 //                           give zero rows (gather) or are skipped (scatter).
+//   KvMove / KvMoveSelected - rows of one plane set -> rows of another, by lists
+//                           per (layer, batch) row, of every batch row or of
+//                           those that a selection names.
 //   RowsDirect / RowsIndirect - experimental/sparse_read.py:11-30 semantics
 //                           over one flat payload tensor.
 #include "../../include/ekv_kernels.h"
@@ -52,7 +55,8 @@ constexpr size_t kGatherLdsReserve = 49152;
 constexpr int64_t kXcdCount = 8;
 
 enum Mode : int {
-    KvGather = 0, KvScatter = 1, RowsDirect = 2, RowsIndirect = 3, KvGather64 = 4, KvScatter64 = 5, KvMove = 6
+    KvGather = 0, KvScatter = 1, RowsDirect = 2, RowsIndirect = 3, KvGather64 = 4, KvScatter64 = 5, KvMove = 6,
+    KvMoveSelected = 7
 };
 
 constexpr bool is_kv_mode(int m) { return m == KvGather || m == KvScatter || m == KvGather64 || m == KvScatter64; }
@@ -97,8 +101,6 @@ struct EngineArgs {
     int64_t mdr_l, mdr_b, mdr_i;
     const int32_t* move_counts;
     int64_t mc_l, mc_b;
-    IndexRef move_selected;  // data null: every batch row; else entry j of B stands for batch row move_selected[j]
-    int64_t move_batch;      // batch rows
 
     // Rows modes: unit u = b * S + s.
     const char* raw;
@@ -114,6 +116,18 @@ struct EngineArgs {
     int64_t out_sb, out_ss;  // output strides in bytes
     int64_t S;
 };
+
+// A move over a selection of batch rows: arguments and a mode of its own. As a part of
+// EngineArgs and of KvMove the selection cost the moves without one 0.25 us
+// (8 x 64 device moves replayed from a graph 3.11 -> 3.35 us), and reading the entries before the count
+// cost lists with unused tails more (20 x 128 x 2048 entries of 64 B rows, none used: 71 -> 89 us).
+struct MoveArgs : EngineArgs {
+    IndexRef move_selected;  // data null: every batch row; else entry j of B stands for batch row move_selected[j]
+    int64_t move_batch;      // batch rows
+};
+
+template <int M>
+using ArgsOf = std::conditional_t<M == KvMoveSelected, MoveArgs, EngineArgs>;
 
 // (source offset, destination offset) in bytes of one row; -1 source means a
 // zero row, -1 destination means the row is not written.
@@ -139,7 +153,7 @@ __device__ __forceinline__ void split_unit(const EngineArgs& a, int64_t u, int64
 }
 
 // Batch row of list row j of a move, or -1 when a selection names none there.
-__device__ __forceinline__ int64_t move_row(const EngineArgs& a, int64_t j) {
+__device__ __forceinline__ int64_t move_row(const MoveArgs& a, int64_t j) {
     if (a.move_selected.data == nullptr) {   // uniform
         return j;
     }
@@ -148,15 +162,31 @@ __device__ __forceinline__ int64_t move_row(const EngineArgs& a, int64_t j) {
 }
 
 template <int M>
-__device__ __forceinline__ void locate(const EngineArgs& a, int64_t u, int64_t& src, int64_t& dst) {
+__device__ __forceinline__ void locate(const ArgsOf<M>& a, int64_t u, int64_t& src, int64_t& dst) {
+    const auto place = [&](int64_t l, int64_t kv, int64_t from, int64_t to) {
+        if (from >= 0 && from < a.ms_rows && to >= a.zero_below && to < a.pool_rows) {
+            src = l * a.ms_layer_stride + kv * a.ms_kv_stride + from * a.ms_row_stride;
+            dst = l * a.layer_stride + kv * a.kv_stride + to * a.row_stride;
+        }
+    };
     if constexpr (M == KvMove) {
+        int64_t l, b, kv, k;
+        split_unit(a, u, l, b, kv, k);
+        src = -1;
+        dst = -1;
+        if (k < a.move_counts[l * a.mc_l + b * a.mc_b]) {
+            const int64_t from = a.move_src_rows[l * a.msr_l + b * a.msr_b + k * a.msr_i];
+            const int64_t to = a.move_dst_rows[l * a.mdr_l + b * a.mdr_b + k * a.mdr_i];
+            place(l, kv, from, to);
+        }
+    } else if constexpr (M == KvMoveSelected) {
+        // The selection entry, and the count and list entries of the row it
+        // names on the guess of the identity selection, are read at once: one
+        // memory level before the row itself instead of three (entries at or past the count are read but not used).
         int64_t l, j, kv, k;
         split_unit(a, u, l, j, kv, k);
         src = -1;
         dst = -1;
-        // The selection entry, and the count and list entries of the row it
-        // names on the guess of the identity selection, are read at once: one
-        // memory level before the row itself instead of three (entries at or past the count are read but not used).
         const int64_t guess = j < a.move_batch ? j : 0;
         int32_t count = a.move_counts[l * a.mc_l + guess * a.mc_b];
         int64_t from = a.move_src_rows[l * a.msr_l + guess * a.msr_b + k * a.msr_i];
@@ -168,10 +198,7 @@ __device__ __forceinline__ void locate(const EngineArgs& a, int64_t u, int64_t& 
             to = a.move_dst_rows[l * a.mdr_l + b * a.mdr_b + k * a.mdr_i];
         }
         if (b >= 0 && k < count) {
-            if (from >= 0 && from < a.ms_rows && to >= a.zero_below && to < a.pool_rows) {
-                src = l * a.ms_layer_stride + kv * a.ms_kv_stride + from * a.ms_row_stride;
-                dst = l * a.layer_stride + kv * a.kv_stride + to * a.row_stride;
-            }
+            place(l, kv, from, to);
         }
     } else if constexpr (is_kv_mode(M)) {
         using SlotT = typename std::conditional<(M == KvGather64 || M == KvScatter64), int64_t, int32_t>::type;
@@ -249,7 +276,7 @@ __device__ __forceinline__ int64_t tile_of(const EngineArgs& a, int64_t iteratio
 }
 
 template <int M, int VW>
-__global__ __launch_bounds__(kThreads) void copy_small_rows(const EngineArgs a) {
+__global__ __launch_bounds__(kThreads) void copy_small_rows(const ArgsOf<M> a) {
     using V = typename Vec<VW>::type;
     constexpr bool kCheckAlign = (M == RowsIndirect) && VW > 1;
     __shared__ int64_t src_off[kThreads];
@@ -306,7 +333,7 @@ __global__ __launch_bounds__(kThreads) void copy_small_rows(const EngineArgs a) 
 }
 
 template <int M, int VW>
-__global__ __launch_bounds__(kThreads) void copy_large_rows(const EngineArgs a) {
+__global__ __launch_bounds__(kThreads) void copy_large_rows(const ArgsOf<M> a) {
     using V = typename Vec<VW>::type;
     constexpr bool kCheckAlign = (M == RowsIndirect) && VW > 1;
     for (int64_t item = blockIdx.x; item < a.tiles; item += gridDim.x) {
@@ -367,7 +394,7 @@ int64_t device_cus() {
 constexpr int64_t kSmallJobGroupsPerCu = 2;
 
 template <int M, int VW>
-void launch_engine(EngineArgs a, hipStream_t stream) {
+void launch_engine(ArgsOf<M> a, hipStream_t stream) {
     const int64_t tile_bytes = int64_t{kThreads} * kUnroll * VW;
     const bool small = a.row_bytes <= tile_bytes;
     if (small) {
@@ -400,7 +427,7 @@ void launch_engine(EngineArgs a, hipStream_t stream) {
 }
 
 template <int M>
-void launch_vw(const EngineArgs& a, int vw, hipStream_t stream) {
+void launch_vw(const ArgsOf<M>& a, int vw, hipStream_t stream) {
     switch (vw) {
         case 16: launch_engine<M, 16>(a, stream); break;
         case 8: launch_engine<M, 8>(a, stream); break;
@@ -447,7 +474,7 @@ constexpr uint32_t kHostRows = kThreads * kHostRowsPerThread;
 constexpr int64_t kHostMoveBytes = int64_t{6} << 20;
 constexpr int64_t kHostRowBytes = 256;
 
-__global__ __launch_bounds__(kThreads) void move_host_rows(const EngineArgs a, uint32_t batch_rows, FastDiv move_div) {
+__global__ __launch_bounds__(kThreads) void move_host_rows(const MoveArgs a, uint32_t batch_rows, FastDiv move_div) {
     constexpr int VW = 16;
     using V = typename Vec<VW>::type;
     constexpr int kWaves = kThreads / 64;
@@ -560,7 +587,7 @@ bool in_host_memory(const void* address) {
 }
 
 // Moves from host memory through move_host_rows; false when the job does not fit its 32-bit counts.
-bool host_move(EngineArgs a, int64_t rows, hipStream_t stream) {
+bool host_move(MoveArgs a, int64_t rows, hipStream_t stream) {
     // Vectors per (layer, batch) row at most; a batch of rows stays below 2^31 with room for the last stride.
     const int64_t per_row = a.K * a.KV * (a.row_bytes / 16);
     const int64_t limit = (int64_t{1} << 30) / per_row;
@@ -787,7 +814,7 @@ int move_kv(const ekv_planes* src, const ekv_tensor* src_rows_p, const ekv_plane
     for (const auto* t : {&src_rows, &dst_rows, &counts}) {
         need_data(*t, "move list");
     }
-    EngineArgs a{};
+    MoveArgs a{};
     a.units = units;
     a.row_bytes = dst->row_bytes;
     a.layer_stride = dst->layer_stride;
@@ -831,7 +858,7 @@ int move_kv(const ekv_planes* src, const ekv_tensor* src_rows_p, const ekv_plane
     const bool linked = vw == 16 && a.row_bytes >= kHostRowBytes && units * a.row_bytes >= kHostMoveBytes &&
                         in_host_memory(src->base);
     if (!linked || !host_move(a, L * list_rows, s)) {
-        launch_vw<KvMove>(a, vw, s);
+        selected != nullptr ? launch_vw<KvMoveSelected>(a, vw, s) : launch_vw<KvMove>(a, vw, s);
     }
     check_hip(hipGetLastError(), "launch KV move");
     return 0;
