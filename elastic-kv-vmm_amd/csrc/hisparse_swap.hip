@@ -39,8 +39,9 @@
 //   4. the same scan over contiguous runs of the old LRU order gives each
 //      slot's place in the new order and the victims (empty slots first, then
 //      untouched slots);
-//   5. a second launch copies the misses' rows from mapped pinned host memory,
-//      16 bytes per lane when rows and bases allow.
+//   5. the misses' rows are copied from mapped pinned host memory, 16 bytes
+//      per lane when rows and bases allow: by the row's own workgroup, or by
+//      a second launch where few batch rows miss much.
 // Locations outside the device buffer are reported as -1 and never written.
 #include "../../include/ekv_kernels.h"
 #include "ekv_common.h"
@@ -170,12 +171,51 @@ __device__ __forceinline__ int64_t device_row(const HsArgs& a, int64_t r, int64_
     return row >= 0 && row < a.dev_rows ? row : -1;
 }
 
+// The K and V rows of this row's misses, copied by its own workgroup: the
+// pieces of all misses (both planes) are dealt to the threads in order,
+// 16 KiB of them in flight with 16-byte pieces whatever the workgroup.
+template <int kThreads, int kVecWidth>
+__device__ __forceinline__ void copy_own_rows(const HsArgs& a, const Lds& s, int32_t misses) {
+    using V = typename Vec<kVecWidth>::type;
+    constexpr int kLoads = kThreads < 1024 ? 1024 / kThreads : 1;
+    const uint32_t per_plane = static_cast<uint32_t>(a.row_bytes / kVecWidth);
+    const uint32_t total = static_cast<uint32_t>(misses) * 2u * per_plane;
+    for (uint32_t first = 0; first < total; first += kLoads * kThreads) {
+        V v[kLoads];
+        int64_t dst[kLoads];
+        bool copies[kLoads];
+#pragma unroll
+        for (int k = 0; k < kLoads; ++k) {
+            const uint32_t q = first + k * kThreads + threadIdx.x;
+            const uint32_t m = q < total ? a.row_div.div(q) : 0u;   // miss rank
+            const uint32_t p = q - m * 2u * per_plane;              // piece within the miss's K and V rows
+            const int64_t kv = p >= per_plane ? 1 : 0;
+            const int64_t within = (static_cast<int64_t>(p) - kv * per_plane) * kVecWidth;
+            const int64_t row = s.miss_loc[m];
+            copies[k] = q < total && row >= 0;
+            dst[k] = kv * a.dev_kv + row * a.dev_rs + within;   // below 0 where V lies before K
+            if (copies[k]) {
+                const int64_t src = s.lane_val[s.miss_lane[m]];
+                v[k] = *reinterpret_cast<const V*>(a.host_k + kv * a.host_kv + src * a.host_rs + within);
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < kLoads; ++k) {
+            if (copies[k]) {
+                *reinterpret_cast<V*>(a.dev_k + dst[k]) = v[k];
+            }
+        }
+    }
+}
+
 // One workgroup per batch row holds its CU nearly alone (134 KiB of LDS at the
 // largest shape) and is a chain of barriers, so the more waves share its loops the
 // shorter it is: kThreads is the smallest size whose threads hold four hot slots
 // and two lanes each. 24 rows of 2048 lanes and 4096 slots: 44 us with 256
 // threads, 23 us with 1024.
-template <int kThreads>
+// kCopyWidth: bytes per copy piece when the workgroup copies its row's misses
+// itself, 0 when the copy launch does (copies_own_rows decides).
+template <int kThreads, int kCopyWidth>
 __global__ __launch_bounds__(kThreads) void hisparse_swap_kernel(const HsArgs a) {
     constexpr int kWaves = kThreads / 64;
     extern __shared__ __align__(16) unsigned char shared[];
@@ -285,7 +325,7 @@ __global__ __launch_bounds__(kThreads) void hisparse_swap_kernel(const HsArgs a)
     }
     __syncthreads();
 
-    // 2. Classify every lane (a thread holds lanes threadIdx.x + 256 k):
+    // 2. Classify every lane (a thread holds lanes threadIdx.x + kThreads k):
     //    the hash probes (a hit marks its slot, a miss claims a bucket), then
     //    one batch of loads: the device row of each hit, the host row of each
     //    miss.
@@ -506,7 +546,7 @@ __global__ __launch_bounds__(kThreads) void hisparse_swap_kernel(const HsArgs a)
         __syncthreads();
     }
 
-    // 6. Outputs of miss lanes and the -1 tail. A token's first lane leaves
+    // 6. Outputs of miss lanes and the -1 tail. Without copies of its own, a token's first lane leaves
     //    -2 - (miss rank << kSlotBits | slot) for the copy launch, which copies
     //    the slot's rows and puts its location there; a repeated token takes
     //    the location at once.
@@ -515,19 +555,22 @@ __global__ __launch_bounds__(kThreads) void hisparse_swap_kernel(const HsArgs a)
             const int32_t owner = s.hash[s.lane_aux[o]] - static_cast<int32_t>(H);
             const int32_t m = s.lane_rank[owner];
             const int32_t loc = s.miss_loc[m];
-            out[s.lane_pos[o] * a.out_so] = owner == o && loc >= 0 ? -2 - (m << kSlotBits | int32_t{s.victim[m]}) : loc;
+            const bool left = kCopyWidth == 0 && owner == o && loc >= 0;
+            out[s.lane_pos[o] * a.out_so] = left ? -2 - (m << kSlotBits | int32_t{s.victim[m]}) : loc;
         }
     }
     for (int64_t o = selected + threadIdx.x; o < W; o += kThreads) {
         out[o * a.out_so] = -1;
     }
+    if constexpr (kCopyWidth > 0) {
+        copy_own_rows<kThreads, kCopyWidth>(a, s, misses);
+    }
 }
 
-// The misses' K and V rows, copied from the host cache by a launch of its own
-// right behind the swap: the host link bounds it, and one workgroup per
-// batch row kept it busy neither with few rows (16 KiB in flight each) nor with
-// many (unequal misses, and the link serves the XCDs unequally once requests
-// queue up). kCopyGroups workgroups of one 16-byte load per lane keep 192 KiB
+// The misses' K and V rows of a few long batch rows, copied from the host cache
+// by a launch of its own right behind the swap: the host link bounds it, and
+// copy_own_rows keeps 16 KiB per batch row in flight, too little for so few.
+// kCopyGroups workgroups of one 16-byte load per lane keep 192 KiB
 // in flight, the amount that reached the link's rate for the row moves (57 GB/s).
 // A miss to copy is an output entry -2 - (miss rank << kSlotBits | slot), left
 // by the swap's step 6. The slot names its token, which names its host row,
@@ -536,31 +579,23 @@ __global__ __launch_bounds__(kThreads) void hisparse_swap_kernel(const HsArgs a)
 // entries and takes the misses whose rank plus batch row is its own modulo
 // the grid: a row's misses are dealt round robin, whatever block-sized runs
 // they come in, and no workgroup acts on an entry that another one replaces.
-// (Entries dealt in runs of 16 left some waves far more rows than others: 511
-// against 477 us for 25.5 MB.) 24 rows took 569 us when each row's workgroup
-// copied its own misses and 476 us so; one row of 512 lanes and 512 B rows,
-// 89 and 21 us.
+constexpr int64_t kCopyRows = 8;                     // batch rows of a copy launch at most
 constexpr uint32_t kCopyGroups = 48;
 constexpr int kCopyThreads = 256;
 constexpr int kScan = 16;                            // entries in flight per thread
 constexpr uint32_t kRound = kCopyThreads * kScan;    // entries per round of the scan
-constexpr uint32_t kCopyBatch = 2048;                // misses whose copy pieces fit 32 bits (checked by the host)
-// The list is copied once it holds more than this, so that a large batch's copies
-// start early in its scan: 128 rows of 2048 lanes 2,340 us, 2,411 with 2,048 (24 rows: 493 both).
-constexpr uint32_t kFlush = 512;
-constexpr uint32_t kListed = kFlush + kRound;        // misses listed at most
+// Misses a workgroup is dealt at most: every kCopyGroups-th of each row's.
+constexpr uint32_t kListed = kCopyRows * ((kMaxLanes + kCopyGroups - 1) / kCopyGroups);
+constexpr int kResolve = (kListed + kCopyThreads - 1) / kCopyThreads;   // per thread
 
 template <typename V>
-__global__ __launch_bounds__(kCopyThreads) void copy_missed_rows(const HsArgs a, int64_t first_row,
-                                                                 uint32_t entries, FastDiv width_div,
+__global__ __launch_bounds__(kCopyThreads) void copy_missed_rows(const HsArgs a, uint32_t entries, FastDiv width_div,
                                                                  FastDiv group_div) {
     constexpr int64_t kWidth = sizeof(V);
-    constexpr int kResolve = 4;            // misses resolved per thread at a time
     __shared__ uint32_t host_of[kListed];  // entry, then host row (all ones: none)
     __shared__ int32_t dev_of[kListed];    // slot, then device row (-1: none)
     __shared__ uint32_t listed;
     const uint32_t per_plane = static_cast<uint32_t>(a.row_bytes / kWidth);
-    const int32_t* out = a.out + first_row * a.out_sb;
     if (threadIdx.x == 0) {
         listed = 0;
     }
@@ -572,7 +607,7 @@ __global__ __launch_bounds__(kCopyThreads) void copy_missed_rows(const HsArgs a,
             const uint32_t e = base + k * kCopyThreads + threadIdx.x;
             const uint32_t at = e < entries ? e : 0u;
             const uint32_t row = width_div.div(at);
-            held[k] = out[row * a.out_sb + (at - row * width_div.divisor) * a.out_so];
+            held[k] = a.out[row * a.out_sb + (at - row * width_div.divisor) * a.out_so];
         }
 #pragma unroll
         for (int k = 0; k < kScan; ++k) {
@@ -587,72 +622,62 @@ __global__ __launch_bounds__(kCopyThreads) void copy_missed_rows(const HsArgs a,
                 }
             }
         }
-        __syncthreads();
-        const uint32_t n = listed;
-        if (n <= kFlush && entries - base > kRound) {   // uniform: more of the scan fits
-            __syncthreads();   // the next round counts on only after every thread has read the count
-            continue;
-        }
-        for (uint32_t first = 0; first < n; first += kResolve * kCopyThreads) {
-            int64_t request[kResolve], loc[kResolve], host[kResolve];
-            int32_t token[kResolve];
-            uint32_t entry[kResolve];
+    }
+    __syncthreads();
+    const uint32_t n = listed;
+    if (n == 0) {
+        return;   // uniform
+    }
+    int64_t request[kResolve], loc[kResolve], host[kResolve];
+    int32_t token[kResolve];
+    uint32_t entry[kResolve];
 #pragma unroll
-            for (int k = 0; k < kResolve; ++k) {
-                const uint32_t i = first + k * kCopyThreads + threadIdx.x;
-                entry[k] = host_of[i < n ? i : first];
-                request[k] = a.req[first_row + width_div.div(entry[k])];
-            }
+    for (int k = 0; k < kResolve; ++k) {
+        const uint32_t i = k * kCopyThreads + threadIdx.x;
+        entry[k] = host_of[i < n ? i : 0u];
+        request[k] = a.req[width_div.div(entry[k])];
+    }
 #pragma unroll
-            for (int k = 0; k < kResolve; ++k) {
-                const uint32_t i = first + k * kCopyThreads + threadIdx.x;
-                const int64_t slot = dev_of[i < n ? i : first];
-                token[k] = a.tokens[request[k] * a.tok_sr + slot * a.tok_ss];
-                loc[k] = device_row(a, request[k], slot);
-            }
+    for (int k = 0; k < kResolve; ++k) {
+        const uint32_t i = k * kCopyThreads + threadIdx.x;
+        const int64_t slot = dev_of[i < n ? i : 0u];
+        token[k] = a.tokens[request[k] * a.tok_sr + slot * a.tok_ss];
+        loc[k] = device_row(a, request[k], slot);
+    }
 #pragma unroll
-            for (int k = 0; k < kResolve; ++k) {
-                const bool known = token[k] >= 0 && token[k] < a.T;
-                const int64_t row = load_index(a.host_locs, a.host_locs64,
-                                               known ? request[k] * a.hl_sr + token[k] * a.hl_st : 0);
-                host[k] = known && row >= 0 && row < a.host_rows ? row : -1;
-            }
-            __syncthreads();   // entry `first` stands in for threads past the list until all of them have read it
+    for (int k = 0; k < kResolve; ++k) {
+        const bool known = token[k] >= 0 && token[k] < a.T;
+        const int64_t row = load_index(a.host_locs, a.host_locs64,
+                                       known ? request[k] * a.hl_sr + token[k] * a.hl_st : 0);
+        host[k] = known && row >= 0 && row < a.host_rows ? row : -1;
+    }
+    __syncthreads();   // entry 0 stands in for threads past the list until all of them have read it
 #pragma unroll
-            for (int k = 0; k < kResolve; ++k) {
-                const uint32_t i = first + k * kCopyThreads + threadIdx.x;
-                if (i < n) {
-                    const uint32_t row = width_div.div(entry[k]);
-                    a.out[(first_row + row) * a.out_sb + (entry[k] - row * width_div.divisor) * a.out_so] =
-                        static_cast<int32_t>(loc[k]);
-                    host_of[i] = static_cast<uint32_t>(host[k]);
-                    dev_of[i] = static_cast<int32_t>(loc[k]);
-                }
-            }
-            __syncthreads();
+    for (int k = 0; k < kResolve; ++k) {
+        const uint32_t i = k * kCopyThreads + threadIdx.x;
+        if (i < n) {
+            const uint32_t row = width_div.div(entry[k]);
+            a.out[row * a.out_sb + (entry[k] - row * width_div.divisor) * a.out_so] = static_cast<int32_t>(loc[k]);
+            host_of[i] = static_cast<uint32_t>(host[k]);
+            dev_of[i] = static_cast<int32_t>(loc[k]);
         }
-        for (uint32_t from = 0; from < n; from += kCopyBatch) {
-            const uint32_t pieces = (n - from < kCopyBatch ? n - from : kCopyBatch) * 2u * per_plane;
-            for (uint32_t q = threadIdx.x; q < pieces; q += kCopyThreads) {
-                const uint32_t m = a.row_div.div(q);
-                const uint32_t p = q - m * 2u * per_plane;   // piece within the miss's K and V rows
-                const int64_t kv = p >= per_plane ? 1 : 0;
-                const int64_t within = (static_cast<int64_t>(p) - kv * per_plane) * kWidth;
-                const uint32_t src = host_of[from + m];
-                const int64_t dst = dev_of[from + m];
-                if (src != ~0u && dst >= 0) {
-                    *reinterpret_cast<V*>(a.dev_k + kv * a.dev_kv + dst * a.dev_rs + within) =
-                        *reinterpret_cast<const V*>(a.host_k + kv * a.host_kv + src * a.host_rs + within);
-                }
-            }
+    }
+    __syncthreads();
+    const uint32_t pieces = n * 2u * per_plane;   // below 2^31 (kMaxLanes misses of any row are, checked by the host)
+    for (uint32_t q = threadIdx.x; q < pieces; q += kCopyThreads) {
+        const uint32_t m = a.row_div.div(q);
+        const uint32_t p = q - m * 2u * per_plane;   // piece within the miss's K and V rows
+        const int64_t kv = p >= per_plane ? 1 : 0;
+        const int64_t within = (static_cast<int64_t>(p) - kv * per_plane) * kWidth;
+        const uint32_t src = host_of[m];
+        const int64_t dst = dev_of[m];
+        if (src != ~0u && dst >= 0) {
+            *reinterpret_cast<V*>(a.dev_k + kv * a.dev_kv + dst * a.dev_rs + within) =
+                *reinterpret_cast<const V*>(a.host_k + kv * a.host_kv + src * a.host_rs + within);
         }
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            listed = 0;
-        }
-        __syncthreads();
     }
 }
+static_assert(kListed <= kMaxLanes, "the listed misses' pieces fit 32 bits when kMaxLanes misses' do");
 
 size_t lds_bytes(int64_t H, int64_t HB, int64_t W) {
     auto round = [](int64_t bytes) { return static_cast<size_t>((bytes + 15) & ~int64_t{15}); };
@@ -660,9 +685,9 @@ size_t lds_bytes(int64_t H, int64_t HB, int64_t W) {
            round((3 * kMaxWaves + 4) * 4);
 }
 
-template <int kThreads>
+template <int kThreads, int kCopyWidth>
 void launch_swap_threads(const HsArgs& a, size_t lds, hipStream_t stream) {
-    const auto kernel = hisparse_swap_kernel<kThreads>;
+    const auto kernel = hisparse_swap_kernel<kThreads, kCopyWidth>;
     // The LDS limit is raised once per device, to the largest size any call
     // needs, so calls recorded into a graph make no attribute call.
     static std::atomic<bool> raised[kMaxDevices];
@@ -682,15 +707,16 @@ void launch_swap_threads(const HsArgs& a, size_t lds, hipStream_t stream) {
     check_hip(hipGetLastError(), "launch hisparse swap-in");
 }
 
+template <int kCopyWidth>
 void launch_swap(const HsArgs& a, size_t lds, hipStream_t stream) {
     const int64_t threads = std::max((a.H + kBatch - 1) / kBatch,
                                      (int64_t{a.width} + kLanesPerThread - 1) / kLanesPerThread);
     if (threads <= 256) {
-        launch_swap_threads<256>(a, lds, stream);
+        launch_swap_threads<256, kCopyWidth>(a, lds, stream);
     } else if (threads <= 512) {
-        launch_swap_threads<512>(a, lds, stream);
+        launch_swap_threads<512, kCopyWidth>(a, lds, stream);
     } else {
-        launch_swap_threads<1024>(a, lds, stream);
+        launch_swap_threads<1024, kCopyWidth>(a, lds, stream);
     }
 }
 
@@ -698,13 +724,27 @@ template <int kVecWidth>
 void launch_copy(const HsArgs& a, hipStream_t stream) {
     // The bytes in flight are what counts: narrower pieces take more workgroups.
     const uint32_t groups = kCopyGroups * (16 / kVecWidth);
-    const int64_t rows_at_once = (int64_t{1} << 30) / a.width;   // entries are counted in 32 bits
-    for (int64_t first = 0; first < a.batch; first += rows_at_once) {
-        const int64_t rows = std::min(rows_at_once, a.batch - first);
-        copy_missed_rows<typename Vec<kVecWidth>::type><<<dim3(groups), dim3(kCopyThreads), 0, stream>>>(
-            a, first, static_cast<uint32_t>(rows * a.width), FastDiv(a.width), FastDiv(groups));
-        check_hip(hipGetLastError(), "launch hisparse row copies");
-    }
+    copy_missed_rows<typename Vec<kVecWidth>::type><<<dim3(groups), dim3(kCopyThreads), 0, stream>>>(
+        a, static_cast<uint32_t>(a.batch * a.width), FastDiv(a.width), FastDiv(groups));
+    check_hip(hipGetLastError(), "launch hisparse row copies");
+}
+
+// Whether every batch row's workgroup copies its own misses, or a launch of
+// its own does: with more than kCopyRows rows the workgroups keep the link busy by
+// themselves, and up to kOwnBytes of rows per batch row are copied sooner than
+// a second launch has scanned the entries. Measured (us; own copies / copy launch, most lanes
+// missing and in brackets none; rows of 512 B):
+//   1 x 256 lanes     31.4 / 19.3  (9.9 / 13.3)     1 x 128 lanes    18.5 / 15.9  (8.8 / 11.8)
+//   1 x 2048 lanes     123 / 43.5  (17.9 / 20.4)    4 x 128 lanes    21.8 / 20.2  (8.7 / 11.9)
+//   8 x 256 lanes     39.7 / 38.7  (11.7 / 14.9)    8 x 128 lanes    23.5 / 24.7  (8.7 / 11.9)
+//   8 x 2048 lanes     188 / 169   (19.0 / 25.6)    8 x 64 lanes     18.0 / 19.4  (8.6 / 12.0)
+//   16 x 256 lanes    53.6 / 59.9  (11.8 / 14.9)    128 x 256 lanes   307 / 338   (13.9 / 24.8)
+//   16 x 2048 lanes    305 / 313   (19.8 / 32.5)    128 x 2048 lanes 2,099 / 2,184 (20.1 / 104)
+//   24 x 2048 lanes    433 / 456   (19.7 / 36.6)    256 x 128 lanes   276 / 303   (9.6 / 21.4)
+constexpr int64_t kOwnBytes = int64_t{128} << 10;
+
+bool copies_own_rows(const HsArgs& a) {
+    return a.batch > kCopyRows || a.width * 2 * a.row_bytes <= kOwnBytes;
 }
 
 void need_index2(const ekv_tensor& t, const char* name) {
@@ -862,7 +902,17 @@ int hisparse_swap_in(const ekv_tensor* topk_p, const ekv_tensor* tokens_p, const
         throw std::invalid_argument("rows too large for one swap-in (copy pieces exceed 2^31)");
     }
     a.row_div = FastDiv(static_cast<uint32_t>(pieces));
-    launch_swap(a, lds, st);
+    if (copies_own_rows(a)) {
+        switch (vw) {
+            case 16: launch_swap<16>(a, lds, st); break;
+            case 8: launch_swap<8>(a, lds, st); break;
+            case 4: launch_swap<4>(a, lds, st); break;
+            case 2: launch_swap<2>(a, lds, st); break;
+            default: launch_swap<1>(a, lds, st); break;
+        }
+        return 0;
+    }
+    launch_swap<0>(a, lds, st);
     if (R == 0 || T == 0) {
         return 0;   // no row has state or no token a host row: nothing missed
     }

@@ -211,10 +211,11 @@ def test_decode_sized_call_matches_the_oracle(gpu):
     assert (out >= 0).all().item()                                          # every lane selected a valid token
 
 
-def test_graph_replays_with_padding_rows_match_the_oracle(gpu):
+@pytest.mark.parametrize("row_bytes", [64, 4096])      # copies of the swap's own, and a copy launch
+def test_graph_replays_with_padding_rows_match_the_oracle(gpu, row_bytes):
     # SGLang replays decode from captured graphs; rows at or past num_real_reqs are padding.
     rng = np.random.default_rng(505)
-    batch, hot, bs, k, context, row_bytes = 4, 64, 4, 6, 400, 64
+    batch, hot, bs, k, context = 4, 64, 4, 6, 400
     host_rows = batch * context
     host_locs = rng.permutation(host_rows).reshape(batch, context)
     dev_locs = rng.permutation(batch * (hot + 1)).reshape(batch, hot + 1) + 1
@@ -272,10 +273,13 @@ def test_graph_replays_with_padding_rows_match_the_oracle(gpu):
         torch.randn(1000, device=gpu).sum().item()        # eager work between replays
 
 
-@pytest.mark.parametrize("batch,row_bytes", [(52, 16), (1, 1024), (3, 72), (7, 6)])
+# Past the largest batch or at the most row bytes that copy their own misses, and (8, 64), (8, 36) the fullest copy
+# launch: 43 of each request's 2,048 misses for one workgroup. 72, 36, 38 and 41 bytes are pieces of 8, 4, 2 and 1.
+@pytest.mark.parametrize("batch,row_bytes", [(52, 16), (1, 1024), (3, 72), (7, 6), (8, 64), (9, 64), (8, 32), (8, 36),
+                                             (2, 38), (2, 41)])
 def test_copy_launch_deals_out_every_miss(gpu, batch, row_bytes):
-    # A cold step (every lane misses: 2,048 rows per request, over 2,048 of them for one copy workgroup at 52
-    # requests), then a mixed one: each miss is copied once, by the workgroup its rank falls to.
+    # A cold step (every lane misses), then a mixed one: each miss is copied once, by its request's workgroup or by the
+    # one of the copy launch that its rank falls to.
     rng = np.random.default_rng(batch)
     hot, bs, k, context = 2048, 16, 128, 4096
     host_rows = batch * context
