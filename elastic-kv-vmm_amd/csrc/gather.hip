@@ -124,6 +124,7 @@ struct EngineArgs {
 struct MoveArgs : EngineArgs {
     IndexRef move_selected;  // data null: every batch row; else entry j of B stands for batch row move_selected[j]
     int64_t move_batch;      // batch rows
+    bool lists_ahead;        // list entries are read with the counts, used or not
 };
 
 template <int M>
@@ -180,13 +181,21 @@ __device__ __forceinline__ void locate(const ArgsOf<M>& a, int64_t u, int64_t& s
             place(l, kv, from, to);
         }
     } else if constexpr (M == KvMoveSelected) {
-        // The selection entry, and the count and list entries of the row it
-        // names on the guess of the identity selection, are read at once: one
-        // memory level before the row itself instead of three (entries at or past the count are read but not used).
         int64_t l, j, kv, k;
         split_unit(a, u, l, j, kv, k);
         src = -1;
         dst = -1;
+        if (!a.lists_ahead) {   // uniform
+            const int64_t b = move_row(a, j);
+            if (b >= 0 && k < a.move_counts[l * a.mc_l + b * a.mc_b]) {
+                place(l, kv, a.move_src_rows[l * a.msr_l + b * a.msr_b + k * a.msr_i],
+                      a.move_dst_rows[l * a.mdr_l + b * a.mdr_b + k * a.mdr_i]);
+            }
+            return;
+        }
+        // The selection entry, and the count and list entries of the row it
+        // names on the guess of the identity selection, are read at once: one
+        // memory level before the row itself instead of three (entries at or past the count are read but not used).
         const int64_t guess = j < a.move_batch ? j : 0;
         int32_t count = a.move_counts[l * a.mc_l + guess * a.mc_b];
         int64_t from = a.move_src_rows[l * a.msr_l + guess * a.msr_b + k * a.msr_i];
@@ -368,6 +377,12 @@ __global__ __launch_bounds__(kThreads) void copy_large_rows(const ArgsOf<M> a) {
         }
     }
 }
+
+// Rows (of both planes) up to which a move over a selection reads its lists ahead of
+// the counts: a short job is a chain of reads (8 x 64 lanes: 0.1 us of 3.3), a long one pays for
+// the tails it does not use. Measured (us, none of the lists used; ahead / behind the counts):
+// 128 x 2048 lanes (524,288 rows) 19.4 / 19.1, 20 layers of them 89 / 71; 40 % used 30.5 / 31.2, 106 / 96.
+constexpr int64_t kListsAhead = int64_t{1} << 19;
 
 // Compute units of the current device (cached per device).
 int64_t device_cus() {
@@ -837,6 +852,7 @@ int move_kv(const ekv_planes* src, const ekv_tensor* src_rows_p, const ekv_plane
     a.KV = dst->kv;
     a.B = list_rows;
     a.move_batch = B;
+    a.lists_ahead = units <= kListsAhead;
     if (selected != nullptr) {
         a.move_selected = index_ref(*selected, 0);
     }

@@ -312,10 +312,12 @@ def test_one_launch_lookup_and_swap_equals_the_kernels(gpu, host, table_dtype, s
             assert torch.equal(a, z), step
 
 
-def test_promotion_of_a_selection_past_the_tile_kernel(gpu):
-    # Lists of 7 MiB of pinned host rows: the step's promotion walks the selection in the host-row kernel. Permuted,
-    # stray and missing entries against the stages, whose move reads every row's count.
-    layers, rows_n, context, hot, lanes, row = 2, 14, 1400, 512, 256, 512
+# Lists of 7 MiB of 512 B host rows take the host-row kernel; of 64 B rows the tile kernel, 573,440 rows of them with
+# the counts read first.
+@pytest.mark.parametrize("rows_n,context,hot,lanes,row", [(14, 1400, 512, 256, 512), (70, 2500, 2048, 2048, 64)])
+def test_promotions_over_a_selection_in_each_kernel(gpu, rows_n, context, hot, lanes, row):
+    # Permuted, stray and missing selection entries against the stages, whose move reads every row's count.
+    layers = 2
     plane = rows_n * context * row
     arena = HostArena(layers * 2 * plane)
     try:
