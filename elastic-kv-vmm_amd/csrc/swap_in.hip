@@ -1191,21 +1191,24 @@ int swap_in(const ekv_tensor* topk_p, int64_t block_size, const ekv_tensor* rows
     const dim3 grid(static_cast<uint32_t>(count), static_cast<uint32_t>(L));
     const auto s = static_cast<hipStream_t>(stream);
     // The workgroup size: the smallest whose threads hold four slots and two
-    // lanes each while every row has a CU to itself, so that the most waves
-    // share a row's phases; with more rows than CUs the smallest whose threads
+    // lanes each, so that the most waves share a row's phases, while such workgroups
+    // fill no more than half of the CUs' threads; past that the smallest whose threads
     // hold eight and four, since what each wave repeats (scans, ranges) then
-    // costs the rows beside it. Measured (us, with the launch; capacity is twice the lanes):
-    //   rows x lanes        eight and four   four and two
-    //   48 x 1024                20.0             15.7
-    //   48 x 2048                23.0             21.0
-    //   256 x 2048               24.7             23.2
-    //   512 x 2048               30.7             38.9
-    //   2560 x 512               39.7             45.8
-    //   2560 x 1024              69.5             74.3
-    //   2560 x 2048             133.5            179.8
-    // (2560 x 256: 34.0 against 28.0, so rows of up to 512 slots stay with
-    // four. Taken before the scans became DPP steps, which took up to 18 us off both.)
-    constexpr int64_t kCus = 256;
+    // costs the rows beside it. Measured (us, the swap alone; lanes and slots of a row):
+    //   rows x lanes, slots     four and two   eight and four
+    //   48 x 1024, 2048             13.0           15.2
+    //   256 x 2048, 4096            21.0           22.6
+    //   512 x 1024, 2048            19.4           21.2
+    //   512 x 512, 1024             14.8           18.7
+    //   384 x 2048, 4096            33.3           26.6
+    //   1024 x 1024, 2048           33.6           27.8
+    //   2560 x 256, 1024            31.0           28.6
+    //   2560 x 512, 1024            38.9           43.1   (on the wrong side of the line)
+    //   2560 x 768, 1536            60.5           48.3
+    //   2560 x 1024, 2048           67.0           62.0
+    //   2560 x 2048, 4096          162.9          115.0
+    // (2560 x 256, 512: 24.7 against 27.8, so rows of up to 512 slots stay with four.)
+    constexpr int64_t kHalfOfThreads = 256 * 1024;
     const bool dense = a.topk_sk == 1 && a.sl_o == 1 && a.mi_o == 1 && a.st_c == 1 && a.sp_c == 1 && a.ps_o == 1 &&
                        a.pd_o == 1 && a.tb_t == 1 && a.host_st == 1 && (a.bits == nullptr || a.bt_w == 1) &&
                        (a.line_counts == nullptr || a.lc_q == 1) && T < (int64_t{1} << 29);
@@ -1216,7 +1219,11 @@ int swap_in(const ekv_tensor* topk_p, int64_t block_size, const ekv_tensor* rows
         a.lengths = index_ref(*lengths_p, 0);
     }
     const int64_t four = std::max((C + 3) / 4, (W + 1) / 2), eight = std::max((C + 7) / 8, (W + 3) / 4);
-    const bool crowded = count * L > kCus && four > 128;
+    int64_t threads = 64;   // of the four-and-two workgroup
+    while (threads < four) {
+        threads *= 2;
+    }
+    const bool crowded = count * L * threads > kHalfOfThreads && four > 128;
     if (four <= 64) {
         launch_swap<64, 4, 2>(a, dense, grid, lds, s);
     } else if (four <= 128) {
