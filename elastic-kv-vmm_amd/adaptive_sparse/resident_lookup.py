@@ -15,9 +15,10 @@ Extensions (all optional, none changes the reference behaviour):
   * resident_bits / bits_shift (single level only): a residency summary
     built by build_residency_bits, one bit per group of 2**bits_shift
     positions (0: per position; 6: per 128-byte line of an int16 table);
-    lanes whose group bit is clear skip their table read. A summary may be a
-    superset of the table's residency (a set bit over unresident positions
-    only costs their table reads), never a subset;
+    lanes whose group bit is clear skip their table read where the lookup
+    reads the summary (small and whole-block lookups read the table alone).
+    A summary may be a superset of the table's residency (a set bit over
+    unresident positions only costs their table reads), never a subset;
   * slot_base (single level only): the table is int16 and holds local slots
     (0 = not resident, v >= 1 = local slot v - 1 of the request); the slot
     written is slot_base[rows[r]] + v - 1. Half the bytes of an int32 table
@@ -68,6 +69,18 @@ def resolve_resident(topk, table, mapping, rows, lengths, selected, output, bloc
     status = helper.resolve(form, entry, topk, table, mapping, slot_base, resident_bits, int(bits_shift), rows,
                             lengths, selected, output, misses, miss_count, int(block_size))
     _native.launch_check(status, "resolve_resident")
+
+
+def lookup_route(topk, table, mapping, rows, lengths, selected, output, block_size, *, misses=None, miss_count=None,
+                 resident_bits=None, bits_shift=0, slot_base=None):
+    """Name of the kernel that resolve_resident takes for these arguments (ekv_lookup_route); launches nothing."""
+    lib = _native.kernel_library()
+    packed = [None if t is None else _native.packed(t) for t in (
+        topk, table, mapping, slot_base, resident_bits, rows, lengths, selected, output, misses, miss_count)]
+    name = lib.ekv_lookup_route(*packed[:5], int(bits_shift), *packed[5:], int(block_size))
+    if name is None:
+        raise RuntimeError("lookup_route: " + lib.ev_error().decode("utf-8", errors="replace"))
+    return name.decode()
 
 
 def summary_words(context, shift=0):

@@ -1620,12 +1620,52 @@ void launch_runs_pipe_loads(const LookupArgs& a, dim3 grid, hipStream_t stream) 
         a, items, count, FastDiv(count));
 }
 
+// The kernel of a lookup.
+enum class Route { kNone, kBlocks, kDirect, kTwoStage, kOneStage, kRuns, kLocal, kSingle, kMappedDirect, kMapped };
+
+const char* route_name(Route route) {
+    switch (route) {
+        case Route::kNone: return "none";
+        case Route::kBlocks: return "blocks";
+        case Route::kDirect: return "direct";
+        case Route::kTwoStage: return "two-stage prefetch";
+        case Route::kOneStage: return "one-stage prefetch";
+        case Route::kRuns: return "runs";
+        case Route::kLocal: return "local";
+        case Route::kSingle: return "strided";
+        case Route::kMappedDirect: return "two-level direct";
+        case Route::kMapped: return "two-level";
+    }
+    return "";
+}
+
 // Summary rows of at most kThreads 16-byte pieces take the two-stage kernel;
 // longer ones (up to 2 * kThreads pieces) the one-stage kernel with two
 // pieces per thread.
+Route route_of(const LookupArgs& a, int32_t topk_dtype, int32_t table_dtype, bool dense) {
+    if (a.mapping != nullptr) {
+        return a.direct ? Route::kMappedDirect : Route::kMapped;
+    }
+    if (a.block_runs) {
+        return Route::kBlocks;
+    }
+    if (a.direct) {
+        return Route::kDirect;
+    }
+    if (dense && a.bits != nullptr && topk_dtype == EKV_INT32) {
+        if (a.pipe) {
+            return (a.bits_words + 3) / 4 <= kThreads ? Route::kTwoStage : Route::kOneStage;
+        }
+        if (table_dtype == EKV_INT16) {
+            return a.runs ? Route::kRuns : Route::kLocal;
+        }
+    }
+    return Route::kSingle;
+}
+
 template <bool kCompact, typename TableT>
-void launch_runs_pipe(const LookupArgs& a, dim3 grid, hipStream_t stream) {
-    if ((a.bits_words + 3) / 4 <= kThreads) {
+void launch_runs_pipe(const LookupArgs& a, Route route, dim3 grid, hipStream_t stream) {
+    if (route == Route::kTwoStage) {
         launch_runs_pipe2<kCompact, TableT>(a, grid, stream);
     } else {
         launch_runs_pipe_loads<kCompact, TableT, 2>(a, grid, stream);
@@ -1659,83 +1699,54 @@ void launch_direct(const LookupArgs& a, bool compact, dim3 grid, hipStream_t str
 }
 
 template <typename TopkT, typename TableT>
-void launch_with_table(const LookupArgs& a, int32_t map_dtype, bool compact, bool dense, dim3 grid,
+void launch_with_table(const LookupArgs& a, Route route, int32_t map_dtype, bool compact, bool dense, dim3 grid,
                        hipStream_t stream) {
     const dim3 block(kThreads);
     const size_t lds = sizeof(uint32_t) * ((a.window ? kWindow : 0) + (a.bits_staged ? a.bits_words : 0));
-    if (a.mapping == nullptr) {
-        const bool bits = a.bits != nullptr;
-        if constexpr (!std::is_same_v<TableT, int64_t>) {
-            if (a.block_runs) {
-                if (compact) {
-                    resolve_blocks_kernel<TopkT, TableT, true><<<grid, block, 0, stream>>>(a);
-                } else {
-                    resolve_blocks_kernel<TopkT, TableT, false><<<grid, block, 0, stream>>>(a);
-                }
-                return;
-            }
-            if (a.direct) {
-                launch_direct<TopkT, TableT>(a, compact, grid, stream);
-                return;
-            }
-        }
-        if (dense) {
-            if constexpr (std::is_same_v<TopkT, int32_t> && std::is_same_v<TableT, int16_t>) {
-                if (bits && a.pipe) {
-                    if (compact) {
-                        launch_runs_pipe<true, int16_t>(a, grid, stream);
-                    } else {
-                        launch_runs_pipe<false, int16_t>(a, grid, stream);
-                    }
-                    return;
-                }
-                if (bits && a.runs) {
-                    if (compact) {
-                        resolve_runs_kernel<true><<<grid, block, lds, stream>>>(a);
-                    } else {
-                        resolve_runs_kernel<false><<<grid, block, lds, stream>>>(a);
-                    }
-                    return;
-                }
-                if (bits) {
-                    if (compact) {
-                        resolve_local_kernel<true><<<grid, block, lds, stream>>>(a);
-                    } else {
-                        resolve_local_kernel<false><<<grid, block, lds, stream>>>(a);
-                    }
-                    return;
-                }
-            }
-            if constexpr (std::is_same_v<TopkT, int32_t> && std::is_same_v<TableT, int32_t>) {
-                if (bits && a.pipe) {
-                    if (compact) {
-                        launch_runs_pipe<true, int32_t>(a, grid, stream);
-                    } else {
-                        launch_runs_pipe<false, int32_t>(a, grid, stream);
-                    }
-                    return;
-                }
-            }
-            if (bits && compact) {
-                resolve_single_kernel<TopkT, TableT, true, true, true><<<grid, block, lds, stream>>>(a);
-            } else if (bits) {
-                resolve_single_kernel<TopkT, TableT, true, false, true><<<grid, block, lds, stream>>>(a);
-            } else if (compact) {
-                resolve_single_kernel<TopkT, TableT, false, true, true><<<grid, block, lds, stream>>>(a);
+    if constexpr (!std::is_same_v<TableT, int64_t>) {
+        if (route == Route::kBlocks) {
+            if (compact) {
+                resolve_blocks_kernel<TopkT, TableT, true><<<grid, block, 0, stream>>>(a);
             } else {
-                resolve_single_kernel<TopkT, TableT, false, false, true><<<grid, block, lds, stream>>>(a);
+                resolve_blocks_kernel<TopkT, TableT, false><<<grid, block, 0, stream>>>(a);
             }
-        } else if (bits && compact) {
-            resolve_single_kernel<TopkT, TableT, true, true, false><<<grid, block, lds, stream>>>(a);
-        } else if (bits) {
-            resolve_single_kernel<TopkT, TableT, true, false, false><<<grid, block, lds, stream>>>(a);
-        } else if (compact) {
-            resolve_single_kernel<TopkT, TableT, false, true, false><<<grid, block, lds, stream>>>(a);
-        } else {
-            resolve_single_kernel<TopkT, TableT, false, false, false><<<grid, block, lds, stream>>>(a);
+            return;
         }
-    } else if constexpr (!std::is_same_v<TableT, int16_t>) {  // local tables are single level
-        if (a.direct) {
+        if (route == Route::kDirect) {
+            launch_direct<TopkT, TableT>(a, compact, grid, stream);
+            return;
+        }
+        if constexpr (std::is_same_v<TopkT, int32_t>) {
+            if (route == Route::kTwoStage || route == Route::kOneStage) {
+                if (compact) {
+                    launch_runs_pipe<true, TableT>(a, route, grid, stream);
+                } else {
+                    launch_runs_pipe<false, TableT>(a, route, grid, stream);
+                }
+                return;
+            }
+        }
+    }
+    if constexpr (std::is_same_v<TopkT, int32_t> && std::is_same_v<TableT, int16_t>) {
+        if (route == Route::kRuns) {
+            if (compact) {
+                resolve_runs_kernel<true><<<grid, block, lds, stream>>>(a);
+            } else {
+                resolve_runs_kernel<false><<<grid, block, lds, stream>>>(a);
+            }
+            return;
+        }
+        if (route == Route::kLocal) {
+            if (compact) {
+                resolve_local_kernel<true><<<grid, block, lds, stream>>>(a);
+            } else {
+                resolve_local_kernel<false><<<grid, block, lds, stream>>>(a);
+            }
+            return;
+        }
+    }
+    if constexpr (!std::is_same_v<TableT, int16_t>) {  // local tables are single level
+        if (route == Route::kMappedDirect) {
             const bool narrow = a.width <= 128 * kDirectLanes;
             if (map_dtype == EKV_INT64) {
                 narrow ? launch_direct_width<TopkT, TableT, 128, int64_t>(a, compact, grid, stream)
@@ -1746,31 +1757,54 @@ void launch_with_table(const LookupArgs& a, int32_t map_dtype, bool compact, boo
             }
             return;
         }
-        if (map_dtype == EKV_INT64) {
-            if (compact) {
-                resolve_mapped_kernel<TopkT, TableT, int64_t, true><<<grid, block, lds, stream>>>(a);
+        if (route == Route::kMapped) {
+            if (map_dtype == EKV_INT64) {
+                if (compact) {
+                    resolve_mapped_kernel<TopkT, TableT, int64_t, true><<<grid, block, lds, stream>>>(a);
+                } else {
+                    resolve_mapped_kernel<TopkT, TableT, int64_t, false><<<grid, block, lds, stream>>>(a);
+                }
             } else {
-                resolve_mapped_kernel<TopkT, TableT, int64_t, false><<<grid, block, lds, stream>>>(a);
+                if (compact) {
+                    resolve_mapped_kernel<TopkT, TableT, int32_t, true><<<grid, block, lds, stream>>>(a);
+                } else {
+                    resolve_mapped_kernel<TopkT, TableT, int32_t, false><<<grid, block, lds, stream>>>(a);
+                }
             }
-        } else {
-            if (compact) {
-                resolve_mapped_kernel<TopkT, TableT, int32_t, true><<<grid, block, lds, stream>>>(a);
-            } else {
-                resolve_mapped_kernel<TopkT, TableT, int32_t, false><<<grid, block, lds, stream>>>(a);
-            }
+            return;
         }
+    }
+    const bool bits = a.bits != nullptr;
+    if (dense) {
+        if (bits && compact) {
+            resolve_single_kernel<TopkT, TableT, true, true, true><<<grid, block, lds, stream>>>(a);
+        } else if (bits) {
+            resolve_single_kernel<TopkT, TableT, true, false, true><<<grid, block, lds, stream>>>(a);
+        } else if (compact) {
+            resolve_single_kernel<TopkT, TableT, false, true, true><<<grid, block, lds, stream>>>(a);
+        } else {
+            resolve_single_kernel<TopkT, TableT, false, false, true><<<grid, block, lds, stream>>>(a);
+        }
+    } else if (bits && compact) {
+        resolve_single_kernel<TopkT, TableT, true, true, false><<<grid, block, lds, stream>>>(a);
+    } else if (bits) {
+        resolve_single_kernel<TopkT, TableT, true, false, false><<<grid, block, lds, stream>>>(a);
+    } else if (compact) {
+        resolve_single_kernel<TopkT, TableT, false, true, false><<<grid, block, lds, stream>>>(a);
+    } else {
+        resolve_single_kernel<TopkT, TableT, false, false, false><<<grid, block, lds, stream>>>(a);
     }
 }
 
 template <typename TopkT>
-void launch_table(const LookupArgs& a, int32_t table_dtype, int32_t map_dtype, bool compact, bool dense, dim3 grid,
-                  hipStream_t stream) {
+void launch_table(const LookupArgs& a, Route route, int32_t table_dtype, int32_t map_dtype, bool compact, bool dense,
+                  dim3 grid, hipStream_t stream) {
     if (table_dtype == EKV_INT64) {
-        launch_with_table<TopkT, int64_t>(a, map_dtype, compact, dense, grid, stream);
+        launch_with_table<TopkT, int64_t>(a, route, map_dtype, compact, dense, grid, stream);
     } else if (table_dtype == EKV_INT16) {
-        launch_with_table<TopkT, int16_t>(a, map_dtype, compact, dense, grid, stream);
+        launch_with_table<TopkT, int16_t>(a, route, map_dtype, compact, dense, grid, stream);
     } else {
-        launch_with_table<TopkT, int32_t>(a, map_dtype, compact, dense, grid, stream);
+        launch_with_table<TopkT, int32_t>(a, route, map_dtype, compact, dense, grid, stream);
     }
 }
 
@@ -1778,7 +1812,7 @@ int resolve_resident(const ekv_tensor* topk_p, const ekv_tensor* table_p, const 
                      const ekv_tensor* rows_p, const ekv_tensor* lengths_p, const ekv_tensor* selected_p,
                      const ekv_tensor* output_p, const ekv_tensor* misses_p, const ekv_tensor* counts_p,
                      const ekv_tensor* bits_p, int64_t block_size, void* stream,
-                     const ekv_tensor* slot_base_p = nullptr, int64_t bits_shift = 0) {
+                     const ekv_tensor* slot_base_p = nullptr, int64_t bits_shift = 0, Route* asked = nullptr) {
     const ekv_tensor& topk = need(topk_p, "topk");
     const ekv_tensor& table = need(table_p, "table");
     const ekv_tensor& rows = need(rows_p, "rows");
@@ -2045,10 +2079,15 @@ int resolve_resident(const ekv_tensor* topk_p, const ekv_tensor* table_p, const 
     if (check_only()) {
         return 0;
     }
+    const Route route = route_of(a, topk.dtype, table.dtype, dense);
+    if (asked != nullptr) {
+        *asked = route;
+        return 0;
+    }
     if (topk.dtype == EKV_INT64) {
-        launch_table<int64_t>(a, table.dtype, map_dtype, compact, dense, grid, s);
+        launch_table<int64_t>(a, route, table.dtype, map_dtype, compact, dense, grid, s);
     } else {
-        launch_table<int32_t>(a, table.dtype, map_dtype, compact, dense, grid, s);
+        launch_table<int32_t>(a, route, table.dtype, map_dtype, compact, dense, grid, s);
     }
     check_hip(hipGetLastError(), "launch resident lookup");
     return 0;
@@ -2502,3 +2541,16 @@ extern "C" int ekv_resolve_resident(const ekv_tensor* topk, const ekv_tensor* ta
 }
 
 extern "C" int ekv_abi_version(void) { return EKV_ABI_VERSION; }
+
+extern "C" const char* ekv_lookup_route(const ekv_tensor* topk, const ekv_tensor* table, const ekv_tensor* mapping,
+                                        const ekv_tensor* slot_base, const ekv_tensor* resident_bits,
+                                        int64_t bits_shift, const ekv_tensor* rows, const ekv_tensor* lengths,
+                                        const ekv_tensor* selected, const ekv_tensor* output,
+                                        const ekv_tensor* misses, const ekv_tensor* miss_count, int64_t block_size) {
+    ekv::Route route = ekv::Route::kNone;
+    const int status = ekv::guarded(-1, [&] {
+        return ekv::resolve_resident(topk, table, mapping, rows, lengths, selected, output, misses, miss_count,
+                                     resident_bits, block_size, nullptr, slot_base, bits_shift, &route);
+    });
+    return status == 0 ? ekv::route_name(route) : nullptr;
+}

@@ -80,6 +80,7 @@ _SIGNATURES = {
                                   + [ct.c_int64, ct.c_void_p], ct.c_int),
     "ekv_resolve_resident_local": ([_TENSOR_ADDRESS] * 4 + [ct.c_int64] + [_TENSOR_ADDRESS] * 6
                                    + [ct.c_int64, ct.c_void_p], ct.c_int),
+    "ekv_lookup_route": ([_TENSOR_ADDRESS] * 5 + [ct.c_int64] + [_TENSOR_ADDRESS] * 6 + [ct.c_int64], ct.c_char_p),
     "ekv_residency_bits": ([_P_TENSOR, _P_TENSOR, ct.c_int64, ct.c_void_p], ct.c_int),
     "ekv_residency_summary": ([_P_TENSOR, _P_TENSOR, _P_TENSOR, ct.c_int64, ct.c_void_p], ct.c_int),
     "ekv_gather_rows": ([_P_TENSOR] * 7 + [ct.c_int64, ct.c_int64, ct.c_int, ct.c_void_p], ct.c_int),
@@ -152,8 +153,8 @@ LAUNCHER_PATH = (Path(__file__).resolve().parents[1] / "lib"
 _LAUNCH = {}   # ELASTIC_VMM_LIBRARY key -> (launch helper module, {entry name: address})
 # The entry points the launch helper calls (by address).
 _LAUNCH_ENTRIES = ("ekv_resolve_resident", "ekv_resolve_resident_bits", "ekv_resolve_resident_local",
-                   "ekv_residency_summary", "ekv_gather_rows", "ekv_gather_kv", "ekv_scatter_kv", "ekv_move_kv", "ekv_swap_in",
-                   "ekv_swap_in_counted", "ekv_hisparse_swap_in", "ekv_host_device_pointer", "ekv_decode_step")
+                   "ekv_residency_summary", "ekv_gather_rows", "ekv_gather_kv", "ekv_scatter_kv", "ekv_move_kv",
+                   "ekv_swap_in", "ekv_swap_in_counted", "ekv_hisparse_swap_in", "ekv_host_device_pointer", "ekv_decode_step")
 
 
 _DEFAULT = object()   # _LAUNCH key of the helper bound on the first call without a library argument

@@ -109,12 +109,15 @@ int ekv_resolve_resident(const ekv_tensor* topk, const ekv_tensor* table,
  * covers positions [q << bits_shift, (q + 1) << bits_shift), so
  * W >= ceil(ceil(T / 2^bits_shift) / 32). Bit q must be set whenever a
  * position it covers has table[., p] != 0; a set bit over positions that
- * are all 0 is allowed (a superset only costs table reads).
+ * are all 0 is allowed (a superset only costs table reads). The summary is a
+ * hint: a lookup may read it or the table alone, as its sizes make faster, so
+ * what a lane returns whose bit is clear over a non-zero entry is unspecified.
  *   bits_shift = 0: one bit per position (ekv_residency_bits keeps it exact);
  *   bits_shift = 6: one bit per 64 positions = one 128-byte line of an int16
  *   table, 1/64 of the per-position bitmap's bytes.
- * Lanes whose bit is clear return slot 0 without reading their table entry,
- * so misses in unresident groups cost one bit instead of a cache line.
+ * Where it is read, lanes whose bit is clear return slot 0 without reading
+ * their table entry, so misses in unresident groups cost one bit instead of a
+ * cache line.
  * 0 <= bits_shift <= 20.
  * No reference counterpart: an acceleration of ekv_resolve_resident
  * (adaptive_sparse/resident_lookup.py:29-40 semantics are unchanged).
@@ -144,6 +147,22 @@ int ekv_resolve_resident_local(const ekv_tensor* topk, const ekv_tensor* table,
                                const ekv_tensor* selected, const ekv_tensor* output,
                                const ekv_tensor* misses, const ekv_tensor* miss_count,
                                int64_t block_size, void* stream);
+
+/*
+ * The kernel that a lookup with these arguments takes ("direct", "blocks",
+ * "two-stage prefetch", "one-stage prefetch", "runs", "local", "strided",
+ * "two-level direct", "two-level"; "none" when it launches nothing), or NULL
+ * for arguments that the lookup refuses (ev_error names the reason).
+ * mapping, slot_base, resident_bits, misses and miss_count may be NULL as in
+ * the entry points above. Host only: reads no element, launches nothing and
+ * needs no device. The names serve tests and profiles; which kernel a form takes may change.
+ * No reference counterpart.
+ */
+const char* ekv_lookup_route(const ekv_tensor* topk, const ekv_tensor* table, const ekv_tensor* mapping,
+                             const ekv_tensor* slot_base, const ekv_tensor* resident_bits,
+                             int64_t bits_shift, const ekv_tensor* rows, const ekv_tensor* lengths,
+                             const ekv_tensor* selected, const ekv_tensor* output,
+                             const ekv_tensor* misses, const ekv_tensor* miss_count, int64_t block_size);
 
 /*
  * Exact residency summary of a table (int16, int32 or int64): bit j of word

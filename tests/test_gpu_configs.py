@@ -32,7 +32,7 @@ import torch
 
 from adaptive_sparse.host_arena import HostArena
 from adaptive_sparse.kv_pool import KVPlanes, PlanePoolLayout
-from adaptive_sparse.resident_lookup import build_residency_bits, resolve_resident
+from adaptive_sparse.resident_lookup import build_residency_bits, lookup_route, resolve_resident
 from adaptive_sparse.sparse_read import gather_kv
 from adaptive_sparse.swap_in import INT32_MIN, HotBuffers, move_kv, residency_counts, swap_in
 from elastic_kv.backing import Backing
@@ -350,8 +350,8 @@ def test_config5_full_size_steps_keep_rows_and_lru_invariants(gpu, shift):
 
 def test_prefetching_lookup_with_a_raised_grid(gpu):
     # 40 layers x 1000 rows = 40,000 items: more than 16 per resident workgroup
-    # (2048 on MI355X), so the host raises the grid; K = 8 lanes per row.
-    L, B, R, T, K, C = 40, 1000, 50, 512, 8, 64
+    # (2048 on MI355X), so the host raises the grid; K = 264 lanes per row (up to 256 take the direct kernel).
+    L, B, R, T, K, C = 40, 1000, 50, 512, 264, 64
     rng = np.random.default_rng(8)
     local = np.zeros((L, R, T), np.int64)
     for layer in range(L):
@@ -371,11 +371,12 @@ def test_prefetching_lookup_with_a_raised_grid(gpu):
         slots = torch.full((L, B, K), -3, dtype=torch.int32, device=gpu)
         misses = torch.full((L, B, K), -2, dtype=torch.int32, device=gpu)
         counts = torch.full((L, B), -2, dtype=torch.int32, device=gpu)
-        resolve_resident(torch.tensor(topk, dtype=torch.int32, device=gpu), table16, None,
-                         torch.tensor(rows, device=gpu), torch.tensor(lengths, device=gpu),
-                         torch.tensor(selected, device=gpu), slots, 1, misses=misses, miss_count=counts,
-                         resident_bits=build_residency_bits(table16, shift=shift), bits_shift=shift,
-                         slot_base=torch.tensor(base, device=gpu))
+        args = (torch.tensor(topk, dtype=torch.int32, device=gpu), table16, None, torch.tensor(rows, device=gpu),
+                torch.tensor(lengths, device=gpu), torch.tensor(selected, device=gpu), slots, 1)
+        extra = dict(misses=misses, miss_count=counts, resident_bits=build_residency_bits(table16, shift=shift),
+                     bits_shift=shift, slot_base=torch.tensor(base, device=gpu))
+        assert lookup_route(*args, **extra) == "two-stage prefetch"
+        resolve_resident(*args, **extra)
         assert np.array_equal(slots.cpu().numpy(), want), shift
         got_counts, got_misses = counts.cpu().numpy(), misses.cpu().numpy()
         for layer in range(L):

@@ -16,7 +16,7 @@ import pytest
 import torch
 
 from adaptive_sparse.kv_pool import KVPlanes
-from adaptive_sparse.resident_lookup import build_residency_bits, resolve_resident
+from adaptive_sparse.resident_lookup import build_residency_bits, lookup_route, resolve_resident
 from adaptive_sparse.sparse_read import gather_kv, scatter_kv
 from adaptive_sparse.swap_in import move_kv
 from oracle import oracle as ref
@@ -125,10 +125,10 @@ def test_lookup_random_configurations(gpu, coracle, seed):
 def test_local_slot_runs_random_configurations(gpu, coracle, seed):
     # The decode default: int32 Top-K, int16 local-slot table with slot bases,
     # residency bitmap, block size 1, K a multiple of 8 and 16-byte aligned
-    # rows, which the contiguous 8-lane-run kernel serves. Widths past one
-    # 2048-lane chunk, bitmaps too wide to stage (T > 131072), stray rows and
+    # rows: the contiguous 8-lane-run kernel past one 2048-lane chunk, the
+    # direct kernel within it. Bitmaps too wide to stage (T > 131072), stray rows and
     # partial selections; a Top-K view shifted by one element must give the
-    # same answer through the strided kernel.
+    # same answer through the strided kernel past one chunk.
     rng = np.random.default_rng(9100 + seed)
     layers = int(rng.integers(1, 4))
     batch = int(rng.integers(1, 9))
@@ -177,6 +177,9 @@ def test_local_slot_runs_random_configurations(gpu, coracle, seed):
                          torch.tensor(lengths, dtype=torch.int32, device=gpu), torch.tensor(selected, device=gpu),
                          output, 1, misses=misses, miss_count=counts, resident_bits=bits, slot_base=base_d)
         case = (seed, layers, batch, k, cols, layered, topk_d.data_ptr() % 16)
+        route = lookup_route(topk_d, table_d, None, torch.tensor(rows), torch.tensor(lengths), torch.tensor(selected),
+                             output, 1, misses=misses, miss_count=counts, resident_bits=bits, slot_base=base_d)
+        assert route == ("direct" if k <= 2048 else "runs" if topk_d is topk_aligned else "local"), case
         assert np.array_equal(output.cpu().numpy(), want), case
         if compact:
             got_counts, got_misses = counts.cpu().numpy(), misses.cpu().numpy()
@@ -196,12 +199,13 @@ def test_local_slot_prefetch_many_items_per_workgroup(gpu, coracle, seed):
     # the prefetching kernel (int16 local-slot and int32 global-slot tables),
     # whose persistent grid gives each workgroup
     # several (row, layer) items once there are more items than resident
-    # workgroups (about 2048 on MI355X): here 3,000-8,000 items, with stray
+    # workgroups (about 2048 on MI355X): here 3,000-8,000 items (of at least 528
+    # lanes, too many bytes for the direct kernel), with stray
     # request rows, stray selections, short lengths and negative entries.
     rng = np.random.default_rng(9400 + seed)
     layers = int(rng.integers(20, 41))
     batch = int(rng.integers(150, 201))
-    k = 8 * int(rng.integers(1, 257))
+    k = 8 * int(rng.integers(66, 257))
     rrows = int(rng.integers(batch // 2, batch + 1))
     cols = int(rng.integers(1, 8193)) if seed % 2 else 128 * int(rng.integers(1, 65))   # odd seeds: any T
     layered = seed != 5
@@ -232,10 +236,11 @@ def test_local_slot_prefetch_many_items_per_workgroup(gpu, coracle, seed):
     output = torch.tensor(initial, device=gpu)
     misses = torch.full((layers, batch, k), -5, dtype=torch.int32, device=gpu) if compact else None
     counts = torch.full((layers, batch), -5, dtype=torch.int32, device=gpu) if compact else None
-    resolve_resident(torch.tensor(topk, dtype=torch.int32, device=gpu), table_d, None, torch.tensor(rows, device=gpu),
-                     torch.tensor(lengths, dtype=torch.int32, device=gpu), torch.tensor(selected, device=gpu),
-                     output, 1, misses=misses, miss_count=counts, resident_bits=bits,
-                     slot_base=torch.tensor(slot_base, device=gpu))
+    args = (torch.tensor(topk, dtype=torch.int32, device=gpu), table_d, None, torch.tensor(rows, device=gpu),
+            torch.tensor(lengths, dtype=torch.int32, device=gpu), torch.tensor(selected, device=gpu), output, 1)
+    extra = dict(misses=misses, miss_count=counts, resident_bits=bits, slot_base=torch.tensor(slot_base, device=gpu))
+    assert lookup_route(*args, **extra) == "two-stage prefetch"
+    resolve_resident(*args, **extra)
     chosen = np.zeros(batch, bool)
     chosen[selected[(selected >= 0) & (selected < batch)]] = True
     lanes = np.arange(k)
@@ -258,19 +263,18 @@ def test_local_slot_prefetch_many_items_per_workgroup(gpu, coracle, seed):
     output = torch.tensor(initial, device=gpu)
     misses = torch.full((layers, batch, k), -5, dtype=torch.int32, device=gpu) if compact else None
     counts = torch.full((layers, batch), -5, dtype=torch.int32, device=gpu) if compact else None
-    resolve_resident(torch.tensor(topk, dtype=torch.int32, device=gpu), table32, None, torch.tensor(rows, device=gpu),
-                     torch.tensor(lengths, dtype=torch.int32, device=gpu), torch.tensor(selected, device=gpu),
-                     output, 1, misses=misses, miss_count=counts, resident_bits=build_residency_bits(table32))
+    args = (args[0], table32, *args[2:6], output, 1)
+    extra = dict(misses=misses, miss_count=counts, resident_bits=build_residency_bits(table32))
+    assert lookup_route(*args, **extra) == "two-stage prefetch"
+    resolve_resident(*args, **extra)
     check(output, misses, counts, (seed, layers, batch, k, cols, layered, "int32"))
 
 
 @pytest.mark.parametrize("seed", range(40))
 def test_summary_lookup_random_configurations(gpu, coracle, seed):
     # Single-level lookups behind residency summaries of random coarseness
-    # (shift 0-9): summaries of at most 64 words per row take the one-wave-per-
-    # item kernel (its rows are walked in passes of 512 lanes, here 1-10 of
-    # them, the last one partial), wider ones the prefetching or strided
-    # kernels. int16 local-slot and int32 global-slot tables; exact summaries
+    # (shift 0-9): rows of up to 2048 lanes take the direct kernel, wider ones the
+    # run kernel (int16) or the strided one (int32). int16 local-slot and int32 global-slot tables; exact summaries
     # and supersets with stray bits past the length and past the table; stray
     # rows and selections, lengths past the table, negative entries.
     rng = np.random.default_rng(9700 + seed)
@@ -322,6 +326,10 @@ def test_summary_lookup_random_configurations(gpu, coracle, seed):
                      output, 1, misses=misses, miss_count=counts, resident_bits=bits, bits_shift=shift,
                      slot_base=base_d)
     case = (seed, layers, batch, k, cols, shift, layered, local)
+    route = lookup_route(torch.tensor(topk, dtype=torch.int32), table_d, None, torch.tensor(rows), torch.tensor(lengths),
+                         torch.tensor(selected), output, 1, misses=misses, miss_count=counts, resident_bits=bits,
+                         bits_shift=shift, slot_base=base_d)
+    assert route == ("direct" if k <= 2048 else "runs" if local else "strided"), case
     assert np.array_equal(output.cpu().numpy(), want), case
     if compact:
         got_counts, got_misses = counts.cpu().numpy(), misses.cpu().numpy()

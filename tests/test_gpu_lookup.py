@@ -8,7 +8,7 @@ import numpy as np
 import pytest
 import torch
 
-from adaptive_sparse.resident_lookup import resolve_resident
+from adaptive_sparse.resident_lookup import lookup_route, resolve_resident
 
 pytestmark = pytest.mark.gpu
 
@@ -386,9 +386,10 @@ def test_whole_block_lookups_match_oracle_and_general_path(gpu, bs, k, cols, dty
                                         (1, 1201, 300), (1, 1200, 700), (1, 2040, 360)])
 @pytest.mark.parametrize("dtype", [torch.int16, torch.int32])
 def test_direct_lookups_match_oracle_and_general_path(gpu, bs, k, batch, dtype):
-    # Rows on both sides of every workgroup width, few rows and more rows than the wide ones take (300 rows over two
-    # layers: the prefetching kernel, whose threads past the row store the last piece again, or the general one), stray
-    # selections and requests, short and negative lengths; a strided output takes the general kernel.
+    # Rows on both sides of every workgroup width, few rows and (700 and 360 rows of two layers) more than the direct
+    # kernel takes: the prefetching kernel, whose threads past the row store the last piece again, or without a summary
+    # the general one. Permuted selections with stray entries, stray requests, short and negative lengths; a strided
+    # output takes the general kernel.
     from adaptive_sparse.resident_lookup import build_residency_bits
     from oracle import oracle as ref
 
@@ -406,7 +407,9 @@ def test_direct_lookups_match_oracle_and_general_path(gpu, bs, k, batch, dtype):
     width = k * bs
     table_d = torch.tensor(local, dtype=dtype, device=gpu)
     bits = build_residency_bits(table_d, shift=6)
-    for selected in (np.arange(batch), np.array([3, 0, -1, 4, batch, 2])):
+    for selected in (np.arange(batch), np.concatenate([rng.permutation(batch), [-1, batch]]),
+                     np.array([3, 0, -1, 4, batch, 2])):
+        large = width > 1024 and layers * len(selected) * width * dtype.itemsize > 11 << 18     # not direct
         want, want_misses, want_counts = ref.resolve_resident(topk, table, None, rows, lengths, selected, bs,
                                                               np.full((layers, batch, width), -77, np.int32),
                                                               with_misses=True)
@@ -418,6 +421,11 @@ def test_direct_lookups_match_oracle_and_general_path(gpu, bs, k, batch, dtype):
                     torch.tensor(lengths, dtype=torch.int32, device=gpu), torch.tensor(selected, device=gpu), out, bs)
             extra = dict(resident_bits=bits if summary else None, bits_shift=6 if summary else 0,
                          slot_base=torch.tensor(base, device=gpu) if dtype == torch.int16 else None)
+            route = lookup_route(*args, misses=misses, miss_count=counts, **extra)
+            if step == 2 or (large and (not summary or width % 8)):
+                assert route == "strided"
+            else:
+                assert route == ("two-stage prefetch" if large else "direct")
             resolve_resident(*args, misses=misses, miss_count=counts, **extra)
             assert np.array_equal(out.cpu().numpy(), want), (len(selected), topk_dtype, step)
             got_counts, got = counts.cpu().numpy(), misses.cpu().numpy()

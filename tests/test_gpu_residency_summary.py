@@ -1,10 +1,10 @@
 """GPU parity of the coarse residency summary (one bit per group of 2**shift positions).
 
-The summary builder must equal the oracle's, and every lookup kernel that
-reads a summary (the prefetching int16 kernel, the contiguous-pieces kernel,
-the strided int16 and int32 kernels) must give the oracle's plain lookup -
-slots, miss lists and counts - for exact summaries and for supersets of
-them (stale group bits). The swap-in keeps a coarse summary exact through
+The summary builder must equal the oracle's, and lookups handed a summary
+(here the contiguous-pieces and strided kernels, which read it, and the direct
+one, which does not; the prefetching ones in test_gpu_lookup_routes.py) must
+give the oracle's plain lookup - slots, miss lists and counts - for exact
+summaries and for supersets of them (stale group bits). The swap-in keeps a coarse summary exact through
 its group counts; without them it leaves a superset behind.
 """
 
@@ -12,7 +12,7 @@ import numpy as np
 import pytest
 import torch
 
-from adaptive_sparse.resident_lookup import build_residency_bits, resolve_resident, summary_words
+from adaptive_sparse.resident_lookup import build_residency_bits, lookup_route, resolve_resident, summary_words
 from adaptive_sparse.swap_in import HotBuffers, swap_in
 from elastic_kv import _native
 from oracle import oracle as ref
@@ -69,11 +69,11 @@ def _superset(bits, rng, density=0.3):
 
 
 @pytest.mark.parametrize("shift", [3, 6])
-@pytest.mark.parametrize("shape", ["pipe", "runs", "strided"])
+@pytest.mark.parametrize("shape", ["direct", "runs", "shifted"])
 def test_lookup_with_summary_matches_oracle(gpu, shift, shape):
-    rng = np.random.default_rng({"pipe": 1, "runs": 2, "strided": 3}[shape] * 10 + shift)
+    rng = np.random.default_rng({"direct": 1, "runs": 2, "shifted": 3}[shape] * 10 + shift)
     L, R, T, C = 3, 6, 9000, 1500
-    K = {"pipe": 1024, "runs": 2560, "strided": 1024}[shape]
+    K = {"direct": 1024, "runs": 2560, "shifted": 2560}[shape]
     topk, local = _decode_case(rng, L, R, T, K, C, 3000)
     base = np.arange(R) * C + 1
     lengths = np.full(R, T)
@@ -84,8 +84,8 @@ def test_lookup_with_summary_matches_oracle(gpu, shift, shape):
                                                           np.arange(R), 1, np.full((L, R, K), -7, np.int32),
                                                           with_misses=True)
     topk_d = torch.tensor(topk, dtype=torch.int32, device=gpu)
-    if shape == "strided":
-        # a Top-K view shifted by one element is not 16-byte aligned: the strided kernel runs
+    if shape == "shifted":
+        # a Top-K view shifted by one element is not 16-byte aligned: the strided kernels run
         wide = torch.zeros((L, R, K + 1), dtype=torch.int32, device=gpu)
         wide[..., 1:] = topk_d
         topk_d = wide[..., 1:]
@@ -97,9 +97,11 @@ def test_lookup_with_summary_matches_oracle(gpu, shift, shape):
             slots = torch.full((L, R, K), -7, dtype=torch.int32, device=gpu)
             misses = torch.full((L, R, K), -3, dtype=torch.int32, device=gpu)
             counts = torch.empty((L, R), dtype=torch.int32, device=gpu)
-            resolve_resident(topk_d, table, None, rows, torch.tensor(lengths, device=gpu), rows, slots, 1,
-                             misses=misses, miss_count=counts, resident_bits=bits, bits_shift=shift,
-                             slot_base=slot_base)
+            args = (topk_d, table, None, rows, torch.tensor(lengths, device=gpu), rows, slots, 1)
+            extra = dict(misses=misses, miss_count=counts, resident_bits=bits, bits_shift=shift, slot_base=slot_base)
+            assert lookup_route(*args, **extra) == ("direct" if shape == "direct" else "strided" if slot_base is None
+                                                    else "runs" if shape == "runs" else "local")
+            resolve_resident(*args, **extra)
             assert np.array_equal(slots.cpu().numpy(), want)
             assert np.array_equal(counts.cpu().numpy(), want_counts)
             got = misses.cpu().numpy()

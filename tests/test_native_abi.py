@@ -5,6 +5,7 @@ validation before any HIP call.
 """
 
 import ctypes as ct
+import math
 import re
 import subprocess
 
@@ -139,6 +140,44 @@ def test_kernel_entry_points_validate_before_launch(lib):
     assert b"unknown stream probe flags" in typed.ev_error()
     assert typed.ekv_stream_probe(3 | 0x10, 4096, 4096, 1 << 20, 0, None) == -1
     assert b"mode must be" in typed.ev_error()
+
+
+def test_lookup_routes_are_told_without_a_device(lib):
+    # Descriptors of tensors that do not exist: the query reads no element.
+    from elastic_kv import _native
+
+    typed = _native.kernel_library(str(LIBRARY))
+
+    def tensor(shape, dtype, strides=None):
+        strides = strides or [int(math.prod(shape[i + 1:])) for i in range(len(shape))]
+        return _native.EkvTensor(4096, dtype, len(shape), (ct.c_int64 * 4)(*shape), (ct.c_int64 * 4)(*strides))
+
+    def route(layers, batch, k, cols, bs=1, topk=1, table=5, bits=True, mapped=False, out_stride=1, selected=None, k_out=None):
+        width = (k if k_out is None else k_out) * bs
+        words = -(--(-cols // 32) // 4) * 4
+        out = tensor((layers, batch, width), 1, (batch * width * out_stride, width * out_stride, out_stride))
+        parts = [tensor((layers, batch, k), topk), tensor((batch, cols), table), tensor((99,), 2) if mapped else None,
+                 tensor((batch,), 2) if table == 5 else None, tensor((batch, words), 1) if bits else None]
+        rest = [tensor((batch,), 2), tensor((batch,), 1), tensor((batch if selected is None else selected,), 2), out]
+        refs = [None if p is None else ct.byref(p) for p in parts + rest]
+        return typed.ekv_lookup_route(*refs[:5], 0, *refs[5:], None, None, bs)
+
+    assert route(1, 32, 2048, 4096) == b"direct"
+    assert route(60, 128, 2048, 4096) == b"two-stage prefetch"
+    assert route(60, 128, 2048, 65536) == b"one-stage prefetch"
+    assert route(60, 128, 2048, 65536 + 32) == b"runs"              # a summary past 2048 words
+    assert route(60, 128, 2047, 4096) == b"local"
+    assert route(60, 128, 2048, 4096, bits=False) == route(60, 128, 2048, 4096, topk=2) == b"strided"
+    assert route(60, 128, 2048, 4096, table=1) == b"two-stage prefetch"
+    assert route(60, 128, 4096, 8192) == b"runs"
+    assert route(60, 128, 4096, 8192, table=1) == b"strided"
+    assert route(60, 128, 256, 4096) == route(60, 128, 256, 4096, bits=False, topk=2) == b"direct"
+    assert route(28, 48, 32, 4096, bs=64) == b"blocks"
+    assert route(28, 48, 32, 4096, bs=64, out_stride=2) == b"strided"
+    assert route(1, 4, 16, 8192, bs=128, table=2, bits=False, mapped=True) == b"two-level direct"
+    assert route(4, 129, 16, 8192, bs=128, table=2, bits=False, mapped=True) == b"two-level"
+    assert route(1, 4, 16, 4096, selected=0) == b"none"
+    assert route(1, 4, 16, 4096, k_out=15) is None and b"output dimension 2 is 15, expected 16" in typed.ev_error()
 
 
 def test_packed_descriptors_are_the_struct_bytes(lib):
