@@ -56,6 +56,10 @@ _capsule_new.argtypes = [ct.c_void_p, ct.c_char_p, ct.c_void_p]
 # address of a live DLManagedTensor -> (struct, shape array, owner)
 _live = {}
 _lock = threading.Lock()
+# A reference that is never given back: a tensor still alive when the interpreter ends is released after the
+# collector has run over the modules, and its deleter is one of this table's entries. Without it the table was
+# cleared under the deleter (a segmentation fault at exit, with owners that hold their own views).
+ct.pythonapi.Py_IncRef(ct.py_object(_live))
 
 
 # The deleter can run during interpreter shutdown, after this module's

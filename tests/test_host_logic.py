@@ -10,6 +10,8 @@ import gc
 import json
 import math
 import random
+import subprocess
+import sys
 from types import SimpleNamespace
 from unittest.mock import Mock, call, patch
 
@@ -19,7 +21,7 @@ from adaptive_sparse.kv_pool import BlockMajorLayout, PlanePoolLayout
 from adaptive_sparse.migration import plan_demote_pages
 from adaptive_sparse.migration_budget import MigrationBandwidthEstimator
 from adaptive_sparse.minimax_vmm import PageFootprints, PhysicalPages
-from conftest import GOLDEN
+from conftest import GOLDEN, PACKAGE
 from elastic_kv.backing import Backing, _load_library
 from elastic_kv.slots import FreeSlots
 from experimental.resident_arena import VmmResidentArena
@@ -904,3 +906,34 @@ def test_hot_buffers_refuse_a_slot_base_on_the_sink():
     with pytest.raises(ValueError, match="slot_base must be >= 1"):
         HotBuffers(1, 2, 16, 4, "cpu", slot_base=torch.tensor([0, 4]))
     assert HotBuffers(1, 2, 16, 4, "cpu", slot_base=torch.tensor([1, 5])).slot_base.tolist() == [1, 5]
+
+
+# ------------------------------------------------------------------ borrowed views at interpreter exit
+
+
+EXIT_SCRIPT = """
+import ctypes as ct, sys, weakref
+sys.path.insert(0, sys.argv[1])
+import torch
+from elastic_kv import _dlpack
+libc = ct.CDLL(None)
+libc.malloc.restype, libc.malloc.argtypes, libc.free.argtypes = ct.c_void_p, [ct.c_size_t], [ct.c_void_p]
+
+class Owner:
+    def __init__(self, size):
+        self.address = libc.malloc(size)
+        weakref.finalize(self, libc.free, self.address)
+        self.view = _dlpack.borrow_bytes(self.address, size, _dlpack.KDL_CPU, 0, self)   # as HostArena.host
+
+for _ in range(20):
+    owner = Owner(4096)
+    owner.view.fill_(1)
+kept = owner.view.narrow(0, 16, 16)
+print(_dlpack.live_borrows(), int(kept.sum()), flush=True)
+"""
+
+
+def test_views_alive_at_exit_are_released_after_the_modules():
+    result = subprocess.run([sys.executable, "-c", EXIT_SCRIPT, str(PACKAGE)], capture_output=True, text=True, timeout=120)
+    assert result.returncode == 0, result.stderr
+    assert result.stdout.split() == ["20", "16"]
