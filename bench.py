@@ -983,7 +983,7 @@ def run_hisparse_swap(torch, args, device):
               "selection": "newest block + 12 of the other 31 recent blocks + 3 older blocks per call"}
     roof = {"bound": "pcie", "achieved": round(achieved, 2), "peak": PCIE_PEAK_GBS, "unit": "GB/s",
             "frac": round(achieved / PCIE_PEAK_GBS, 4), "traffic": None,
-            "kernel": "hisparse_swap_kernel<16> (ekv_hisparse_swap_in)",
+            "kernel": "hisparse_swap_kernel<1024, 16> (ekv_hisparse_swap_in)",
             "algorithmic_bytes_per_launch": round(statistics.mean(promoted)), "avg_launch_ms": round(mean_ms, 4)}
     extra = {"call_ms": spread(call_ms), "misses_per_call": round(statistics.mean(misses), 1),
              "hit_rate": round(hit_rate, 4), "tokens_per_s": round(R * W / (mean_ms / 1e3), 1),

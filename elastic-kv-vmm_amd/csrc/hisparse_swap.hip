@@ -34,8 +34,8 @@
 //      other lanes reuse that lane's location, so the hot buffer never holds
 //      a token twice;
 //   3. ranks in selection order (output position, hit rank, miss rank): each
-//      thread counts a contiguous run of lanes, one workgroup scan (wave64
-//      shuffles + one LDS exchange) turns the counts into ranks;
+//      thread counts a contiguous run of lanes, one workgroup scan (DPP steps
+//      in each wave + one LDS exchange) turns the counts into ranks;
 //   4. the same scan over contiguous runs of the old LRU order gives each
 //      slot's place in the new order and the victims (empty slots first, then
 //      untouched slots);
@@ -211,8 +211,8 @@ __device__ __forceinline__ void copy_own_rows(const HsArgs& a, const Lds& s, int
 // One workgroup per batch row holds its CU nearly alone (134 KiB of LDS at the
 // largest shape) and is a chain of barriers, so the more waves share its loops the
 // shorter it is: kThreads is the smallest size whose threads hold four hot slots
-// and two lanes each. 24 rows of 2048 lanes and 4096 slots: 44 us with 256
-// threads, 23 us with 1024.
+// and two lanes each. 24 rows of 2048 lanes and 4096 slots, none missing: 41.4 us
+// with 256 threads, 19.7 us with 1024.
 // kCopyWidth: bytes per copy piece when the workgroup copies its row's misses
 // itself, 0 when the copy launch does (copies_own_rows decides).
 template <int kThreads, int kCopyWidth>

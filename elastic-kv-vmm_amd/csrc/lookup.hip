@@ -5,7 +5,12 @@
 // leading layer dimension, an optional second indirection level and an
 // ordered miss list (lanes whose slot is 0 = not resident).
 //
-// Launch shape: one 256-thread workgroup (4 waves) per (selected row, layer).
+// Small jobs - the decode step's lookups of one layer, narrow rows, the
+// reference's microbenchmark - take resolve_direct_kernel: 64 to 512 threads of four
+// strided lanes for a row of up to 2048, ids and then entries read at once, no summary
+// (its rule, in resolve_resident, has both sides measured).
+//
+// The general launch shape: one 256-thread workgroup (4 waves) per (selected row, layer).
 // A row of `width` lanes is walked in chunks of 2048 lanes; wave w owns lanes
 // [512w, 512w + 512) of a chunk and processes them as 8 iterations of 64
 // consecutive lanes, so a wave's lane order is the row's lane order.
@@ -32,7 +37,8 @@
 // resolve_runs_kernel, and for rows of one chunk the persistent prefetching
 // forms resolve_runs_pipe_kernel and resolve_runs_pipe2_kernel (two stages:
 // the next item's table reads are in flight during the current item's
-// compaction; the default for summary rows of at most 1024 words).
+// compaction; the default for summary rows of at most 1024 words). route_of
+// names the kernel of a call.
 // Recent window: decode Top-K sets concentrate on the most recent tokens, and
 // lanes that gather single table entries cost one L2 request each. Both
 // kernels therefore stage the table entries of the last kWindow positions
@@ -2064,6 +2070,9 @@ int resolve_resident(const ekv_tensor* topk_p, const ekv_tensor* table_p, const 
     //   7680 x 512          26.62 / 26.68    7680 x 512, int32   28.59 / 30.82
     //   7680 x 511 ragged   42.89 / 28.85    7680 x 511, int32   43.14 / 32.41
     //   7680 x 256          25.78 / 16.99    7680 x 256, int32   26.37 / 20.64
+    // Lookups without a summary keep the same lines, with the strided kernel past them; on this side of them
+    // (us; strided / direct): 32 x 2048 5.9 / 4.9, 512 x 2048 8.2 / 6.3, 2560 x 1024 22.6 / 17.6, 2560 x 256 14.8 / 7.6.
+    // On the first pass over new inputs the small ones gain nothing: the inputs' way from HBM is all of it.
     const int64_t entries_read = count * layers * std::min<int64_t>(width, kChunkLanes) * entry_bytes;   // bytes
     const bool ragged = a.pipe == 0;
     const bool spared = width <= 256    ? false

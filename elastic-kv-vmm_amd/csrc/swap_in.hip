@@ -292,9 +292,10 @@ __device__ __forceinline__ void hash_miss_tokens(uint32_t* hash, const int32_t* 
 // and 8 registers of unrolled code, 53 KB of instructions fetched once per
 // row, and the same code ran for a row of 256 slots. Scans are DPP steps,
 // the summary is changed in LDS and written once, and dense rows are addressed
-// with 32-bit offsets. With the launch, against those 256 threads and global
-// atomics: 48 rows of 1024 lanes (2048 slots) 27.2 -> 14.4 us, 2560 rows of 256 lanes
-// 77.3 -> 26.3, of 2048 lanes 187.9 -> 115.1. The last moves 246 MB from and
+// with 32-bit offsets. The swap alone, against those 256 threads and global
+// atomics: 48 rows of 1024 lanes (2048 slots) 23.1 -> 12.8 us, 2560 rows of 256 lanes
+// 67.1 -> 24.7, of 2048 lanes 183.7 -> 115.0; 1280 rows of 4096 lanes and 8192 slots
+// 262 -> 163 with the lookup. The 2560 x 2048 launch moves 246 MB from and
 // 215 MB to HBM by the counters (scattered table entries as whole lines), 84 us
 // at the rate of a copy.
 //
