@@ -465,7 +465,7 @@ void launch_vw(const ArgsOf<M>& a, int vw, hipStream_t stream) {
 // moves, in list order, are strided over the grid, so rows of unequal counts
 // and the unused tails of the lists cost nothing. The list entries of an
 // iteration are read while the load of the one before is in flight.
-// Beside the driver's unmaps the few requests cost the move itself (each waits
+// Beside the HIP driver's unmaps the few requests cost the move itself (each waits
 // for the TLB flushes: 6.9 GB took 168-172 ms, 132-134 through the tile kernel),
 // but the unmaps run faster beside them (341-357 against 451-459 us a chunk), and they
 // are what the elastic step waits for: 348-370 ms a step with 774 chunks remapped
@@ -484,8 +484,9 @@ constexpr uint32_t kHostRows = kThreads * kHostRowsPerThread;
 //   8 x 1024 x 512 B (8 MiB)    75.3 /  70.6     48 x 1024 x 516 B (4 B)    451 / 527
 //   48 x 256 x 512 B (12 MiB)    109 /  92.4     48 x 1024 x 520 B (8 B)    455 / 485
 //   4 x 128 x 8 KiB (8 MiB)     78.3 /  62.9     4 layers 128 x 2048 x 512 B  7,800 / 7,540
-// Lists of which 2 % are used take 0.7-1.5 us longer here up to 24 MiB (24 x 256: 6.1 / 6.8) and the same past it; host rows
-// that the call itself reads a dozen times come from the memory-side cache, where more in flight is 4-11 % faster.
+// Lists of which 2 % are used take 0.7-1.5 us longer here up to 24 MiB (24 x 256: 6.1 / 6.8) and the same past it;
+// host rows that the call itself reads a dozen times come from the memory-side cache, where more in flight is 4-11 %
+// faster.
 constexpr int64_t kHostMoveBytes = int64_t{6} << 20;
 constexpr int64_t kHostRowBytes = 256;
 

@@ -2071,7 +2071,7 @@ int resolve_resident(const ekv_tensor* topk_p, const ekv_tensor* table_p, const 
     //   7680 x 511 ragged   42.89 / 28.85    7680 x 511, int32   43.14 / 32.41
     //   7680 x 256          25.78 / 16.99    7680 x 256, int32   26.37 / 20.64
     // Lookups without a summary keep the same lines, with the strided kernel past them; on this side of them
-    // (us; strided / direct): 32 x 2048 5.9 / 4.9, 512 x 2048 8.2 / 6.3, 2560 x 1024 22.6 / 17.6, 2560 x 256 14.8 / 7.6.
+    // (us; strided / direct): 32 x 2048 5.9 / 4.9, 512 x 2048 8.2 / 6.3, 2560 x 256 14.8 / 7.6, 7680 x 256 36.0 / 19.9.
     // On the first pass over new inputs the small ones gain nothing: the inputs' way from HBM is all of it.
     const int64_t entries_read = count * layers * std::min<int64_t>(width, kChunkLanes) * entry_bytes;   // bytes
     const bool ragged = a.pipe == 0;

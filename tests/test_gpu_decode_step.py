@@ -326,12 +326,14 @@ def test_promotions_over_a_selection_in_each_kernel(gpu, rows_n, context, hot, l
                         row_stride=row, row_bytes=row, rows=rows_n * context, owner=arena)
         host_table = torch.arange(rows_n * context, dtype=torch.int32, device=gpu).reshape(rows_n, context)
         rng = np.random.default_rng(11)
-        buffers = [HotBuffers(layers, rows_n, context, hot, gpu, table_dtype=torch.int16, bits_shift=6) for _ in range(2)]
+        buffers = [HotBuffers(layers, rows_n, context, hot, gpu, table_dtype=torch.int16, bits_shift=6)
+                   for _ in range(2)]
         pools = [torch.zeros((layers, 2, 1 + rows_n * hot, row), dtype=torch.uint8, device=gpu) for _ in range(2)]
         rows = torch.tensor(rng.permutation(rows_n), device=gpu)
         lengths = torch.tensor(rng.integers(context // 2, context + 5, rows_n), dtype=torch.int32, device=gpu)
         for step in range(3):
-            picks = [np.arange(rows_n), np.concatenate([rng.permutation(rows_n), [-1, rows_n]]), rng.permutation(rows_n)[:9]][step]
+            picks = [np.arange(rows_n), np.concatenate([rng.permutation(rows_n), [-1, rows_n]]),
+                     rng.permutation(rows_n)[:9]][step]
             selected = torch.tensor(rng.permutation(picks) if step == 1 else picks, device=gpu)
             topk = torch.tensor(np.stack([rng.permutation(context)[:lanes] for _ in range(layers * rows_n)]).reshape(
                 layers, rows_n, lanes), dtype=torch.int32, device=gpu)
@@ -343,7 +345,8 @@ def test_promotions_over_a_selection_in_each_kernel(gpu, rows_n, context, hot, l
                 slots = torch.full((layers, rows_n, lanes), -9, dtype=torch.int32, device=gpu)
                 out = torch.empty((rows_n, layers, 2, lanes, row), dtype=torch.uint8, device=gpu)
                 if staged:
-                    misses, counts = torch.empty_like(slots), torch.zeros((layers, rows_n), dtype=torch.int32, device=gpu)
+                    misses = torch.empty_like(slots)
+                    counts = torch.zeros((layers, rows_n), dtype=torch.int32, device=gpu)
                     resolve_resident(topk, b.table, None, rows, lengths, selected, slots, 1, misses=misses,
                                      miss_count=counts, resident_bits=b.bits, bits_shift=6, slot_base=b.slot_base)
                     src, dst = torch.empty_like(slots), torch.empty_like(slots)

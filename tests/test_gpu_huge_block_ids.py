@@ -41,19 +41,22 @@ def test_lookups_return_no_slot_for_huge_ids(gpu, coracle, bs, form):
     stored = np.where(table > 0, base.reshape(1, -1, 1) + table - 1, 0) if form == "int16" else table
     mapping = np.concatenate([[0], rng.integers(1, 1 << 20, 1 << 14)]) if form == "mapped" else None
     topk, clean = with_huge_ids(rng, (layers, batch, k), cols // bs)
-    rows, lengths, selected = rng.integers(0, table_rows, batch), np.array([cols, cols - 5, 9, -4, 1 << 30]), np.arange(batch)
+    rows, selected = rng.integers(0, table_rows, batch), np.arange(batch)
+    lengths = np.array([cols, cols - 5, 9, -4, 1 << 30])
     blank = np.full((layers, batch, k * bs), -77, np.int32)
-    want, want_misses, want_counts = coracle.resolve_resident(clean, stored, mapping, rows, lengths, selected, bs, blank,
-                                                              with_misses=True)
+    want, want_misses, want_counts = coracle.resolve_resident(clean, stored, mapping, rows, lengths, selected, bs,
+                                                              blank, with_misses=True)
     dtype = {"int16": torch.int16, "int64": torch.int64}.get(form, torch.int32)
     table_d = torch.tensor(table, dtype=dtype, device=gpu)
     step = 2 if form == "strided" else 1
     out = torch.full((*blank.shape, step), -77, dtype=torch.int32, device=gpu)[..., 0]
-    misses, counts = torch.full(blank.shape, -5, dtype=torch.int32, device=gpu), torch.zeros((layers, batch), dtype=torch.int32, device=gpu)
+    misses = torch.full(blank.shape, -5, dtype=torch.int32, device=gpu)
+    counts = torch.zeros((layers, batch), dtype=torch.int32, device=gpu)
+    mapping_d = None if mapping is None else torch.tensor(mapping, device=gpu)
     for bits in ([None] if form in ("mapped", "int64") else [None, build_residency_bits(table_d)]):
-        resolve_resident(torch.tensor(topk, device=gpu), table_d, None if mapping is None else torch.tensor(mapping, device=gpu),
-                         torch.tensor(rows, device=gpu), torch.tensor(lengths, device=gpu), torch.tensor(selected, device=gpu),
-                         out, bs, misses=misses, miss_count=counts, resident_bits=bits,
+        resolve_resident(torch.tensor(topk, device=gpu), table_d, mapping_d, torch.tensor(rows, device=gpu),
+                         torch.tensor(lengths, device=gpu), torch.tensor(selected, device=gpu), out, bs,
+                         misses=misses, miss_count=counts, resident_bits=bits,
                          slot_base=torch.tensor(base, device=gpu) if form == "int16" else None)
         assert np.array_equal(out.cpu().numpy(), want)
         assert np.array_equal(counts.cpu().numpy(), want_counts)

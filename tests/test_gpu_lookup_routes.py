@@ -50,8 +50,9 @@ def check(coracle, gpu, route, layers, batch, k, cols, dtype, *, bs=1, shift=0, 
     misses = torch.full(blank.shape, -5, dtype=torch.int32, device=gpu) if compact else None
     counts = torch.full(blank.shape[:2], -5, dtype=torch.int32, device=gpu) if compact else None
     args = (torch.tensor(topk, dtype=topk_dtype, device=gpu), table,
-            None if mapping is None else torch.tensor(mapping, dtype=mapped, device=gpu), torch.tensor(rows, device=gpu),
-            torch.tensor(lengths, dtype=torch.int32, device=gpu), torch.tensor(selected, device=gpu), slots, bs)
+            None if mapping is None else torch.tensor(mapping, dtype=mapped, device=gpu),
+            torch.tensor(rows, device=gpu), torch.tensor(lengths, dtype=torch.int32, device=gpu),
+            torch.tensor(selected, device=gpu), slots, bs)
     extra = dict(misses=misses, miss_count=counts, resident_bits=summary, bits_shift=shift,
                  slot_base=torch.tensor(base, device=gpu) if dtype == torch.int16 else None)
     assert lookup_route(*args, **extra) == route

@@ -934,6 +934,7 @@ print(_dlpack.live_borrows(), int(kept.sum()), flush=True)
 
 
 def test_views_alive_at_exit_are_released_after_the_modules():
-    result = subprocess.run([sys.executable, "-c", EXIT_SCRIPT, str(PACKAGE)], capture_output=True, text=True, timeout=120)
+    result = subprocess.run([sys.executable, "-c", EXIT_SCRIPT, str(PACKAGE)], capture_output=True, text=True,
+                            timeout=120)
     assert result.returncode == 0, result.stderr
     assert result.stdout.split() == ["20", "16"]

@@ -152,7 +152,8 @@ def test_lookup_routes_are_told_without_a_device(lib):
         strides = strides or [int(math.prod(shape[i + 1:])) for i in range(len(shape))]
         return _native.EkvTensor(4096, dtype, len(shape), (ct.c_int64 * 4)(*shape), (ct.c_int64 * 4)(*strides))
 
-    def route(layers, batch, k, cols, bs=1, topk=1, table=5, bits=True, mapped=False, out_stride=1, selected=None, k_out=None):
+    def route(layers, batch, k, cols, bs=1, topk=1, table=5, bits=True, mapped=False, out_stride=1, selected=None,
+              k_out=None):
         width = (k if k_out is None else k_out) * bs
         words = -(--(-cols // 32) // 4) * 4
         out = tensor((layers, batch, width), 1, (batch * width * out_stride, width * out_stride, out_stride))
